@@ -6,6 +6,7 @@
 // launch anything: they append an Op (with host-precomputed constants) to the bunch's
 // queue, and the queue is applied by one fused kernel when the bunch is next needed.
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstring>
 #include <mutex>
@@ -131,6 +132,18 @@ void check_statuses(bool wait) {
   OB_REQUIRE(err.empty(), err);
 }
 
+void host_wait_seq(const uint64_t* host, uint64_t want, hipStream_t s) {
+  const auto t0 = std::chrono::steady_clock::now();
+  while (__atomic_load_n(host, __ATOMIC_ACQUIRE) != want) {
+    if (std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(20)) {
+      OB_HIP(hipStreamSynchronize(s));
+      OB_REQUIRE(__atomic_load_n(host, __ATOMIC_ACQUIRE) == want,
+                 "a reduction's result did not reach the host");
+      break;
+    }
+  }
+}
+
 }  // namespace ob
 
 // ---------------------------------------------------------------------------
@@ -159,6 +172,7 @@ struct ob_bunch {
 
   std::vector<ob::Op> queue;
   ob_batch* owner = nullptr;  // batch applying this bunch's maps, if any
+  ob::DiagWork diag;
 };
 
 namespace ob {
@@ -329,6 +343,30 @@ void bunch_sort_commit(ob_bunch* b) {
 }
 
 void bunch_device_written(ob_bunch* b) { b->host_valid = false; }
+
+DiagWork& bunch_diag_work(ob_bunch* b, size_t dev_doubles, size_t host_doubles) {
+  DiagWork& w = b->diag;
+  if (dev_doubles > w.dev_cap) {
+    if (w.dev) OB_HIP(hipFree(w.dev));  // (waits for the kernels that read it)
+    w.dev = nullptr;
+    w.dev_cap = 0;
+    const size_t cap = std::max<size_t>(dev_doubles, 1 << 15);
+    OB_HIP(hipMalloc((void**)&w.dev, sizeof(double) * cap));
+    w.dev_cap = cap;
+  }
+  if (host_doubles > w.host_cap) {
+    if (w.host) OB_HIP(hipHostFree(w.host));
+    w.host = w.host_dev = nullptr;
+    w.host_cap = 0;
+    const size_t cap = std::max<size_t>(host_doubles, 511);
+    OB_HIP(hipHostMalloc((void**)&w.host, sizeof(double) * (cap + 1), hipHostMallocCoherent));
+    std::memset(w.host, 0, sizeof(double) * (cap + 1));
+    OB_HIP(hipHostGetDevicePointer((void**)&w.host_dev, w.host, 0));
+    w.host_cap = cap;
+    w.seq = 0;
+  }
+  return w;
+}
 
 std::vector<Op> bunch_take_queue(ob_bunch* b) {
   std::vector<Op> q;
@@ -508,8 +546,9 @@ OB_API int ob_bunch_destroy(ob_bunch* b) {
   lb.erase(std::remove(lb.begin(), lb.end(), b), lb.end());
   (void)hipStreamSynchronize(ob::stream());
   for (void* p : {(void*)b->d, (void*)b->d_msize, (void*)b->d_alt, (void*)b->d_msize_alt,
-                  (void*)b->d_perm, (void*)b->d_perm_alt})
+                  (void*)b->d_perm, (void*)b->d_perm_alt, (void*)b->diag.dev})
     if (p) (void)hipFree(p);
+  if (b->diag.host) (void)hipHostFree(b->diag.host);
   delete b;
   OB_CATCH
 }

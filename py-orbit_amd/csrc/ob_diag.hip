@@ -22,51 +22,118 @@ constexpr int kThreads = 256;
 constexpr int kMaxBlocks = 1024;
 constexpr int kSums = 28;  // weight, 6 first moments, 21 products (i <= j)
 
-__device__ __forceinline__ double block_sum(double v, double* sh) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+// Sums of NV values over the workgroup's kThreads threads: each wave adds its lanes with
+// shuffles (the NV chains are independent, so their latencies overlap), one barrier, then
+// thread k < NV adds the waves' sums of value k in wave order and stores it to out[k].  A
+// barrier pair per value instead made the 28 sums cost as much as reading the particles.
+template <int NV>
+__device__ __forceinline__ void block_sums(double (&s)[NV], double* sh, double* __restrict__ out) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+    for (int k = 0; k < NV; k++) s[k] += __shfl_xor(s[k], o, 64);
+  const int w = threadIdx.x >> 6;
+  if ((threadIdx.x & 63) == 0)
+#pragma unroll
+    for (int k = 0; k < NV; k++) sh[w * NV + k] = s[k];
   __syncthreads();
-  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
-  __syncthreads();
-  double s = 0.0;
-  for (int w = 0; w < (int)(blockDim.x >> 6); w++) s += sh[w];
-  return s;
+  if (threadIdx.x < NV) {
+    double t = 0.0;
+    for (int j = 0; j < kThreads / 64; j++) t += sh[j * NV + threadIdx.x];
+    out[threadIdx.x] = t;
+  }
 }
 
+// Two particles per thread and round: twice the loads in flight (a masked lane reloads the
+// first particle with weight 0, and NaN or infinite coordinates of it are not touched).
 __global__ __launch_bounds__(kThreads) void moment_partials(DeviceBunchView v,
                                                             double* __restrict__ part) {
-  __shared__ double sh[kThreads / 64];
+  __shared__ double sh[kThreads / 64 * kSums];
   double s[kSums];
 #pragma unroll
   for (int k = 0; k < kSums; k++) s[k] = 0.0;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < v.n;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const double w = v.msize ? v.msize[i] : 1.0;
-    double c[6];
+  gptr<const double> c[6];
 #pragma unroll
-    for (int k = 0; k < 6; k++) c[k] = v.c[k][i];
-    s[0] += w;
+  for (int k = 0; k < 6; k++) c[k] = to_global((const double*)v.c[k]);
+  const gptr<const double> pm = to_global((const double*)v.msize);
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  constexpr int U = 2;
+  for (int64_t i0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i0 < v.n; i0 += U * stride) {
+    double q[U][6], w[U];
 #pragma unroll
-    for (int k = 0; k < 6; k++) s[1 + k] += w * c[k];
-    int p = 7;
+    for (int u = 0; u < U; u++) {
+      const int64_t i = i0 + u * stride < v.n ? i0 + u * stride : i0;
 #pragma unroll
-    for (int a = 0; a < 6; a++)
+      for (int k = 0; k < 6; k++) q[u][k] = c[k][i];
+      w[u] = pm ? pm[i] : 1.0;
+    }
 #pragma unroll
-      for (int b = a; b < 6; b++) s[p++] += w * c[a] * c[b];
+    for (int u = 0; u < U; u++) {
+      if (i0 + u * stride >= v.n) break;
+      s[0] += w[u];
+#pragma unroll
+      for (int k = 0; k < 6; k++) s[1 + k] += w[u] * q[u][k];
+      int p = 7;
+#pragma unroll
+      for (int a = 0; a < 6; a++)
+#pragma unroll
+        for (int b = a; b < 6; b++) s[p++] += w[u] * q[u][a] * q[u][b];
+    }
   }
-#pragma unroll
-  for (int k = 0; k < kSums; k++) {
-    const double t = block_sum(s[k], sh);
-    if (threadIdx.x == 0) part[(size_t)blockIdx.x * kSums + k] = t;
-  }
+  block_sums<kSums>(s, sh, part + (size_t)blockIdx.x * kSums);
 }
 
-__global__ __launch_bounds__(64) void moment_reduce(const double* __restrict__ part, int nblk,
-                                                    double* __restrict__ out) {
-  const int k = threadIdx.x;
-  if (k >= kSums) return;
-  double s = 0.0;
-  for (int b = 0; b < nblk; b++) s += part[(size_t)b * kSums + k];
-  out[k] = s;
+// Rows part[nblk][nt] added (OP 0) or their extrema taken (OP 1: min of even columns, max
+// of odd ones; OP 2: max) per column, nt <= 128.  One workgroup: kRedThreads / C threads
+// per column (C = nt rounded up to a power of two) walk the rows, eight loads in flight,
+// and meet in LDS in row-group order, so the result does not depend on timing.  The former
+// form, one thread per column walking up to 1024 rows one load at a time, took 215-235 us
+// for any bunch of 262k particles or more; this one takes 8-9 us.  seq_out, if given: a
+// host word that gets seq once the result is written (pinned memory).
+constexpr int kRedThreads = 1024;
+template <int OP>
+__device__ __forceinline__ double red_op(double a, double b, int k) {
+  if (OP == 0) return a + b;
+  if (OP == 1 && !(k & 1)) return b < a ? b : a;
+  return b > a ? b : a;
+}
+template <int OP>
+__device__ __forceinline__ double red_init(int k) {
+  return OP == 0 ? 0.0 : (OP == 2 ? 0.0 : ((k & 1) ? -DBL_MAX : DBL_MAX));
+}
+template <int OP>
+__global__ __launch_bounds__(kRedThreads) void row_reduce(const double* __restrict__ part,
+                                                          int nblk, int nt, int cbits,
+                                                          double* __restrict__ out,
+                                                          uint64_t* __restrict__ seq_out,
+                                                          uint64_t seq) {
+  __shared__ double sh[kRedThreads];
+  const int C = 1 << cbits, k = threadIdx.x & (C - 1), r = threadIdx.x >> cbits;
+  const int g = kRedThreads >> cbits;
+  double acc = red_init<OP>(k);
+  if (k < nt) {
+    int b = r;
+    for (; b + 7 * g < nblk; b += 8 * g) {
+      double v[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) v[u] = part[(size_t)(b + u * g) * nt + k];
+#pragma unroll
+      for (int u = 0; u < 8; u++) acc = red_op<OP>(acc, v[u], k);
+    }
+    for (; b < nblk; b += g) acc = red_op<OP>(acc, part[(size_t)b * nt + k], k);
+  }
+  sh[threadIdx.x] = acc;
+  for (int h = g >> 1; h > 0; h >>= 1) {
+    __syncthreads();
+    if (r < h) sh[threadIdx.x] = red_op<OP>(sh[threadIdx.x], sh[threadIdx.x + (h << cbits)], k);
+  }
+  if (r == 0 && k < nt) out[k] = sh[k];
+  if (seq_out) {  // the total is visible to the host before the number it watches
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0)
+      __hip_atomic_store(seq_out, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
 }
 
 // ---- extrema of the six coordinates -------------------------------------------------
@@ -79,23 +146,35 @@ __global__ __launch_bounds__(kThreads) void extrema6_partials(DeviceBunchView v,
                                                               double* __restrict__ part) {
   __shared__ double sh[kThreads / 64][12];
   double e[12];
+  gptr<const double> c[6];
 #pragma unroll
   for (int k = 0; k < 6; k++) {
     e[2 * k] = DBL_MAX;
     e[2 * k + 1] = -DBL_MAX;
+    c[k] = to_global((const double*)v.c[k]);
   }
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < v.n;
-       i += (int64_t)gridDim.x * blockDim.x) {
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  constexpr int U = 2;  // a masked lane reloads the first particle: it cannot change an extremum
+  for (int64_t i0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i0 < v.n; i0 += U * stride) {
+    double q[U][6];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int64_t i = i0 + u * stride < v.n ? i0 + u * stride : i0;
+#pragma unroll
+      for (int k = 0; k < 6; k++) q[u][k] = c[k][i];
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++)
+#pragma unroll
+      for (int k = 0; k < 6; k++) {
+        e[2 * k] = lo(e[2 * k], q[u][k]);
+        e[2 * k + 1] = hi(e[2 * k + 1], q[u][k]);
+      }
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1)
 #pragma unroll
     for (int k = 0; k < 6; k++) {
-      const double c = v.c[k][i];
-      e[2 * k] = lo(e[2 * k], c);
-      e[2 * k + 1] = hi(e[2 * k + 1], c);
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < 6; k++)
-    for (int o = 32; o > 0; o >>= 1) {
       e[2 * k] = lo(e[2 * k], __shfl_xor(e[2 * k], o, 64));
       e[2 * k + 1] = hi(e[2 * k + 1], __shfl_xor(e[2 * k + 1], o, 64));
     }
@@ -110,47 +189,26 @@ __global__ __launch_bounds__(kThreads) void extrema6_partials(DeviceBunchView v,
   }
 }
 
-__global__ __launch_bounds__(64) void extrema6_reduce(const double* __restrict__ part, int nblk,
-                                                      double* __restrict__ out) {
-  const int k = threadIdx.x;
-  if (k >= 12) return;
-  double r = (k & 1) ? -DBL_MAX : DBL_MAX;
-  for (int b = 0; b < nblk; b++) r = (k & 1) ? hi(r, part[(size_t)b * 12 + k]) : lo(r, part[(size_t)b * 12 + k]);
-  out[k] = r;
-}
-
 // ---- extremaR: largest distance from the mean transverse position -----------------------
-// Pass 1: per-workgroup sums of x and y (unweighted, as the reference's mean); pass 2: each
-// workgroup adds the sums in a fixed order, forms the mean and its particles' largest
-// distance; pass 3: the largest of the workgroups'.
+// Per-workgroup sums of x and y (unweighted, as the reference's mean), their total
+// (row_reduce), each workgroup's largest distance from the mean, the largest of those.
 __global__ __launch_bounds__(kThreads) void xy_sum_partials(DeviceBunchView v,
                                                             double* __restrict__ part) {
-  __shared__ double sh[kThreads / 64];
-  double sx = 0.0, sy = 0.0;
+  __shared__ double sh[kThreads / 64 * 2];
+  double s[2] = {0.0, 0.0};
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < v.n;
        i += (int64_t)gridDim.x * blockDim.x) {
-    sx += v.c[0][i];
-    sy += v.c[2][i];
+    s[0] += v.c[0][i];
+    s[1] += v.c[2][i];
   }
-  sx = block_sum(sx, sh);
-  __syncthreads();
-  sy = block_sum(sy, sh);
-  if (threadIdx.x == 0) {
-    part[2 * blockIdx.x] = sx;
-    part[2 * blockIdx.x + 1] = sy;
-  }
+  block_sums<2>(s, sh, part + 2 * (size_t)blockIdx.x);
 }
 
 __global__ __launch_bounds__(kThreads) void rmax_partials(DeviceBunchView v,
                                                           const double* __restrict__ sums,
-                                                          int nblk, double* __restrict__ part) {
+                                                          double* __restrict__ part) {
   __shared__ double sh[kThreads / 64];
-  double sx = 0.0, sy = 0.0;
-  for (int b = 0; b < nblk; b++) {
-    sx += sums[2 * b];
-    sy += sums[2 * b + 1];
-  }
-  const double xa = sx / (double)v.n, ya = sy / (double)v.n;
+  const double xa = sums[0] / (double)v.n, ya = sums[1] / (double)v.n;
   double r = 0.0;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < v.n;
        i += (int64_t)gridDim.x * blockDim.x) {
@@ -168,14 +226,6 @@ __global__ __launch_bounds__(kThreads) void rmax_partials(DeviceBunchView v,
     for (int w = 1; w < kThreads / 64; w++) r = sh[w] > r ? sh[w] : r;
     part[blockIdx.x] = r;
   }
-}
-
-__global__ __launch_bounds__(64) void max_reduce(const double* __restrict__ part, int nblk,
-                                                 double* __restrict__ out) {
-  if (threadIdx.x != 0) return;
-  double r = 0.0;
-  for (int b = 0; b < nblk; b++) r = part[b] > r ? part[b] : r;
-  *out = r;
 }
 
 // ---- Grid1D::binBunch along one coordinate --------------------------------------------
@@ -223,14 +273,35 @@ __global__ __launch_bounds__(kThreads) void bin1d_partials(DeviceBunchView v, Bi
   }
 }
 
+// Sixteen bins per workgroup (128-byte row segments), sixteen row groups per bin with eight
+// loads in flight each, added in row-group order: 115 us as one thread per bin walking 512
+// rows (128 bins: half a workgroup on the whole chip), 4 us so.
+constexpr int kBinCols = 16;
 __global__ __launch_bounds__(kThreads) void bin1d_reduce(const double* __restrict__ part,
                                                          int nblk, int nz,
                                                          double* __restrict__ out) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= nz) return;
+  __shared__ double sh[kThreads];
+  constexpr int g = kThreads / kBinCols;
+  const int k = blockIdx.x * kBinCols + (int)threadIdx.x % kBinCols;
+  const int r = (int)threadIdx.x / kBinCols;
   double s = 0.0;
-  for (int b = 0; b < nblk; b++) s += part[(size_t)b * nz + k];
-  out[k] = s;
+  if (k < nz) {
+    int b = r;
+    for (; b + 7 * g < nblk; b += 8 * g) {
+      double t[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) t[u] = part[(size_t)(b + u * g) * nz + k];
+#pragma unroll
+      for (int u = 0; u < 8; u++) s += t[u];
+    }
+    for (; b < nblk; b += g) s += part[(size_t)b * nz + k];
+  }
+  sh[threadIdx.x] = s;
+  __syncthreads();
+  if (r == 0 && k < nz) {
+    for (int j = 1; j < g; j++) s += sh[j * kBinCols + threadIdx.x];
+    out[k] = s;
+  }
 }
 
 // ---- computeBunchMoments: sums of x-y power products --------------------------------
@@ -240,67 +311,53 @@ __global__ __launch_bounds__(kThreads) void bin1d_reduce(const double* __restric
 // (m = 1 without the macrosize attribute); with the attribute each term also adds
 // momX[i] momY[j].  Without the attribute the statement after the loops adds
 // momX[2] momY[order] to entry [2][order] once per particle (it sits outside the braces).
-// Each lane keeps its sums in an LDS column (one wave per workgroup); the lanes' sums are
-// added in lane order, then the workgroups' in workgroup order.
+// The kernel adds momX[i] momY[j] (the divisors are the same for every particle: the host
+// divides the sums once, two roundings instead of three per particle), each thread's sums
+// in registers for the order it is compiled for.  Sums in LDS columns with two divisions
+// per term and particle took 57 us at 1M particles and order 4, against 16 us.
 constexpr int kMaxMomOrder = 12;
-constexpr int kMomLanes = 64;
+__host__ __device__ constexpr int mom_terms(int order) { return order * (order + 3) / 2; }
 
 struct XYMom {
-  int order, nterms, disp, stray;  // nterms = order (order + 3) / 2
-  double xAvg, yAvg, D, Em, b2;    // Em = E_kin + mass, b2 = beta^2
-  double px[kMaxMomOrder + 1], py[kMaxMomOrder + 1];  // xb^i, yb^j
+  int disp, stray;
+  double xAvg, yAvg, D, Em, b2;  // Em = E_kin + mass, b2 = beta^2
 };
 
-__global__ __launch_bounds__(kMomLanes) void xy_moment_partials(DeviceBunchView v, XYMom p,
-                                                                double* __restrict__ part) {
-  extern __shared__ double acc[];  // [nterms + 2][kMomLanes]
-  __shared__ double spx[kMaxMomOrder + 1], spy[kMaxMomOrder + 1];
-  const int t = threadIdx.x;
-  const int nt = p.nterms + 2;
-  for (int k = 0; k < nt; k++) acc[k * kMomLanes + t] = 0.0;
-  if (t <= p.order) {
-    spx[t] = p.px[t];
-    spy[t] = p.py[t];
-  }
-  __syncthreads();
-  const bool ms = v.msize != nullptr;
-  for (int64_t i = (int64_t)blockIdx.x * kMomLanes + t; i < v.n;
-       i += (int64_t)gridDim.x * kMomLanes) {
-    const double m = ms ? v.msize[i] : 1.0;
-    const double dispterm = p.disp ? p.D * v.c[5][i] / p.Em / p.b2 : 0.0;
-    const double dx = (v.c[0][i] - dispterm) - p.xAvg;
-    const double dy = v.c[2][i] - p.yAvg;
+template <int ORDER>
+__global__ __launch_bounds__(kThreads) void xy_moment_partials(DeviceBunchView v, XYMom p,
+                                                               double* __restrict__ part) {
+  constexpr int NT = mom_terms(ORDER) + 2;
+  __shared__ double sh[kThreads / 64 * NT];
+  double s[NT];
+#pragma unroll
+  for (int k = 0; k < NT; k++) s[k] = 0.0;
+  const gptr<const double> cx = to_global((const double*)v.c[0]);
+  const gptr<const double> cy = to_global((const double*)v.c[2]);
+  const gptr<const double> cd = to_global((const double*)v.c[5]);
+  const gptr<const double> pm = to_global((const double*)v.msize);
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < v.n;
+       i += (int64_t)gridDim.x * blockDim.x) {
+    const double m = pm ? pm[i] : 1.0;
+    const double dispterm = p.disp ? p.D * cd[i] / p.Em / p.b2 : 0.0;
+    const double dx = (cx[i] - dispterm) - p.xAvg;
+    const double dy = cy[i] - p.yAvg;
+    const double fx = pm ? m * dx : dx, fy = pm ? m * dy : dy;
+    double mX[ORDER + 1];
+    mX[0] = 1.0;
+#pragma unroll
+    for (int a = 1; a <= ORDER; a++) mX[a] = mX[a - 1] * fx;
     double mY = 1.0;
     int k = 0;
-    for (int j = 0; j < p.order; j++) {
-      double mX = 1.0;
-      for (int a = 0; a <= p.order - j; a++, k++) {
-        double s = acc[k * kMomLanes + t];
-        s += mX / spx[a] * mY / spy[j];
-        if (ms) s += mX * mY;
-        acc[k * kMomLanes + t] = s;
-        mX = ms ? mX * m * dx : mX * dx;
-      }
-      mY = ms ? mY * m * dy : mY * dy;
+#pragma unroll
+    for (int j = 0; j < ORDER; j++) {
+#pragma unroll
+      for (int a = 0; a <= ORDER - j; a++) s[k++] += mX[a] * mY;
+      mY = mY * fy;
     }
-    if (p.stray) acc[k * kMomLanes + t] += dx * dx * mY;  // momX[2] momY[order]
-    acc[(k + 1) * kMomLanes + t] += m;
+    if (p.stray) s[NT - 2] += dx * dx * mY;  // momX[2] momY[order]
+    s[NT - 1] += m;
   }
-  __syncthreads();
-  for (int k = t; k < nt; k += kMomLanes) {
-    double s = 0.0;
-    for (int l = 0; l < kMomLanes; l++) s += acc[k * kMomLanes + l];
-    part[(size_t)blockIdx.x * nt + k] = s;
-  }
-}
-
-__global__ __launch_bounds__(128) void xy_moment_reduce(const double* __restrict__ part, int nblk,
-                                                        int nt, double* __restrict__ out) {
-  const int k = threadIdx.x;
-  if (k >= nt) return;
-  double s = 0.0;
-  for (int b = 0; b < nblk; b++) s += part[(size_t)b * nt + k];
-  out[k] = s;
+  block_sums<NT>(s, sh, part + (size_t)blockIdx.x * NT);
 }
 
 // Scratch of ob_bunch_moments_noalloc: the per-workgroup partial sums (at most kMaxBlocks
@@ -320,20 +377,37 @@ namespace {
 constexpr int kMaxDevices = 64;
 double* g_scratch_dev[kMaxDevices] = {};
 
+// Column sums or extrema (row_reduce) of part[nblk][nt] into out[nt].
+template <int OP>
+void launch_row_reduce(const double* part, int nblk, int nt, double* out, hipStream_t s,
+                       uint64_t* seq_out = nullptr, uint64_t seq = 0) {
+  int cbits = 0;
+  while ((1 << cbits) < nt) cbits++;
+  OB_REQUIRE(cbits <= 7, "row_reduce: more than 128 columns");
+  hipLaunchKernelGGL(row_reduce<OP>, dim3(1), dim3(kRedThreads), 0, s, part, nblk, nt, cbits, out,
+                     seq_out, seq);
+}
+
+// The total of part[nblk][nt] to the host array out[nt] through the bunch's pinned words:
+// no copy command and no wait for the stream to drain.
+template <int OP>
+void rows_to_host(DiagWork& w, const double* part, int nblk, int nt, double* out,
+                  hipStream_t s) {
+  const uint64_t want = ++w.seq;
+  launch_row_reduce<OP>(part, nblk, nt, w.host_dev + 1, s,
+                        reinterpret_cast<uint64_t*>(w.host_dev), want);
+  OB_HIP(hipGetLastError());
+  host_wait_seq(reinterpret_cast<uint64_t*>(w.host), want, s);
+  std::memcpy(out, w.host + 1, sizeof(double) * nt);
+}
+
 // Partial sums into buf[0 .. nblk * kSums), their total at buf + nblk * kSums, copied to
 // the host array out[kSums]; waits for the copy.  Every partial row and the total are
-// written before they are read, so buf needs no clearing.  timed: record the partials
-// kernel in the kernel profiler (which creates HIP events when it is on).
-void moments_into(const DeviceBunchView& v, int nblk, double* buf, double* out, hipStream_t s,
-                  bool timed) {
-  if (timed) {
-    ProfScope ps("moment_partials");
-    hipLaunchKernelGGL(moment_partials, dim3(nblk), dim3(kThreads), 0, s, v, buf);
-  } else {
-    hipLaunchKernelGGL(moment_partials, dim3(nblk), dim3(kThreads), 0, s, v, buf);
-  }
-  hipLaunchKernelGGL(moment_reduce, dim3(1), dim3(64), 0, s, buf, nblk,
-                     buf + (size_t)nblk * kSums);
+// written before they are read, so buf needs no clearing.  Not recorded in the kernel
+// profiler (which creates HIP events when it is on).
+void moments_into(const DeviceBunchView& v, int nblk, double* buf, double* out, hipStream_t s) {
+  hipLaunchKernelGGL(moment_partials, dim3(nblk), dim3(kThreads), 0, s, v, buf);
+  launch_row_reduce<0>(buf, nblk, kSums, buf + (size_t)nblk * kSums, s);
   OB_HIP(hipGetLastError());
   OB_HIP(hipMemcpyAsync(out, buf + (size_t)nblk * kSums, sizeof(double) * kSums,
                         hipMemcpyDeviceToHost, s));
@@ -374,15 +448,12 @@ OB_API int ob_bunch_moments(ob_bunch* b, double* out) {
   }
   const int nblk =
       (int)std::min<int64_t>(ob::kMaxBlocks, (v.n + ob::kThreads - 1) / ob::kThreads);
-  double* buf = nullptr;
-  OB_HIP(hipMalloc((void**)&buf, sizeof(double) * (nblk + 1) * ob::kSums));
-  try {
-    ob::moments_into(v, nblk, buf, out, s, true);
-  } catch (...) {
-    (void)hipFree(buf);
-    throw;
+  ob::DiagWork& w = ob::bunch_diag_work(b, (size_t)nblk * ob::kSums);
+  {
+    ob::ProfScope ps("moment_partials");
+    hipLaunchKernelGGL(ob::moment_partials, dim3(nblk), dim3(ob::kThreads), 0, s, v, w.dev);
   }
-  OB_HIP(hipFree(buf));
+  ob::rows_to_host<0>(w, w.dev, nblk, ob::kSums, out, s);
   OB_CATCH
 }
 
@@ -410,7 +481,7 @@ OB_API int ob_bunch_moments_noalloc(ob_bunch* b, double* out) {
              "ob_bunch_moments_noalloc: " + std::to_string(need) +
                  " doubles of scratch needed, the maximum is " +
                  std::to_string(ob::kScratchDoubles));
-  ob::moments_into(v, nblk, ob::g_scratch_dev[dev], out, ob::stream(), false);
+  ob::moments_into(v, nblk, ob::g_scratch_dev[dev], out, ob::stream());
   OB_CATCH
 }
 
@@ -431,24 +502,12 @@ OB_API int ob_bunch_extrema(ob_bunch* b, double* out) {
   }
   const int nblk =
       (int)std::min<int64_t>(ob::kMaxBlocks, (v.n + ob::kThreads - 1) / ob::kThreads);
-  double* buf = nullptr;
-  OB_HIP(hipMalloc((void**)&buf, sizeof(double) * (nblk + 1) * 12));
-  try {
-    {
-      ob::ProfScope ps("extrema6_partials");
-      hipLaunchKernelGGL(ob::extrema6_partials, dim3(nblk), dim3(ob::kThreads), 0, s, v, buf);
-    }
-    hipLaunchKernelGGL(ob::extrema6_reduce, dim3(1), dim3(64), 0, s, buf, nblk,
-                       buf + (size_t)nblk * 12);
-    OB_HIP(hipGetLastError());
-    OB_HIP(hipMemcpyAsync(out, buf + (size_t)nblk * 12, sizeof(double) * 12,
-                          hipMemcpyDeviceToHost, s));
-    OB_HIP(hipStreamSynchronize(s));
-  } catch (...) {
-    (void)hipFree(buf);
-    throw;
+  ob::DiagWork& w = ob::bunch_diag_work(b, (size_t)nblk * 12);
+  {
+    ob::ProfScope ps("extrema6_partials");
+    hipLaunchKernelGGL(ob::extrema6_partials, dim3(nblk), dim3(ob::kThreads), 0, s, v, w.dev);
   }
-  OB_HIP(hipFree(buf));
+  ob::rows_to_host<1>(w, w.dev, nblk, 12, out, s);
   OB_CATCH
 }
 
@@ -478,28 +537,32 @@ OB_API int ob_grid1d_bin_bunch(ob_bunch* b, int axis, int by_particle, int nz, d
   const bool lds = nz <= ob::kBinLds;
   const int64_t want = (v.n + ob::kThreads - 1) / ob::kThreads;
   const int nblk = (int)std::min<int64_t>(lds ? 512 : ob::kMaxBlocks, want);
-  const size_t part_n = lds ? (size_t)nblk * nz : (size_t)nz;
-  double* buf = nullptr;
-  OB_HIP(hipMalloc((void**)&buf, sizeof(double) * (part_n + nz)));
-  std::vector<double> h((size_t)nz);
-  try {
-    double* res = buf + part_n;
-    if (lds) {
+  if (lds) {
+    ob::DiagWork& w = ob::bunch_diag_work(b, (size_t)nblk * nz, nz);
+    {
       ob::ProfScope ps("bin1d_partials");
       hipLaunchKernelGGL(ob::bin1d_partials<true>, dim3(nblk), dim3(ob::kThreads),
-                         sizeof(double) * nz, s, v, g, buf);
-      OB_HIP(hipGetLastError());
-      hipLaunchKernelGGL(ob::bin1d_reduce, dim3((nz + ob::kThreads - 1) / ob::kThreads),
-                         dim3(ob::kThreads), 0, s, buf, nblk, nz, res);
-    } else {
-      OB_HIP(hipMemsetAsync(buf, 0, sizeof(double) * nz, s));
+                         sizeof(double) * nz, s, v, g, w.dev);
+    }
+    hipLaunchKernelGGL(ob::bin1d_reduce, dim3((nz + ob::kBinCols - 1) / ob::kBinCols),
+                       dim3(ob::kThreads), 0, s, w.dev, nblk, nz, w.host_dev + 1);
+    OB_HIP(hipGetLastError());
+    OB_HIP(hipStreamSynchronize(s));
+    for (int k = 0; k < nz; k++) arr[k] += w.host[1 + k];
+    return 0;
+  }
+  double* buf = nullptr;  // a large grid's histogram is not kept
+  OB_HIP(hipMalloc((void**)&buf, sizeof(double) * nz));
+  std::vector<double> h((size_t)nz);
+  try {
+    OB_HIP(hipMemsetAsync(buf, 0, sizeof(double) * nz, s));
+    {
       ob::ProfScope ps("bin1d_partials");
       hipLaunchKernelGGL(ob::bin1d_partials<false>, dim3(nblk), dim3(ob::kThreads), 0, s, v, g,
                          buf);
-      res = buf;
     }
     OB_HIP(hipGetLastError());
-    OB_HIP(hipMemcpyAsync(h.data(), res, sizeof(double) * nz, hipMemcpyDeviceToHost, s));
+    OB_HIP(hipMemcpyAsync(h.data(), buf, sizeof(double) * nz, hipMemcpyDeviceToHost, s));
     OB_HIP(hipStreamSynchronize(s));
   } catch (...) {
     (void)hipFree(buf);
@@ -524,41 +587,40 @@ OB_API int ob_bunch_xy_moments(ob_bunch* b, int order, const double* prm, double
   const ob::DeviceBunchView v = ob::bunch_device_view(b);
   hipStream_t s = ob::stream();
   ob::XYMom p;
-  p.order = order;
-  p.nterms = order * (order + 3) / 2;
+  const bool ms = v.msize != nullptr;
   p.disp = prm[7] > 0 ? 1 : 0;
-  p.stray = (v.msize == nullptr && order >= 2) ? 1 : 0;
+  p.stray = (!ms && order >= 2) ? 1 : 0;
   p.xAvg = prm[0]; p.yAvg = prm[1]; p.D = prm[2]; p.Em = prm[3]; p.b2 = prm[4];
-  for (int k = 0; k <= ob::kMaxMomOrder; k++) {
-    p.px[k] = pow(prm[5], (double)k);
-    p.py[k] = pow(prm[6], (double)k);
-  }
-  const int nt = p.nterms + 2;
+  const int nt = ob::mom_terms(order) + 2;
   if (v.n == 0) {
     for (int k = 0; k < nt; k++) out[k] = 0.0;
     return 0;
   }
-  const int nblk = (int)std::min<int64_t>(1024, (v.n + ob::kMomLanes - 1) / ob::kMomLanes);
-  double* buf = nullptr;
-  OB_HIP(hipMalloc((void**)&buf, sizeof(double) * (size_t)(nblk + 1) * nt));
-  try {
-    {
-      ob::ProfScope ps("xy_moment_partials");
-      hipLaunchKernelGGL(ob::xy_moment_partials, dim3(nblk), dim3(ob::kMomLanes),
-                         sizeof(double) * nt * ob::kMomLanes, s, v, p, buf);
+  const int nblk =
+      (int)std::min<int64_t>(ob::kMaxBlocks, (v.n + ob::kThreads - 1) / ob::kThreads);
+  ob::DiagWork& w = ob::bunch_diag_work(b, (size_t)nblk * nt);
+  {
+    ob::ProfScope ps("xy_moment_partials");
+    switch (order) {
+#define OB_CASE(o)                                                                            \
+  case o:                                                                                     \
+    hipLaunchKernelGGL(ob::xy_moment_partials<o>, dim3(nblk), dim3(ob::kThreads), 0, s, v, p, \
+                       w.dev);                                                                \
+    break;
+      OB_CASE(1) OB_CASE(2) OB_CASE(3) OB_CASE(4) OB_CASE(5) OB_CASE(6)
+      OB_CASE(7) OB_CASE(8) OB_CASE(9) OB_CASE(10) OB_CASE(11) OB_CASE(12)
+#undef OB_CASE
+      default: break;
     }
-    OB_HIP(hipGetLastError());
-    hipLaunchKernelGGL(ob::xy_moment_reduce, dim3(1), dim3(128), 0, s, buf, nblk, nt,
-                       buf + (size_t)nblk * nt);
-    OB_HIP(hipGetLastError());
-    OB_HIP(hipMemcpyAsync(out, buf + (size_t)nblk * nt, sizeof(double) * nt,
-                          hipMemcpyDeviceToHost, s));
-    OB_HIP(hipStreamSynchronize(s));
-  } catch (...) {
-    (void)hipFree(buf);
-    throw;
   }
-  OB_HIP(hipFree(buf));
+  ob::rows_to_host<0>(w, w.dev, nblk, nt, out, s);
+  int k = 0;
+  for (int j = 0; j < order; j++)
+    for (int a = 0; a <= order - j; a++, k++) {
+      const double raw = out[k];
+      out[k] = raw / pow(prm[5], (double)a) / pow(prm[6], (double)j);
+      if (ms) out[k] += raw;
+    }
   OB_CATCH
 }
 
@@ -576,27 +638,14 @@ OB_API int ob_bunch_extrema_r(ob_bunch* b, double* rmax) {
   }
   const int nblk =
       (int)std::min<int64_t>(ob::kMaxBlocks, (v.n + ob::kThreads - 1) / ob::kThreads);
-  double* buf = nullptr;
-  OB_HIP(hipMalloc((void**)&buf, sizeof(double) * (3 * (size_t)nblk + 1)));
-  try {
-    double* sums = buf;
-    double* rpart = buf + 2 * (size_t)nblk;
-    {
-      ob::ProfScope ps("rmax_partials");
-      hipLaunchKernelGGL(ob::xy_sum_partials, dim3(nblk), dim3(ob::kThreads), 0, s, v, sums);
-      hipLaunchKernelGGL(ob::rmax_partials, dim3(nblk), dim3(ob::kThreads), 0, s, v, sums,
-                         nblk, rpart);
-    }
-    hipLaunchKernelGGL(ob::max_reduce, dim3(1), dim3(64), 0, s, rpart, nblk,
-                       buf + 3 * (size_t)nblk);
-    OB_HIP(hipGetLastError());
-    OB_HIP(hipMemcpyAsync(rmax, buf + 3 * (size_t)nblk, sizeof(double), hipMemcpyDeviceToHost,
-                          s));
-    OB_HIP(hipStreamSynchronize(s));
-  } catch (...) {
-    (void)hipFree(buf);
-    throw;
+  ob::DiagWork& w = ob::bunch_diag_work(b, 3 * (size_t)nblk + 2);
+  double *sums = w.dev, *total = w.dev + 2 * (size_t)nblk, *rpart = total + 2;
+  {
+    ob::ProfScope ps("rmax_partials");
+    hipLaunchKernelGGL(ob::xy_sum_partials, dim3(nblk), dim3(ob::kThreads), 0, s, v, sums);
+    ob::launch_row_reduce<0>(sums, nblk, 2, total, s);
+    hipLaunchKernelGGL(ob::rmax_partials, dim3(nblk), dim3(ob::kThreads), 0, s, v, total, rpart);
   }
-  OB_HIP(hipFree(buf));
+  ob::rows_to_host<2>(w, rpart, nblk, 1, rmax, s);
   OB_CATCH
 }

@@ -40,6 +40,10 @@ void ensure_init();
 // fixed scratch array of the no-allocation entry points (ob_diag.hip).
 void diag_scratch_setup(int device);
 
+// Wait until a kernel has written want to the pinned word *host (system-scope release):
+// spins for at most 20 ms, then synchronises the stream.
+void host_wait_seq(const uint64_t* host, uint64_t want, hipStream_t s);
+
 // Kernel timing with HIP events on the library stream (ob_profile_enable/_report).  A
 // ProfScope brackets one launch when profiling is on and costs nothing otherwise.
 bool profiling();
@@ -289,6 +293,16 @@ void bunch_queue(ob_bunch* b, const Op& op);
 // Apply queued ops; if ext_partials != nullptr compute partial extrema too.
 int bunch_flush(ob_bunch* b, double* ext_partials);
 int64_t bunch_size(ob_bunch* b);
+// Workspace of the diagnostics, kept with the bunch (grown on demand, freed with it): dev
+// holds at least dev_doubles, host_dev is the device address of the pinned words host:
+// word 0 the sequence number of the last result, from word 1 on at least host_doubles.
+struct DiagWork {
+  double* dev = nullptr;
+  double *host = nullptr, *host_dev = nullptr;
+  size_t dev_cap = 0, host_cap = 0;
+  uint64_t seq = 0;
+};
+DiagWork& bunch_diag_work(ob_bunch* b, size_t dev_doubles, size_t host_doubles = 128);
 // Whether the bunch belongs to a batch (its flush then applies the batch's work).
 bool bunch_in_batch(ob_bunch* b);
 // Tile sorting of the device arrays: begin returns the current and spare buffers (the

@@ -16,7 +16,6 @@
 // The Green spectrum of the even function 1/r is real and even in kx and ky, so only the
 // quadrant kx <= M0/2, ky <= M1/2 of its real part is stored (8x less than the complex
 // spectrum the reference keeps; the discarded imaginary part is rounding noise).
-#include <chrono>
 #include <cmath>
 #include <cstring>
 
@@ -157,15 +156,7 @@ const double* extrema_to_host(ExtremaLink& e, const double* partials, int nblk, 
                        reinterpret_cast<uint64_t*>(e.dev + 6), want);
   }
   OB_HIP(hipGetLastError());
-  const auto t0 = std::chrono::steady_clock::now();
-  while (__atomic_load_n(seq_host, __ATOMIC_ACQUIRE) != want) {
-    if (std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(20)) {
-      OB_HIP(hipStreamSynchronize(s));
-      OB_REQUIRE(__atomic_load_n(seq_host, __ATOMIC_ACQUIRE) == want,
-                 "bunch extrema: the reduction did not reach the host");
-      break;
-    }
-  }
+  host_wait_seq(seq_host, want, s);
   return e.host;
 }
 
