@@ -253,6 +253,120 @@ __device__ __forceinline__ void lds_fft(double* __restrict__ re, double* __restr
   fft_stages_from<N, 0, LMAX, NT, SIGN>(re, im, lines, ls, tw, nmax);
 }
 
+// ---- one line per workgroup: a small loop instead of unrolled stages -------------------
+// The 2D solves transform one line per workgroup in a few microseconds, and a step's kernels
+// follow one another, so each starts with its code out of the instruction cache (64 KiB for
+// two CUs): the unrolled radix-8 stages of lds_fft (some 5 KiB per transform) took 2.9 us for
+// 128 to 512 points alike, with their twiddles in LDS or not (row pass of 200 rows of 512
+// points 15.4 us, with this 13.2).  Here one loop body of a radix-4
+// Stockham stage (a radix-2 stage at the end for odd powers) serves every stage and both
+// directions, between two LDS buffers with one barrier per stage.
+//   a, b   N points each; the input in a, ready before the caller's barrier;
+//   tw     exp(-2 pi i q / N) at tw[q << tshift] (LDS or global), q < N / 2;
+//   sign   +1 forward (exponent -1), -1 inverse.
+// Returns the buffer that holds the result, after a barrier; the other is free.
+template <int N, int NT>
+__device__ __forceinline__ double2* line_fft(double2* a, double2* b, const double2* tw,
+                                             int tshift, double sign) {
+#pragma clang fp contract(fast)
+  constexpr int L = clog2(N);
+  static_assert(N >= 8, "line_fft: at least 8 points");
+#pragma unroll 1
+  for (int ls = 0; ls + 1 < L; ls += 2) {
+    const int Ns = 1 << ls;
+#pragma unroll 1
+    for (int j = threadIdx.x; j < N / 4; j += NT) {
+      const int k = j & (Ns - 1);
+      const double2 v0 = a[j], x1 = a[j + N / 4], x2 = a[j + N / 2], x3 = a[j + 3 * (N / 4)];
+      double2 w = tw[(k << (L - 2 - ls)) << tshift];
+      w.y *= sign;
+      const double2 w2 = make_double2(w.x * w.x - w.y * w.y, 2.0 * w.x * w.y);
+      const double2 w3 = make_double2(w2.x * w.x - w2.y * w.y, w2.x * w.y + w2.y * w.x);
+      const double2 v1 = make_double2(x1.x * w.x - x1.y * w.y, x1.x * w.y + x1.y * w.x);
+      const double2 v2 = make_double2(x2.x * w2.x - x2.y * w2.y, x2.x * w2.y + x2.y * w2.x);
+      const double2 v3 = make_double2(x3.x * w3.x - x3.y * w3.y, x3.x * w3.y + x3.y * w3.x);
+      const double2 s02 = make_double2(v0.x + v2.x, v0.y + v2.y);
+      const double2 d02 = make_double2(v0.x - v2.x, v0.y - v2.y);
+      const double2 s13 = make_double2(v1.x + v3.x, v1.y + v3.y);
+      // -i (v1 - v3) forward, +i (v1 - v3) inverse
+      const double2 e13 = make_double2(sign * (v1.y - v3.y), -sign * (v1.x - v3.x));
+      double2* o = b + ((j - k) << 2) + k;
+      o[0] = make_double2(s02.x + s13.x, s02.y + s13.y);
+      o[Ns] = make_double2(d02.x + e13.x, d02.y + e13.y);
+      o[2 * Ns] = make_double2(s02.x - s13.x, s02.y - s13.y);
+      o[3 * Ns] = make_double2(d02.x - e13.x, d02.y - e13.y);
+    }
+    __syncthreads();
+    double2* t = a;
+    a = b;
+    b = t;
+  }
+  if constexpr (L & 1) {
+#pragma unroll 1
+    for (int j = threadIdx.x; j < N / 2; j += NT) {
+      const double2 v0 = a[j], x1 = a[j + N / 2];
+      double2 w = tw[j << tshift];
+      w.y *= sign;
+      const double2 v1 = make_double2(x1.x * w.x - x1.y * w.y, x1.x * w.y + x1.y * w.x);
+      b[j] = make_double2(v0.x + v1.x, v0.y + v1.y);
+      b[j + N / 2] = make_double2(v0.x - v1.x, v0.y - v1.y);
+    }
+    __syncthreads();
+    double2* t = a;
+    a = b;
+    b = t;
+  }
+  return a;
+}
+
+// The LDS of a line_fft kernel: two line buffers and, up to 1024 points, the twiddles, loaded
+// beside the kernel's data at its start and stored with it (commit, before the barrier).
+__host__ __device__ constexpr bool line_tw_in_lds(int n) { return n <= 1024; }
+__host__ __device__ constexpr size_t line_lds_bytes(int n) {
+  return sizeof(double2) * (2 * n + (line_tw_in_lds(n) ? n / 2 : 0));
+}
+template <int N, int NT>
+struct LineFft {
+  static constexpr bool LDS = line_tw_in_lds(N);
+  static constexpr int CNT = N / 2, IT = LDS ? (CNT + NT - 1) / NT : 1;
+  double2 *a, *b;
+  const double2* tw;
+  int tshift;
+  double2 v[IT];
+  __device__ __forceinline__ LineFft(double* lds, const double2* __restrict__ tw_, int nmax)
+      : a((double2*)lds), b((double2*)lds + N), tw(tw_) {
+    tshift = 0;
+    while ((N << tshift) < nmax) tshift++;
+    if constexpr (LDS) {
+#pragma unroll
+      for (int u = 0; u < IT; u++) {
+        const int i = (int)threadIdx.x + u * NT;
+        v[u] = tw_[(i < CNT ? i : 0) << tshift];
+      }
+    }
+  }
+  __device__ __forceinline__ void commit() {
+    if constexpr (LDS) {
+      double2* t = b + N;
+#pragma unroll
+      for (int u = 0; u < IT; u++) {
+        const int i = (int)threadIdx.x + u * NT;
+        if (i < CNT) t[i] = v[u];
+      }
+      tw = t;
+      tshift = 0;
+    }
+  }
+  // The transform of the line in a (see line_fft); afterwards a holds the result.
+  __device__ __forceinline__ void run(double sign) {
+    double2* r = line_fft<N, NT>(a, b, tw, tshift, sign);
+    if (r != a) {
+      b = a;
+      a = r;
+    }
+  }
+};
+
 // ---- transforms with register-resident ends ------------------------------------------
 // A plan runs the radices of fft_radix in order (REV = false) or reversed (REV = true); any
 // order is a valid Stockham factorisation.  The first stage of a plan takes its butterflies

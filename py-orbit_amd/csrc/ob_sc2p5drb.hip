@@ -3,18 +3,20 @@
 // Per trackBunch (SpaceChargeCalc2p5Drb.cc:110-168), all on the library stream with no
 // host round trip:
 //   1. fused map kernel flushes the bunch's queued maps and emits per-block extrema;
-//   2. bin     (every block reduces the extrema and sizes the grids, bunchAnalysis
-//               :170-213): clears rho, counts particles per tile and writes per-block rows
-//               of the periodic 2-point z line density (Grid1D.cc:241-275, 568-626);
-//   3. deposit : 9-point TSC charge (Grid2D.cc:120-166).  Grids up to 128x128 nodes: each
-//               workgroup deposits its particles into a private copy of the grid in LDS
-//               and adds it to rho with FP64 atomics.  Larger grids: counting-sort scatter
-//               of x, y by tile, then one LDS tile block per work item;
-//   4. post    (1 block): dlambda/dz by 3-point LSQ (:257-310), rho moments (:229-254),
-//                         kick factors;
-//   5. Poisson (3 kernels, PoissonSolverFFT2D.cc:174-256): row r2c of two rows per complex
-//      FFT, column FFT x Green x inverse column FFT (zero-padding pruned: only the nx
-//      non-zero rows are read and only the nx needed rows written), row c2r;
+//   2. deposit: every workgroup reduces the extrema and sizes the grids (bunchAnalysis,
+//               :170-213), then puts its particles' 9-point TSC charge (Grid2D.cc:120-166) and
+//               periodic 2-point z line density (Grid1D.cc:241-275, 568-626) into LDS copies
+//               of a slab of grid rows and of the z bins, which it stores whole;
+//   3. rows    : the copies of a grid row added into rho, the row's share of the rho moments,
+//               its r2c transform; one more workgroup adds the line densities;
+//   4. columns : column FFT x Green x inverse column FFT (PoissonSolverFFT2D.cc:174-256;
+//               zero-padding pruned: only the nx non-zero rows are read and written); two more
+//               workgroups: moments and kick factors (:229-254), dlambda/dz by 3-point LSQ
+//               (:257-310);
+//   5. rows    : c2r of two rows per complex FFT;
+//      Grids whose rows need more than four slabs of LDS take a tile sort instead of 2: bin
+//      (grid, tile counts, line density), counting-sort scatter of x, y by tile, one LDS tile
+//      block per work item; the row pass then reads a finished rho.
 //   6. the kick (:146-167) is queued on the bunch and runs fused into the next map kernel.
 #include <algorithm>
 #include <cmath>
@@ -47,14 +49,23 @@ constexpr int kDepositThreads = 256;
 constexpr int kMaxZBinsLDS = 4096;
 constexpr int kUnroll = 4;  // particles per thread whose loads are issued together
 constexpr int kFFTThreads = 256;
-// Private-grid single-bunch deposit: grids up to kPrivNodes nodes (128 KiB of LDS),
-// bunches up to kPrivMaxParticles, kPrivPerBlock particles per workgroup of kPrivThreads
-// (at 100k particles on 128x128: 12.0 us against 18.6 us for the tile sort's scatter and
-// deposit; 2048 particles per workgroup 12.6 us, 4096 15.7 us, 512 11.7 us).
-constexpr int kPrivNodes = 128 * 128;
-constexpr int64_t kPrivMaxParticles = 1 << 18;
-constexpr int64_t kPrivPerBlock = 1024;
-constexpr int kPrivThreads = 1024;
+// Grid-copy deposit of a single bunch (sc2d_gdeposit): the x rows of the grid are cut into
+// at most kSlabMax slabs whose LDS copy (rows with a one-node halo, plus the z bins) fits
+// kSlabLds bytes, in workgroups of kSlabThreads.
+constexpr int kSlabLds = 150 * 1024;
+constexpr int kSlabMax = 4;  // 256 x 256: 2M 2301 us a cell as a tile sort, 1685 in four slabs
+constexpr int kSlabMaxNy = 512;  // the row pass sums a row's copies in LDS
+constexpr int kSlabThreads = 1024;
+// Parts of kSlabPart particles (1024 up to sixteen of them), at most one workgroup per CU.
+// Grids that fit one slab take two up to kSlabSplitMax particles: each slab's workgroups read
+// the whole part, but there are half as many copies to store and add (100k on 128 x 128, the
+// FODO cell of 12 steps: 1 slab of 98 parts 468 us, 2 of 98 453, 2 of 49 432, 4 of 49 434, 4 of
+// 25 461; 10k on 64 x 64: 1 of 10 344, 2 of 10 338, 2 of 5 355).  Above, reading and testing
+// the particles twice costs more (2M on 128 x 128: 1 of 256 1241, 2 of 128 1277).  An even
+// number of slabs cuts a centred beam evenly: where three would do, four are taken (300k on
+// 200 x 200: 3 of 74 714, 4 of 64 653).
+constexpr int64_t kSlabPart = 2048;
+constexpr int64_t kSlabSplitMax = 1 << 17;
 
 struct SC2DParams {
   int nx, ny, nz, nblk;       // grid sizes, number of extrema partial blocks
@@ -84,30 +95,56 @@ struct Grid2Step {
   double sol[4];    // SpaceChargeCalc2p5D: the solver box after this step
 };
 
-// Every thread of the block gets the grid of partials [pb, pe) (blockDim.x <= 1024).
-// st is read (entry P.par) only for SpaceChargeCalc2p5D.
+// Every thread of the block gets the grid of partials [pb, pe) (blockDim.x <= 1024, a
+// multiple of 64).  st is read (entry P.par) only for SpaceChargeCalc2p5D.  The first four
+// waves, one per SIMD, read the partials (all sixteen would queue 1152 shuffles on the LDS);
+// their extrema meet in LDS and wave 0 alone reduces them and sizes the grid.  One thread
+// walking sixteen rows of six values, as before, took 5.5 us of a 1024-thread workgroup.
+constexpr int kGridWaves = 4;
 __device__ __forceinline__ void sc2d_grid_body(const SC2DParams& P,
                                                const double* __restrict__ partials, int pb,
                                                int pe, const SC2DState* st, Grid2Step& out) {
-  __shared__ double red[16][6];
+  __shared__ double red[6][kGridWaves];
   __shared__ Grid2Step gs;
+  const int nw = min((int)(blockDim.x >> 6), kGridWaves), nt = 64 * nw;
   double r[6] = {DBL_MAX, -DBL_MAX, DBL_MAX, -DBL_MAX, DBL_MAX, -DBL_MAX};
-  for (int b = pb + threadIdx.x; b < pe; b += blockDim.x)
-    for (int k = 0; k < 6; k++) {
-      const double v = partials[b * 6 + k];
-      r[k] = (k & 1) ? fmax(r[k], v) : fmin(r[k], v);
+  if ((int)threadIdx.x < nt) {
+    const gptr<const double> part = to_global(partials);
+    constexpr int U = 4;  // rows in flight; a row past the last repeats the first
+    for (int b = pb + (int)threadIdx.x; b < pe; b += U * nt) {
+      double v[U][6];
+#pragma unroll
+      for (int u = 0; u < U; u++)
+#pragma unroll
+        for (int k = 0; k < 6; k++)
+          v[u][k] = part[(int64_t)(b + u * nt < pe ? b + u * nt : b) * 6 + k];
+#pragma unroll
+      for (int u = 0; u < U; u++)
+#pragma unroll
+        for (int k = 0; k < 6; k++) r[k] = (k & 1) ? fmax(r[k], v[u][k]) : fmin(r[k], v[u][k]);
     }
-  for (int k = 0; k < 6; k++)
-    for (int o = 32; o > 0; o >>= 1) {
-      const double v = __shfl_xor(r[k], o, 64);
-      r[k] = (k & 1) ? fmax(r[k], v) : fmin(r[k], v);
-    }
-  if ((threadIdx.x & 63) == 0)
-    for (int k = 0; k < 6; k++) red[threadIdx.x >> 6][k] = r[k];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+      for (int k = 0; k < 6; k++) {
+        const double v = __shfl_xor(r[k], o, 64);
+        r[k] = (k & 1) ? fmax(r[k], v) : fmin(r[k], v);
+      }
+    if ((threadIdx.x & 63) == 0)
+#pragma unroll
+      for (int k = 0; k < 6; k++) red[k][threadIdx.x >> 6] = r[k];
+  }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int w = 1; w < (int)(blockDim.x >> 6); w++)
-      for (int k = 0; k < 6; k++) r[k] = (k & 1) ? fmax(r[k], red[w][k]) : fmin(r[k], red[w][k]);
+  if (threadIdx.x < 64) {
+#pragma unroll
+    for (int k = 0; k < 6; k++) {
+      r[k] = red[k][0];
+#pragma unroll
+      for (int w = 1; w < kGridWaves; w++) {
+        const double v = red[k][w < nw ? w : 0];
+        r[k] = (k & 1) ? fmax(r[k], v) : fmin(r[k], v);
+      }
+    }
     Grid2Step g;
     for (int k = 0; k < 6; k++) g.ext[k] = r[k];
     double xMin = r[0], xMax = r[1], yMin = r[2], yMax = r[3];
@@ -169,11 +206,26 @@ __device__ __forceinline__ void sc2d_grid_body(const SC2DParams& P,
     g.zMin = zMin;
     g.zMax = zMax;
     g.dz = (zMax - zMin) / P.nz;        // Grid1D.cc:88-93
-    gs = g;
+    if (threadIdx.x == 0) gs = g;
   }
   __syncthreads();
   out = gs;
 }
+
+// Grid-copy deposit: workgroup s * parts + p deposits the particles of part p whose TSC
+// centre row lies in slab s (centre rows 1 + s * rows .. (s + 1) * rows) into its own LDS
+// copy of the slab's nodes (rows s * rows .. s * rows + rows + 1, R = rows + 2 of them) and
+// stores it as copy s * parts + p.
+struct SlabDep {
+  int slabs, parts, rows, R;
+  int64_t per;     // particles per part
+  double* copies;  // [slabs * parts][R * ny]
+  double* zpart;   // [parts][nz] z line densities
+  double* mrows;   // [nx][5] rho moments of the grid rows, written by the row pass
+  int green_blocks;  // SpaceChargeCalc2p5D: workgroups after the deposit's that transform
+  double2* gspec;    // the rows of a new Green function into gspec ([M0][H]); 0 otherwise
+  int M0;
+};
 
 // The step's grid into the state; on a zero-extent bunch the grid of the last good step
 // stays (it is not used) and the status word reports it.
@@ -293,9 +345,8 @@ __device__ __forceinline__ void hist_load(const DeviceBunchView& v, double macro
 // PIPE: each pass's loads are issued before the previous pass is binned (the single-bunch
 // kernel, whose workgroups make one or two passes; the batch's, with many, keep their
 // registers for occupancy instead); pre: the first pass's particles, already loaded (by
-// hist_load at `first`), or null.  COUNT: count particles per tile (not needed by the
-// private-grid deposit).
-template <bool PIPE, bool COUNT = true>
+// hist_load at `first`), or null.
+template <bool PIPE>
 __device__ __forceinline__ void sc2d_hist_body(const SC2DParams& P, const DeviceBunchView& v,
                                                const Grid2Step& g, const Tile2D& tg,
                                                double* __restrict__ zg, double* __restrict__ zrow,
@@ -329,10 +380,8 @@ __device__ __forceinline__ void sc2d_hist_body(const SC2DParams& P, const Device
 #pragma unroll
       for (int u = 0; u < kUnroll; u++) {
         if (i0 + u * stride >= end) break;
-        if (COUNT) {
-          const int k = tile2d_key(tg, P.nx, P.ny, g, c.x[u], c.y[u]);
-          if (k >= 0) atomicAdd(&lh[k], 1u);
-        }
+        const int k = tile2d_key(tg, P.nx, P.ny, g, c.x[u], c.y[u]);
+        if (k >= 0) atomicAdd(&lh[k], 1u);
         // Grid1D::binValue (Grid1D.cc:422-440)
         if (!(c.z[u] < g.zMin || c.z[u] > g.zMax)) {
           int i0z, ip;
@@ -583,7 +632,6 @@ __device__ __forceinline__ void sc2d_tdeposit_body(const SC2DParams& P, const Gr
 // Single bunch: the grid from the extrema partials in every block (block 0 writes the
 // state and clears the scatter cursors); blocks clear rho in turn (it is next written by
 // the deposit, two launches later) and write their z line density rows.
-template <bool COUNT>
 __global__ __launch_bounds__(kDepositThreads) void sc2d_bin(SC2DParams P, DeviceBunchView v,
                                                             const double* __restrict__ partials,
                                                             SC2DState* st, SC2DState* gate,
@@ -608,7 +656,7 @@ __global__ __launch_bounds__(kDepositThreads) void sc2d_bin(SC2DParams P, Device
   const int ng = P.nx * P.ny;
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < ng; i += gridDim.x * blockDim.x)
     rho[i] = 0.0;
-  sc2d_hist_body<true, COUNT>(P, v, g, tg, nullptr, tg.zpart + (size_t)blockIdx.x * P.nz, first, v.n, stride,
+  sc2d_hist_body<true>(P, v, g, tg, nullptr, tg.zpart + (size_t)blockIdx.x * P.nz, first, v.n, stride,
                  dyn, (uint32_t*)(dyn + P.nz), nullptr, &pre);
 }
 
@@ -635,98 +683,180 @@ __global__ __launch_bounds__(kDepositThreads) void sc2d_tdeposit(SC2DParams P,
                      acc, moments ? tg.mpart + (size_t)blockIdx.x * 5 : nullptr);
 }
 
-// Single bunch, grids that fit in LDS (nx*ny <= kPrivNodes): deposit without the tile
-// sort.  Workgroup b takes particles [b*per, min(n, (b+1)*per)) in particle order and
-// deposits them (Grid2D::binValue, Grid2D.cc:142-166, the same weights as the tiled
-// deposit) into its own copy of the whole grid in LDS, then adds the non-zero nodes to
-// rho with global atomics and its share of the rho moments to mpart row b.  Block 0 sets
-// the row count the post pass reads and keeps the tile counts zero for the tiled path.
-__global__ __launch_bounds__(kPrivThreads) void sc2d_pdeposit(SC2DParams P, DeviceBunchView v,
-                                                                 const SC2DState* st, Tile2D tg,
-                                                                 int64_t per,
-                                                                 double* __restrict__ rho_ptr,
-                                                                 int moments) {
+// Green function of PoissonSolverFFT2D::_defineGreenF (:115-172) at point (i, j) of the
+// padded M0 x M1 grid.
+__device__ __forceinline__ double green2d_value(int i, int j, int M0, int M1, double dx,
+                                                double dy) {
+  const int ii = (i <= M0 / 2) ? i : M0 - i;
+  const int jj = (j <= M1 / 2) ? j : M1 - j;
+  const double rTransX = ii * dx, rTransY = jj * dy;
+  const double rTot2 = rTransX * rTransX + rTransY * rTransY;
+  return (ii != 0 || jj != 0) ? -log(rTot2) / 2 : 0.0;
+}
+
+// Row pairs of the new Green function's row transforms per workgroup of sc2d_gdeposit.
+__host__ __device__ constexpr int green_pairs(int n) { return n >= 1024 ? 1 : 4; }
+
+// Single bunch: grid, z line density and charge of the step in one pass over x, y, z, for
+// grids whose rows fit the LDS in at most kSlabMax slabs.  Every workgroup sizes the grid
+// from the extrema partials (workgroup 0 writes the state), deposits its part of the bunch
+// (Grid2D::binValue, Grid2D.cc:142-166) into its LDS copy of a slab and stores the copy
+// whole; the row pass adds the copies.  There is no rho to clear beforehand, no tile sort
+// and no global atomic: at 100k on 128 x 128 it takes 11.9 us in the place of a bin pass
+// (7.4 us) and a private-grid deposit with atomics (11.8 us), at 1M on 200 x 150 26 us in the
+// place of bin (21 us), scatter (20 us) and tile deposit (25 us).  What bounds it is the LDS
+// atomic rate (nine per particle, 0.6 clocks a lane) and, for few particles, the extrema and
+// grid (2.5 us), clearing and storing the copy (2 us).  The workgroups of a part are `parts`
+// apart, so with a multiple of 8 parts its slabs read x, y, z through the same L2.
+// GN > 0: SpaceChargeCalc2p5D, M1 = GN; the workgroups after the deposit's transform the
+// rows of the Green function on the new solver box when the grid asks for a rebuild.
+template <int GN>
+__global__ __launch_bounds__(kSlabThreads) void sc2d_gdeposit(
+    SC2DParams P, DeviceBunchView v, const double* __restrict__ partials, SC2DState* st,
+    SC2DState* gate, SlabDep D, int* status, const double2* __restrict__ tw, int nmax) {
   extern __shared__ double grid[];
-  const Grid2Step g = sc2d_load_grid(st);
-  if (blockIdx.x == 0) {
-    for (int t = threadIdx.x; t < tg.ntiles; t += blockDim.x) tg.counts[t] = 0u;
-    if (threadIdx.x == 0) *tg.nitems = g.skip ? 0u : gridDim.x;
-  }
-  if (g.skip) return;
+  const int slab = (int)blockIdx.x / D.parts, part = (int)blockIdx.x - slab * D.parts;
+  const bool dep = GN == 0 || slab < D.slabs;
+  const int nx = P.nx, ny = P.ny, nz = P.nz, nodes = D.R * ny;
+  const bool doz = dep && (part % D.slabs) == slab;
+  double* zl = grid + nodes;
   const gptr<const double> px = to_global((const double*)v.c[0]);
   const gptr<const double> py = to_global((const double*)v.c[2]);
+  const gptr<const double> pz = to_global((const double*)v.c[4]);
   const gptr<const double> pm = to_global((const double*)v.msize);
-  const gptr<double> rho = to_global(rho_ptr);
-  const int nx = P.nx, ny = P.ny, nodes = nx * ny;
-  const int64_t lo = (int64_t)blockIdx.x * per, hi = min(v.n, lo + per);
+  const int64_t lo = (int64_t)part * D.per, hi = dep ? min(v.n, lo + D.per) : lo;
   const int64_t stride = blockDim.x;
   // kUnroll particles per thread per pass, loaded together; the first pass's loads go out
-  // before the LDS grid is cleared
-  double x[kUnroll], y[kUnroll], m[kUnroll];
+  // before the grid is computed and the LDS cleared
+  double x[kUnroll], y[kUnroll], z[kUnroll], m[kUnroll];
   auto load = [&](int64_t i0) {
 #pragma unroll
     for (int u = 0; u < kUnroll; u++) {
       const int64_t i = i0 + u * stride;
       x[u] = i < hi ? px[i] : 0.0;
       y[u] = i < hi ? py[i] : 0.0;
+      z[u] = (doz && i < hi) ? pz[i] : 0.0;
       m[u] = pm ? (i < hi ? pm[i] : 0.0) : P.macrosize;
     }
   };
   load(lo + threadIdx.x);
-  for (int c = threadIdx.x; c < nodes; c += blockDim.x) grid[c] = 0.0;
-  __syncthreads();
+  if (dep)
+    for (int c = threadIdx.x; c < nodes + (doz ? nz : 0); c += blockDim.x) grid[c] = 0.0;
+  Grid2Step g;
+  sc2d_grid_body(P, partials, 0, P.nblk, st, g);  // (barriers: the copy is clear as well)
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    sc2d_write_state(st, g);
+    if (P.plain) sc2d_write_solver(P, st, gate, g);
+    if (!g.skip)  // PoissonSolverFFT2D.cc:216
+      st->scale_coeff = log((P.plain ? st->sdx : P.dx_solver) / g.dx);
+    if (g.skip) *status = 1;  // zero extent: the reference aborts (:176-189)
+  }
+  if constexpr (GN > 0) {
+    if (!dep) {  // PoissonSolverFFT2D::setGridXY (PoissonSolverFFT2D.cc:103-111)
+      if (!g.rebuild) return;
+      constexpr int LP = green_pairs(GN), ls = fft_line_stride(GN), H = GN / 2 + 1;
+      double* re = grid;
+      double* im = grid + LP * ls;
+      const double sdx = (g.sol[1] - g.sol[0]) / (nx - 1), sdy = (g.sol[3] - g.sol[2]) / (ny - 1);
+      const int pair0 = ((int)blockIdx.x - D.slabs * D.parts) * LP;
+      for (int k = threadIdx.x; k < LP * GN; k += kSlabThreads) {
+        const int l = k / GN, j = k - l * GN;
+        re[l * ls + j] = green2d_value(2 * (pair0 + l), j, D.M0, GN, sdx, sdy);
+        im[l * ls + j] = green2d_value(2 * (pair0 + l) + 1, j, D.M0, GN, sdx, sdy);
+      }
+      __syncthreads();
+      lds_fft<GN, LP, kSlabThreads, -1>(re, im, LP, ls, tw, nmax);
+      for (int k = threadIdx.x; k < LP * H; k += kSlabThreads) {
+        const int l = k / H, j = k - l * H;
+        const int r = 2 * (pair0 + l), nk = (GN - j) & (GN - 1);
+        if (r >= D.M0) continue;
+        const double zr = re[l * ls + j], zi = im[l * ls + j];
+        const double nr = re[l * ls + nk], ni = im[l * ls + nk];
+        D.gspec[(int64_t)r * H + j] = make_double2((zr + nr) * 0.5, (zi - ni) * 0.5);
+        D.gspec[(int64_t)(r + 1) * H + j] = make_double2((zi + ni) * 0.5, -(zr - nr) * 0.5);
+      }
+      return;
+    }
+  }
   const double xMin = g.xMin, yMin = g.yMin, dx = g.dx, dy = g.dy;
-  for (int64_t i0 = lo + threadIdx.x; i0 < hi; i0 += kUnroll * stride) {
-    if (i0 != lo + (int64_t)threadIdx.x) load(i0);
+  const int row0 = slab * D.rows;  // first grid row of the copy
+  const int c0 = row0 + 1, c1 = min(nx - 2, row0 + D.rows);  // its centre rows
+  if (!g.skip)
+    for (int64_t i0 = lo + threadIdx.x; i0 < hi; i0 += kUnroll * stride) {
+      if (i0 != lo + (int64_t)threadIdx.x) load(i0);
 #pragma unroll
-    for (int u = 0; u < kUnroll; u++) {
-      if (i0 + u * stride >= hi) break;
-      if (x[u] < g.xMin || x[u] > g.xMax || y[u] < g.yMin || y[u] > g.yMax) continue;
-      int iX, iY;
-      double xF, yF;
-      node_ind_frac(x[u], xMin, dx, nx, iX, xF);
-      node_ind_frac(y[u], yMin, dy, ny, iY, yF);
-      const double xF2 = xF * xF, yF2 = yF * yF;
-      const double wx[3] = {0.5 * (0.25 - xF + xF2), 0.75 - xF2, 0.5 * (0.25 + xF + xF2)};
-      const double wy[3] = {0.5 * (0.25 - yF + yF2), 0.75 - yF2, 0.5 * (0.25 + yF + yF2)};
-      double* base = grid + (iX - 1) * ny + (iY - 1);  // 1 <= iX <= nx-2, 1 <= iY <= ny-2
+      for (int u = 0; u < kUnroll; u++) {
+        if (i0 + u * stride >= hi) break;
+        // Grid1D::binValue (Grid1D.cc:422-440)
+        if (doz && !(z[u] < g.zMin || z[u] > g.zMax)) {
+          int i0z, ip;
+          double w0, wp;
+          grid1d_ind_wz(z[u], g.zMin, g.dz, nz, i0z, ip, w0, wp);
+          if (nz > 1) {
+            atomicAdd(&zl[i0z], w0 * m[u]);
+            atomicAdd(&zl[ip], wp * m[u]);
+          } else {
+            atomicAdd(&zl[0], m[u]);
+          }
+        }
+        if (x[u] < g.xMin || x[u] > g.xMax || y[u] < g.yMin || y[u] > g.yMax) continue;
+        int iX, iY;
+        double xF, yF;
+        node_ind_frac(x[u], xMin, dx, nx, iX, xF);
+        if (iX < c0 || iX > c1) continue;
+        node_ind_frac(y[u], yMin, dy, ny, iY, yF);
+        const double xF2 = xF * xF, yF2 = yF * yF;
+        const double wx[3] = {0.5 * (0.25 - xF + xF2), 0.75 - xF2, 0.5 * (0.25 + xF + xF2)};
+        const double wy[3] = {0.5 * (0.25 - yF + yF2), 0.75 - yF2, 0.5 * (0.25 + yF + yF2)};
+        double* base = grid + (iX - 1 - row0) * ny + (iY - 1);  // 1 <= iY <= ny-2
 #pragma unroll
-      for (int a = 0; a < 3; a++)
+        for (int a = 0; a < 3; a++)
 #pragma unroll
-        for (int c = 0; c < 3; c++) atomicAdd(base + a * ny + c, wx[a] * wy[c] * m[u]);
+          for (int c = 0; c < 3; c++) atomicAdd(base + a * ny + c, wx[a] * wy[c] * m[u]);
+      }
     }
-  }
   __syncthreads();
-  double mom[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-  // node c = gx*ny + gy, stepped by blockDim.x without a division per node
-  const int step_x = (int)blockDim.x / ny, step_y = (int)blockDim.x - step_x * ny;
-  int gx = (int)threadIdx.x / ny, gy = (int)threadIdx.x - gx * ny;
-  for (int c = threadIdx.x; c < nodes; c += blockDim.x) {
-    const double val = grid[c];
-    if (val != 0.0) {
-      global_add(rho + c, val);
-      moment_add(mom, val, gx, gy, xMin, dx);
-    }
-    gx += step_x;
-    gy += step_y;
-    if (gy >= ny) {
-      gy -= ny;
-      gx++;
+  if (!g.skip) {
+    const gptr<double> out = to_global(D.copies + (size_t)blockIdx.x * nodes);
+    for (int c = threadIdx.x; c < nodes; c += blockDim.x) out[c] = grid[c];
+  }
+  if (doz)
+    for (int i = threadIdx.x; i < nz; i += blockDim.x) D.zpart[(size_t)part * nz + i] = zl[i];
+}
+
+// Sum of the slab copies at column j of grid row gx, copies first, first + step, ... of each
+// slab that holds the row (two where a slab ends): rounds of eight loads in flight, those past
+// the last copy repeating it with weight 0.
+__device__ __forceinline__ double slab_sum(const SlabDep& D, int ny, int gx, int j, int first,
+                                           int step) {
+  const int s1 = min(D.slabs - 1, gx / D.rows);
+  const int s0 = gx >= 2 ? (gx - 2) / D.rows : 0;
+  const gptr<const double> cp = to_global((const double*)D.copies);
+  const int64_t ld = (int64_t)D.R * ny;
+  double acc = 0.0;
+  for (int s = s0; s <= s1; s++) {
+    const int64_t at = (int64_t)s * D.parts * ld + (int64_t)(gx - s * D.rows) * ny + j;
+    for (int p = first; p < D.parts; p += 8 * step) {
+      double t[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++)
+        t[u] = cp[at + (p + u * step < D.parts ? p + u * step : p) * ld];
+#pragma unroll
+      for (int u = 0; u < 8; u++)
+        if (p + u * step < D.parts) acc += t[u];
     }
   }
-  if (moments) {
-    __shared__ double red[kPrivThreads / 64][5];
-    for (int k = 0; k < 5; k++)
-      for (int o = 32; o > 0; o >>= 1) mom[k] += __shfl_xor(mom[k], o, 64);
-    if ((threadIdx.x & 63) == 0)
-      for (int k = 0; k < 5; k++) red[threadIdx.x >> 6][k] = mom[k];
-    __syncthreads();
-    if (threadIdx.x < 5) {
-      double sum = 0.0;
-      for (int w = 0; w < (int)(blockDim.x >> 6); w++) sum += red[w][threadIdx.x];
-      tg.mpart[(size_t)blockIdx.x * 5 + threadIdx.x] = sum;
-    }
-  }
+  return acc;
+}
+
+// rho from the slab copies, when something reads it before the row pass (the denoiser).
+__global__ __launch_bounds__(256) void sc2d_slab_rho(SlabDep D, int nx, int ny,
+                                                     const SC2DState* st,
+                                                     double* __restrict__ rho) {
+  if (st->skip) return;
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= nx * ny) return;
+  rho[t] = slab_sum(D, ny, t / ny, t - (t / ny) * ny, 0, 1);
 }
 
 // ---- 4: post (one block) ---------------------------------------------------
@@ -748,23 +878,26 @@ __device__ __forceinline__ double ipow(double x, int j) {  // exact for the smal
 }
 
 // zg: when zpart is given, the sum of its zrows rows of per-block line densities.
-// Moments: the sum of the deposit items' partial moments mpart[nitems][5], or (mpart
-// nullptr, when rho was changed after the deposit) a pass over rho.
+// Moments: the sum of the deposit items' partial moments mpart[nitems][5] (or mpart[mrows][5]
+// without nitems: the solve beside this pass reads the scale coefficient, which the deposit
+// has set), or (mpart nullptr, when rho was changed after the deposit) a pass over rho.
 __device__ __forceinline__ void sc2d_post_body(const SC2DParams& P, SC2DState* st,
                                                const double* __restrict__ rho,
                                                double* __restrict__ zg,
                                                double* __restrict__ zd,
                                                const double* __restrict__ zpart, int zrows,
                                                const double* __restrict__ mpart,
-                                               const uint32_t* nitems, int part = 3) {
+                                               const uint32_t* nitems, int part = 7,
+                                               int mrows = 0) {
   __shared__ double sh[kSetupThreads / 64];
   // the z line density, read below many times per bin, is kept in LDS
   __shared__ double zl[kMaxZBinsLDS];
   const int nz = P.nz;
-  // part 1: z line density and its derivative; part 2: rho moments and kick factors (two
-  // workgroups may run them side by side: neither reads what the other writes); 3: both
-  if (!(part & 1)) {
-  } else if (zpart) {
+  // part 1: z line density (SpaceChargeCalc2p5D: and the total); 4: its derivative, of zg when
+  // part 1 ran earlier; 2: rho moments and kick factors (parts 2 and 4, and 2 and 1 with 4, may
+  // run side by side: neither reads what the other writes)
+  if (!(part & 5)) {
+  } else if ((part & 1) && zpart) {
     // g = blockDim / nz threads per bin (when nz < blockDim) sum the rows in turn, then
     // their partial sums meet in LDS
     __shared__ double zs[kSetupThreads];
@@ -773,16 +906,17 @@ __device__ __forceinline__ void sc2d_post_body(const SC2DParams& P, SC2DState* s
       const int i = i0 + (int)threadIdx.x / g, r = (int)threadIdx.x % g;
       double acc = 0.0;
       if (i < nz && (int)threadIdx.x < g * ((int)blockDim.x / g)) {
-        // eight rows' loads in flight per round, added in the same order as one by one
-        int b = r;
-        for (; b + 7 * g < zrows; b += 8 * g) {
+        // eight rows' loads in flight per round (past the last row: a row repeated and not
+        // added), added in the same order as one by one
+        for (int b = r; b < zrows; b += 8 * g) {
           double v[8];
 #pragma unroll
-          for (int u = 0; u < 8; u++) v[u] = zpart[(size_t)(b + u * g) * nz + i];
+          for (int u = 0; u < 8; u++)
+            v[u] = zpart[(size_t)(b + u * g < zrows ? b + u * g : b) * nz + i];
 #pragma unroll
-          for (int u = 0; u < 8; u++) acc += v[u];
+          for (int u = 0; u < 8; u++)
+            if (b + u * g < zrows) acc += v[u];
         }
-        for (; b < zrows; b += g) acc += zpart[(size_t)b * nz + i];
       }
       zs[threadIdx.x] = acc;
       __syncthreads();
@@ -799,13 +933,13 @@ __device__ __forceinline__ void sc2d_post_body(const SC2DParams& P, SC2DState* s
     __syncthreads();
   }
   if (st->skip) {
-    if (part & 1)
+    if (part & 4)
       for (int i = threadIdx.x; i < nz; i += blockDim.x) zd[i] = 0.0;
     return;
   }
   const double z_step = st->dz;
   const double zMin = st->zMin;
-  if (P.plain) {  // (part 3 only: the total comes from the line density)
+  if (P.plain) {  // (with part 1: the total comes from the line density)
     // SpaceChargeCalc2p5D.cc:229-233, 100: the total macrosize is the sum of the z line
     // density; no derivative and no rho moments are used
     double t = 0.0;
@@ -819,7 +953,7 @@ __device__ __forceinline__ void sc2d_post_body(const SC2DParams& P, SC2DState* s
     return;
   }
   // calculateLongDerivative (:257-310)
-  if (!(part & 1)) {
+  if (!(part & 4)) {
   } else if (nz == 1) {
     if (threadIdx.x == 0) zd[0] = 0.;
   } else if (nz == 2) {
@@ -878,7 +1012,7 @@ __device__ __forceinline__ void sc2d_post_body(const SC2DParams& P, SC2DState* s
   const double gx0 = st->xMin, gdx = st->dx;
   double s0 = 0., s1 = 0., s2 = 0., s3 = 0., s4 = 0.;
   if (mpart) {
-    const int ni = (int)*nitems;
+    const int ni = nitems ? (int)*nitems : mrows;
     for (int j = threadIdx.x; j < ni; j += blockDim.x) {
       const double* m = mpart + (size_t)j * 5;
       s0 += m[0];
@@ -918,7 +1052,7 @@ __device__ __forceinline__ void sc2d_post_body(const SC2DParams& P, SC2DState* s
     st->factor = P.factor0 / (z_step * total);                 // :133
     st->lsf_in = 1.0 + 2 * log(P.pipe_radius / a_bunch);       // :138
     st->a2 = a_bunch * a_bunch;                                // :140
-    st->scale_coeff = log(P.dx_solver / st->dx);               // PoissonSolverFFT2D.cc:216
+    if (!mrows) st->scale_coeff = log(P.dx_solver / st->dx);   // PoissonSolverFFT2D.cc:216
   }
 }
 
@@ -943,22 +1077,20 @@ __device__ __forceinline__ void rows_r2c_body(const double* __restrict__ in, int
                                               const SC2DState* st, int blk) {
   if (st && st->skip) return;
   extern __shared__ double sm[];
-  double* re = sm;
-  constexpr int LINE = fft_line(N);  // evaluated at compile time
-  double* im = sm + LINE;
+  LineFft<N, kFFTThreads> F(sm, tw, nmax);
   const int r0 = 2 * blk, r1 = r0 + 1;
-  for (int j = threadIdx.x; j < N; j += kFFTThreads) {
-    re[j] = (j < ncols_in) ? in[(int64_t)r0 * ld_in + j] : 0.0;
-    im[j] = (j < ncols_in && r1 < nrows_in) ? in[(int64_t)r1 * ld_in + j] : 0.0;
-  }
+  for (int j = threadIdx.x; j < N; j += kFFTThreads)
+    F.a[j] = make_double2((j < ncols_in) ? in[(int64_t)r0 * ld_in + j] : 0.0,
+                          (j < ncols_in && r1 < nrows_in) ? in[(int64_t)r1 * ld_in + j] : 0.0);
+  F.commit();
   __syncthreads();
-  lds_fft<N, 1, kFFTThreads, -1>(re, im, 1, N, tw, nmax);
+  F.run(1.0);
   constexpr int H = N / 2 + 1;
   for (int k = threadIdx.x; k < H; k += kFFTThreads) {
-    const int nk = (N - k) & (N - 1);
-    const double zr = re[k], zi = im[k], nr = re[nk], ni = im[nk];
-    out[(int64_t)r0 * H + k] = make_double2((zr + nr) * 0.5, (zi - ni) * 0.5);
-    if (r1 < nrows_in) out[(int64_t)r1 * H + k] = make_double2((zi + ni) * 0.5, -(zr - nr) * 0.5);
+    const double2 z = F.a[k], n = F.a[(N - k) & (N - 1)];
+    out[(int64_t)r0 * H + k] = make_double2((z.x + n.x) * 0.5, (z.y - n.y) * 0.5);
+    if (r1 < nrows_in)
+      out[(int64_t)r1 * H + k] = make_double2((z.y + n.y) * 0.5, -(z.x - n.x) * 0.5);
   }
 }
 
@@ -989,7 +1121,64 @@ __global__ __launch_bounds__(kFFTThreads) void fft_rows_r2c_post(
   }
   // two more workgroups: the line density part and the moments part of the post pass
   sc2d_post_body(P, st, rho, zg, zd, tg.zpart, zrows, moments ? tg.mpart : nullptr, tg.nitems,
-                 (int)blockIdx.x == rb ? 1 : 2);
+                 (int)blockIdx.x == rb ? 5 : 2);
+}
+
+// The row pass after sc2d_gdeposit: workgroup r < nx adds the slab copies of grid row r
+// (kSumGroups groups of threads take every kSumGroups-th copy, their sums meet in LDS in group
+// order), writes the row of rho and its share of the rho moments (mpart row) and transforms
+// it; one more workgroup adds the parts' line densities.  One row per workgroup
+// and many threads, where the row pass of a finished rho takes two rows in one complex
+// transform: the loads of the copies set the time, not the transform.
+constexpr int kSumThreads = 1024;
+constexpr int kSumGroups = 8;
+template <int N>
+__global__ __launch_bounds__(kSumThreads) void fft_rows_sum_post(
+    SlabDep D, double* __restrict__ rho, double2* __restrict__ out,
+    const double2* __restrict__ tw, int nmax, SC2DParams P, SC2DState* st,
+    double* __restrict__ zg, double* __restrict__ zd, double* __restrict__ mpart) {
+  const int nx = P.nx, ny = P.ny, r = blockIdx.x;
+  if (r == nx) {
+    sc2d_post_body(P, st, rho, zg, zd, D.zpart, D.parts, nullptr, nullptr, 1);
+    return;
+  }
+  if (st->skip) return;
+  extern __shared__ double sm[];
+  __shared__ double red[kSumThreads / 64][5];
+  constexpr int H = N / 2 + 1;
+  double* acc = sm + line_lds_bytes(N) / sizeof(double);
+  LineFft<N, kSumThreads> F(sm, tw, nmax);
+  constexpr int NG = kSumThreads / kSumGroups;
+  const int grp = (int)threadIdx.x / NG, l = (int)threadIdx.x % NG;
+  for (int j = l; j < ny; j += NG) acc[grp * ny + j] = slab_sum(D, ny, r, j, grp, kSumGroups);
+  F.commit();
+  __syncthreads();
+  double mom[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+  const double xMin = st->xMin, dx = st->dx;
+  for (int j = threadIdx.x; j < N; j += kSumThreads) {
+    double t = 0.0;
+    if (j < ny) {
+      for (int q = 0; q < kSumGroups; q++) t += acc[q * ny + j];
+      rho[(int64_t)r * ny + j] = t;
+      moment_add(mom, t, r, j, xMin, dx);
+    }
+    F.a[j] = make_double2(t, 0.0);
+  }
+  const int nw = (ny + 63) / 64;  // waves that hold nodes
+  if (mpart && (int)threadIdx.x < 64 * nw) {
+    for (int k = 0; k < 5; k++)
+      for (int o = 32; o > 0; o >>= 1) mom[k] += __shfl_xor(mom[k], o, 64);
+    if ((threadIdx.x & 63) == 0)
+      for (int k = 0; k < 5; k++) red[threadIdx.x >> 6][k] = mom[k];
+  }
+  __syncthreads();
+  if (mpart && threadIdx.x < 5) {
+    double t = 0.0;
+    for (int w = 0; w < nw; w++) t += red[w][threadIdx.x];
+    mpart[(size_t)r * 5 + threadIdx.x] = t;
+  }
+  F.run(1.0);
+  for (int k = threadIdx.x; k < H; k += kSumThreads) out[(int64_t)r * H + k] = F.a[k];
 }
 
 // (b) column transforms along x (N = M0).  GREEN: full forward transform of all N rows,
@@ -1002,9 +1191,7 @@ __device__ __forceinline__ void cols_body(double2* __restrict__ spec, int nrows_
                                           const SC2DState* st, double npad, int k) {
   if (st && st->skip) return;
   extern __shared__ double sm[];
-  double* re = sm;
-  constexpr int LINE = fft_line(N);  // evaluated at compile time
-  double* im = sm + LINE;
+  LineFft<N, kFFTThreads> F(sm, tw, nmax);
   // The column and (for a solve) its Green values are requested together before the
   // transform; a masked lane loads element 0 and drops it.
   constexpr int CI = (N + kFFTThreads - 1) / kFFTThreads;
@@ -1018,16 +1205,13 @@ __device__ __forceinline__ void cols_body(double2* __restrict__ spec, int nrows_
 #pragma unroll
   for (int u = 0; u < CI; u++) {
     const int i = (int)threadIdx.x + u * kFFTThreads;
-    if (i < N) {
-      re[i] = i < nrows_in ? cv[u].x : 0.0;
-      im[i] = i < nrows_in ? cv[u].y : 0.0;
-    }
+    if (i < N) F.a[i] = i < nrows_in ? cv[u] : make_double2(0.0, 0.0);
   }
+  F.commit();
   __syncthreads();
-  lds_fft<N, 1, kFFTThreads, -1>(re, im, 1, N, tw, nmax);
+  F.run(1.0);
   if constexpr (GREEN) {
-    for (int i = threadIdx.x; i < N; i += kFFTThreads)
-      ghat_t[(int64_t)k * N + i] = make_double2(re[i], im[i]);
+    for (int i = threadIdx.x; i < N; i += kFFTThreads) ghat_t[(int64_t)k * N + i] = F.a[i];
     return;
   } else {
     // PoissonSolverFFT2D.cc:215-236: Green spectrum rescaled to the rho grid step
@@ -1036,18 +1220,40 @@ __device__ __forceinline__ void cols_body(double2* __restrict__ spec, int nrows_
     for (int u = 0; u < CI; u++) {
       const int i = (int)threadIdx.x + u * kFFTThreads;
       if (i >= N) continue;
-      const double2 g = gv[u];
+      const double2 g = gv[u], z = F.a[i];
       const double gr_re = ((i == 0 && k == 0) ? (g.x + s * npad) : g.x) - s;
       const double gr_im = g.y;
-      const double a = re[i], b = im[i];
-      re[i] = a * gr_re - b * gr_im;
-      im[i] = a * gr_im + b * gr_re;
+      F.a[i] = make_double2(z.x * gr_re - z.y * gr_im, z.x * gr_im + z.y * gr_re);
     }
     __syncthreads();
-    lds_fft<N, 1, kFFTThreads, +1>(re, im, 1, N, tw, nmax);
+    F.run(-1.0);
     for (int i = threadIdx.x; i < nrows_in; i += kFFTThreads)
-      spec[(int64_t)i * H + k] = make_double2(re[i], im[i]);
+      spec[(int64_t)i * H + k] = F.a[i];
   }
+}
+
+// The column pass of a step after fft_rows_sum_post.  gate, gspec (SpaceChargeCalc2p5D): a
+// column whose Green function was rebuilt in this step transforms its column of gspec into
+// ghat_t first.  Two workgroups more than columns (SpaceChargeCalc2p5Drb): the rho moments and
+// kick factors of the post pass, from the row pass's mpart rows, and the derivative of the line
+// density (in the row pass it made that launch's longest workgroup).
+template <int N>
+__global__ __launch_bounds__(kFFTThreads) void fft_cols_post(
+    double2* __restrict__ spec, int nrows_in, int H, double2* __restrict__ ghat_t,
+    const double2* __restrict__ tw, int nmax, SC2DState* st, double npad,
+    const SC2DState* gate, double2* __restrict__ gspec, SC2DParams P,
+    const double* __restrict__ mpart, int mrows, double* __restrict__ zg,
+    double* __restrict__ zd) {
+  const int k = blockIdx.x;
+  if (k >= H) {
+    sc2d_post_body(P, st, nullptr, zg, zd, nullptr, 0, mpart, nullptr, k == H ? 2 : 4, mrows);
+    return;
+  }
+  if (gate && !gate->skip) {
+    cols_body<true, N>(gspec, N, H, ghat_t, tw, nmax, nullptr, 0.0, k);
+    __syncthreads();  // this workgroup's column of ghat_t, read back below
+  }
+  cols_body<false, N>(spec, nrows_in, H, ghat_t, tw, nmax, st, npad, k);
 }
 
 template <bool GREEN, int N>
@@ -1066,9 +1272,7 @@ __device__ __forceinline__ void rows_c2r_body(const double2* __restrict__ spec, 
                                               int nmax, const SC2DState* st, int blk) {
   if (st && st->skip) return;
   extern __shared__ double sm[];
-  double* re = sm;
-  constexpr int LINE = fft_line(N);  // evaluated at compile time
-  double* im = sm + LINE;
+  LineFft<N, kFFTThreads> F(sm, tw, nmax);
   constexpr int H = N / 2 + 1;
   const int r0 = 2 * blk, r1 = r0 + 1;
   const bool has1 = r1 < nrows;
@@ -1080,18 +1284,16 @@ __device__ __forceinline__ void rows_c2r_body(const double2* __restrict__ spec, 
       b.y = 0.0;
     }
     // Z = X0 + i X1 with X(N-k) = conj(X(k))
-    re[k] = a.x - b.y;
-    im[k] = a.y + b.x;
-    if (k > 0 && k < N / 2) {
-      re[N - k] = a.x + b.y;
-      im[N - k] = b.x - a.y;
-    }
+    F.a[k] = make_double2(a.x - b.y, a.y + b.x);
+    if (k > 0 && k < N / 2) F.a[N - k] = make_double2(a.x + b.y, b.x - a.y);
   }
+  F.commit();
   __syncthreads();
-  lds_fft<N, 1, kFFTThreads, +1>(re, im, 1, N, tw, nmax);
+  F.run(-1.0);
   for (int j = threadIdx.x; j < ncols_out; j += kFFTThreads) {
-    out[(int64_t)r0 * ld_out + j] = denom * re[j];
-    if (has1) out[(int64_t)r1 * ld_out + j] = denom * im[j];
+    const double2 z = F.a[j];
+    out[(int64_t)r0 * ld_out + j] = denom * z.x;
+    if (has1) out[(int64_t)r1 * ld_out + j] = denom * z.y;
   }
 }
 
@@ -1251,17 +1453,13 @@ __global__ __launch_bounds__(kFFTThreads) void rows_c2r_batch(const BatchBunch* 
   }
 }
 
-// Green function of PoissonSolverFFT2D::_defineGreenF (:115-172) on the padded grid.
+// The Green function on the padded grid.
 __device__ __forceinline__ void green2d_fill_body(double* __restrict__ G, int M0, int M1,
                                                   double dx, double dy) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= (int64_t)M0 * M1) return;
   const int i = (int)(t / M1), j = (int)(t - (int64_t)i * M1);
-  const int ii = (i <= M0 / 2) ? i : M0 - i;
-  const int jj = (j <= M1 / 2) ? j : M1 - j;
-  const double rTransX = ii * dx, rTransY = jj * dy;
-  const double rTot2 = rTransX * rTransX + rTransY * rTransY;
-  G[t] = (ii != 0 || jj != 0) ? -log(rTot2) / 2 : 0.0;
+  G[t] = green2d_value(i, j, M0, M1, dx, dy);
 }
 
 __global__ void green2d_fill(double* __restrict__ G, int M0, int M1, double dx, double dy) {
@@ -1299,7 +1497,11 @@ struct ob_sc2p5drb {
   int plain = 0;
   int par = 0;                      // state entry the next step reads
   ob::SC2DState* gate = nullptr;
-  double* gbuf = nullptr;           // M0 x M1 Green function values
+  double* gbuf = nullptr;           // M0 x M1 Green function values (tile-sorted deposit)
+  double2* gspec = nullptr;         // M0 x H row transforms of a new Green function
+  // grid-copy deposit (slabs 0: the grid is too large, tile sort)
+  ob::SlabDep slab{};
+  int64_t copies_cap = 0;           // doubles of slab.copies
   ob::StatusBox status{nullptr, nullptr};  // set when a step finds a zero-extent bunch
 };
 
@@ -1309,7 +1511,7 @@ struct ob_sc2p5d : ob_sc2p5drb {};
 namespace ob {
 namespace {
 template <int N>
-size_t fft_lds() { return sizeof(double) * 2 * fft_line(N); }
+size_t fft_lds() { return line_lds_bytes(N); }
 
 // Dynamic LDS above 64 KiB has to be allowed per kernel; done once per instantiation.
 template <typename K>
@@ -1363,6 +1565,25 @@ struct PostArgs {
   int zrows, moments;
 };
 
+void launch_rows_c2r(ob_sc2p5drb* c, SC2DState* st) {
+  const double denom = 1.0 / (c->M0 * c->M1);
+  dispatch_pow2(c->M1, [&](auto NC) {
+    constexpr int N = decltype(NC)::value;
+    if constexpr (N >= 8) {
+      static bool ready = false;
+      if (!ready) {
+        allow_lds(fft_rows_c2r<N>, fft_lds<N>());
+        ready = true;
+      }
+      ob::ProfScope ps_("fft_rows_c2r");
+      hipLaunchKernelGGL(fft_rows_c2r<N>, dim3((c->nx + 1) / 2), dim3(kFFTThreads), fft_lds<N>(),
+                         stream(), c->spec, c->nx, c->phi, c->ny, c->ny, denom, c->tw, c->nmax,
+                         st);
+    }
+  });
+  OB_HIP(hipGetLastError());
+}
+
 void launch_fft_pipeline(ob_sc2p5drb* c, SC2DState* st, const PostArgs* post = nullptr) {
   if (post) {
     dispatch_pow2(c->M1, [&](auto NC) {
@@ -1385,22 +1606,48 @@ void launch_fft_pipeline(ob_sc2p5drb* c, SC2DState* st, const PostArgs* post = n
     launch_rows_r2c(c, c->rho, c->nx, c->ny, c->ny, st);
   }
   launch_cols<false>(c, c->nx, st, (double)c->M0 * (double)c->M1);
-  const double denom = 1.0 / (c->M0 * c->M1);
+  launch_rows_c2r(c, st);
+}
+
+// The solve after sc2d_gdeposit: row pass (adds the copies), column pass with the rest of the
+// post pass (and a rebuilt Green function's columns), inverse row pass.
+void launch_slab_solve(ob_sc2p5drb* c, const SC2DParams& P, const SlabDep& D) {
   dispatch_pow2(c->M1, [&](auto NC) {
+    constexpr int N = decltype(NC)::value;
+    if constexpr (N >= 8 && N <= 2 * kSlabMaxNy) {
+      const size_t lds = line_lds_bytes(N) + sizeof(double) * kSumGroups * c->ny;
+      static bool ready = false;
+      if (!ready) {
+        OB_HIP(hipFuncSetAttribute((const void*)fft_rows_sum_post<N>,
+                                   hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   (int)(line_lds_bytes(N) +
+                                         sizeof(double) * kSumGroups * (N / 2 + 1))));
+        ready = true;
+      }
+      ob::ProfScope ps_("fft_rows_sum_post");
+      hipLaunchKernelGGL(fft_rows_sum_post<N>, dim3(c->nx + 1), dim3(kSumThreads), lds, stream(), D,
+                         c->rho, c->spec, c->tw, c->nmax, P, c->st, c->zg, c->zd,
+                         P.plain ? nullptr : D.mrows);
+    }
+  });
+  OB_HIP(hipGetLastError());
+  dispatch_pow2(c->M0, [&](auto NC) {
     constexpr int N = decltype(NC)::value;
     if constexpr (N >= 8) {
       static bool ready = false;
       if (!ready) {
-        allow_lds(fft_rows_c2r<N>, fft_lds<N>());
+        allow_lds(fft_cols_post<N>, fft_lds<N>());
         ready = true;
       }
-      ob::ProfScope ps_("fft_rows_c2r");
-      hipLaunchKernelGGL(fft_rows_c2r<N>, dim3((c->nx + 1) / 2), dim3(kFFTThreads), fft_lds<N>(),
-                         stream(), c->spec, c->nx, c->phi, c->ny, c->ny, denom, c->tw, c->nmax,
-                         st);
+      ob::ProfScope ps_("fft_cols_post");
+      hipLaunchKernelGGL(fft_cols_post<N>, dim3(c->H + (P.plain ? 0 : 2)), dim3(kFFTThreads),
+                         fft_lds<N>(), stream(), c->spec, c->nx, c->H, c->ghat_t, c->tw, c->nmax,
+                         c->st, (double)c->M0 * (double)c->M1, P.plain ? c->gate : nullptr,
+                         c->gspec, P, D.mrows, c->nx, c->zg, c->zd);
     }
   });
   OB_HIP(hipGetLastError());
+  launch_rows_c2r(c, c->st);
 }
 
 void define_green(ob_sc2p5drb* c) {
@@ -1497,6 +1744,83 @@ Tile2D sc2d_tile_reserve(ob_sc2p5drb* c, int64_t n, bool per_particle_m, int ite
   return g;
 }
 
+namespace {
+// The slab split of a calculator's grid (slabs 0: it does not fit, tile sort).
+SlabDep slab_split(int nx, int ny, int nz, int M0) {
+  SlabDep D{};
+  const int centre = nx - 2;
+  const int64_t max_rows = (kSlabLds / 8 - nz) / ny - 2;
+  if (ny > kSlabMaxNy || max_rows < 1 || centre > kSlabMax * max_rows) return D;
+  D.slabs = (int)((centre + max_rows - 1) / max_rows);
+  if (D.slabs == 3) D.slabs = 4;
+  D.M0 = M0;
+  return D;
+}
+
+// The deposit of a bunch of n particles: parts per slab, and the copies' buffers.
+SlabDep slab_reserve(ob_sc2p5drb* c, int64_t n) {
+  SlabDep D = c->slab;
+  const int centre = c->nx - 2;
+  if (D.slabs == 1 && n <= kSlabSplitMax && centre > 1) D.slabs = 2;
+  D.rows = (centre + D.slabs - 1) / D.slabs;
+  D.R = D.rows + 2;
+  const int64_t want = std::max<int64_t>(
+      1, std::min<int64_t>(std::max<int64_t>((n + kSlabPart - 1) / kSlabPart,
+                                             std::min<int64_t>((n + 1023) / 1024, 16)),
+                           device_cu_count() / D.slabs));
+  D.parts = (int)want;
+  D.per = (n + want - 1) / want;
+  // one buffer: copies, line densities of the parts, moments of the grid rows
+  const int64_t ncopy = (int64_t)D.slabs * D.parts * D.R * c->ny;
+  const int64_t need = ncopy + (int64_t)D.parts * c->nz + 5 * c->nx;
+  if (need > c->copies_cap) {
+    OB_HIP(hipStreamSynchronize(stream()));  // it may be in use by queued work
+    if (c->slab.copies) OB_HIP(hipFree(c->slab.copies));
+    c->slab.copies = nullptr;
+    c->copies_cap = 0;
+    OB_HIP(hipMalloc((void**)&c->slab.copies, sizeof(double) * need));
+    c->copies_cap = need;
+  }
+  if (c->plain && !c->gspec)
+    OB_HIP(hipMalloc((void**)&c->gspec, sizeof(double2) * (size_t)c->M0 * c->H));
+  D.copies = c->slab.copies;
+  D.zpart = D.copies + ncopy;
+  D.mrows = D.zpart + (int64_t)D.parts * c->nz;
+  D.gspec = c->gspec;
+  return D;
+}
+
+void launch_gdeposit(ob_sc2p5drb* c, const SC2DParams& P, const DeviceBunchView& v, SlabDep D) {
+  const size_t dep_lds = sizeof(double) * ((size_t)D.R * c->ny + c->nz);
+  auto go = [&](auto kernel, size_t lds, size_t most, bool& ready) {
+    if (!ready) {
+      OB_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                 (int)most));
+      ready = true;
+    }
+    ob::ProfScope ps_("sc2d_gdeposit");
+    hipLaunchKernelGGL(kernel, dim3(D.slabs * D.parts + D.green_blocks), dim3(kSlabThreads), lds,
+                       stream(), P, v, c->partials, c->st, c->gate, D, c->status.dev, c->tw,
+                       c->nmax);
+  };
+  if (!c->plain) {
+    static bool ready = false;
+    go(sc2d_gdeposit<0>, dep_lds, kSlabLds, ready);
+  } else {
+    dispatch_pow2(c->M1, [&](auto NC) {
+      constexpr int N = decltype(NC)::value;
+      if constexpr (N >= 8 && N <= 2 * kSlabMaxNy) {
+        static bool ready = false;
+        constexpr size_t gl = sizeof(double) * 2 * green_pairs(N) * fft_line_stride(N);
+        D.green_blocks = (c->M0 / 2 + green_pairs(N) - 1) / green_pairs(N);
+        go(sc2d_gdeposit<N>, std::max(dep_lds, gl), std::max<size_t>(kSlabLds, gl), ready);
+      }
+    });
+  }
+  OB_HIP(hipGetLastError());
+}
+}  // namespace
+
 bool sc2d_tile_same(ob_sc2p5drb* c, const Tile2D& t, int64_t n, bool per_particle_m) {
   const Tile2D& g = c->tg;
   return g.sxy == t.sxy && g.items == t.items && g.item == t.item && n <= c->tile_ncap &&
@@ -1550,7 +1874,7 @@ void launch_sc2d_batch(const BatchBunch* bb, const BatchItem* items, const Batch
     hipLaunchKernelGGL(sc2d_post_batch, dim3(sh.nb), dim3(kSetupThreads), 0, s, bb, length,
                        pipe_radius);
   }
-  const size_t fl = sizeof(double) * 2 * fft_line(sh.max_M);  // fft_line grows with N
+  const size_t fl = line_lds_bytes(sh.max_M);  // (grows with N; at most 1024 points here)
   {
     ProfScope ps("fft_rows_r2c_batch");
     hipLaunchKernelGGL(rows_r2c_batch, dim3(sh.row_blocks), dim3(kFFTThreads), fl, s, bb, sh.nb);
@@ -1636,8 +1960,8 @@ Calc* sc2d_create(int nx, int ny, int nz, double xy_ratio, bool plain, const std
     std::memset(&g, 0, sizeof(g));
     g.skip = 1;
     OB_HIP(hipMemcpy(c->gate, &g, sizeof(g), hipMemcpyHostToDevice));
-    OB_HIP(hipMalloc((void**)&c->gbuf, sizeof(double) * c->M0 * c->M1));
   }
+  c->slab = slab_split(nx, ny, nz, c->M0);
   c->tw = make_twiddles(c->nmax);
   define_green(c);
   c->status = status_box_create(
@@ -1663,10 +1987,69 @@ void sc2d_destroy(ob_sc2p5drb* c) {
                   (void*)c->ghat_t, (void*)c->tw, (void*)c->partials, (void*)c->st,
                   (void*)c->gate, (void*)c->gbuf, (void*)c->tg.counts, (void*)c->tg.items,
                   (void*)c->tg.sxy, (void*)c->tg.sm, (void*)c->tg.zpart,
-                  (void*)c->tg.mpart, (void*)c->tg.icounts})
+                  (void*)c->tg.mpart, (void*)c->tg.icounts, (void*)c->gspec,
+                  (void*)c->slab.copies})
     if (p) (void)hipFree(p);
   delete c;
   OB_REQUIRE(err.empty(), err);
+}
+
+// Deposit and solve of a step on a grid too large for the slab copies: bin (grid, tile counts,
+// z line density), scatter (scan, counting sort), tile deposit, post pass and FFT passes.
+void sc2d_tile_step(ob_sc2p5drb* c, ob_bunch* b, const DeviceBunchView& v, const SC2DParams& P,
+                    int64_t n) {
+  hipStream_t s = stream();
+  const int hb = (int)std::max<int64_t>(
+      1, std::min<int64_t>({(n + 2047) / 2048, (int64_t)4 * device_cu_count(),
+                            (int64_t)std::max(1, (1 << 18) / c->nz)}));
+  const Tile2D tg = sc2d_tile_reserve(c, n, v.msize != nullptr, c->tile_item, hb);
+  {
+    ProfScope ps_("sc2d_bin");
+    hipLaunchKernelGGL(sc2d_bin, dim3(hb), dim3(kDepositThreads),
+                       sizeof(double) * c->nz + sizeof(uint32_t) * tg.ntiles, s, P, v,
+                       c->partials, c->st, c->gate, tg, c->rho, c->status.dev);
+  }
+  if (c->plain) {
+    // PoissonSolverFFT2D::setGridXY (PoissonSolverFFT2D.cc:103-111) when the grid pass
+    // asked for it; each pass returns at once otherwise.  spec is free until the solve.
+    const int64_t tot = (int64_t)c->M0 * c->M1;
+    if (!c->gbuf) OB_HIP(hipMalloc((void**)&c->gbuf, sizeof(double) * tot));
+    {
+      ProfScope ps_("green2d_fill_state");
+      hipLaunchKernelGGL(green2d_fill_state, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0,
+                         s, c->gbuf, c->M0, c->M1, c->st, c->gate);
+    }
+    launch_rows_r2c(c, c->gbuf, c->M0, c->M1, c->M1, c->gate);
+    launch_cols<true>(c, c->M0, c->gate, 0.0);
+    c->par ^= 1;
+  }
+  // rb: the rho moments come from the deposit unless the denoiser changes rho after it
+  const int moments = (c->denoiser || c->plain) ? 0 : 1;
+  {
+    ProfScope ps_("sc2d_scatter");
+    const int64_t per = std::max<int64_t>(2048, (n + 1023) / 1024);
+    hipLaunchKernelGGL(sc2d_scatter, dim3((unsigned)((n + per - 1) / per)),
+                       dim3(kDepositThreads), 2 * sizeof(uint32_t) * tg.ntiles, s, P, v,
+                       c->st, tg, per);
+  }
+  {
+    ProfScope ps_("sc2d_tdeposit");
+    hipLaunchKernelGGL(sc2d_tdeposit, dim3((unsigned)(n / tg.item + tg.ntiles + 1)),
+                       dim3(kDepositThreads), sizeof(double) * (tg.T + 2) * (tg.T + 2), s,
+                       P, c->st, tg, v.msize != nullptr ? 1 : 0, c->rho, moments);
+  }
+  if (c->denoiser) dn_denoise_rho(c->denoiser, c->rho, c->nx, c->ny, &c->st->skip);
+  if (c->plain) {  // its solve reads the post pass's results: it runs first
+    {
+      ProfScope ps_("sc2d_post");
+      hipLaunchKernelGGL(sc2d_post, dim3(1), dim3(kSetupThreads), 0, s, P, c->st, c->rho,
+                         c->zg, c->zd, tg, hb, moments);
+    }
+    launch_fft_pipeline(c, c->st);
+  } else {
+    const PostArgs pa{P, tg, hb, moments};
+    launch_fft_pipeline(c, c->st, &pa);
+  }
 }
 
 // One trackBunch: SpaceChargeCalc2p5Drb.cc:110-168, or SpaceChargeCalc2p5D.cc:77-120
@@ -1692,84 +2075,26 @@ void sc2d_track(ob_sc2p5drb* c, ob_bunch* b, double length, double pipe_radius,
   P.par = c->par;
   for (int k = 0; k < 6; k++) P.bnd[k] = 0.0;
   P.bnd_type = bnd ? boundary_describe(bnd, P.bnd) : 0;
-  // bin (grid + tile counts + z line density), scatter (scan + counting sort), deposit
-  // the whole grid fits in LDS: private-grid deposit in particle order, no tile sort
-  const bool private_grid = (int64_t)c->nx * c->ny <= kPrivNodes && n <= kPrivMaxParticles;
-  // bin workgroups of 2048 particles; 1024 with the private-grid deposit, whose bin pass
-  // counts no tiles (100k on 128x128: 0.8% faster per step than 2048, 512 4% slower)
-  const int64_t bin_per = private_grid ? 1024 : 2048;
-  const int hb = (int)std::max<int64_t>(
-      1, std::min<int64_t>({(n + bin_per - 1) / bin_per, (int64_t)4 * device_cu_count(),
-                            (int64_t)std::max(1, (1 << 18) / c->nz)}));
-  const Tile2D tg = sc2d_tile_reserve(c, n, v.msize != nullptr, c->tile_item, hb);
-  {
-    ProfScope ps_("sc2d_bin");
-    if (private_grid)
-      hipLaunchKernelGGL(sc2d_bin<false>, dim3(hb), dim3(kDepositThreads),
-                         sizeof(double) * c->nz + sizeof(uint32_t) * tg.ntiles, s, P, v,
-                         c->partials, c->st, c->gate, tg, c->rho, c->status.dev);
-    else
-      hipLaunchKernelGGL(sc2d_bin<true>, dim3(hb), dim3(kDepositThreads),
-                         sizeof(double) * c->nz + sizeof(uint32_t) * tg.ntiles, s, P, v,
-                         c->partials, c->st, c->gate, tg, c->rho, c->status.dev);
-  }
-  if (c->plain) {
-    // PoissonSolverFFT2D::setGridXY (PoissonSolverFFT2D.cc:103-111) when the grid pass
-    // asked for it; each pass returns at once otherwise.  spec is free until the solve.
-    const int64_t tot = (int64_t)c->M0 * c->M1;
-    {
-      ProfScope ps_("green2d_fill_state");
-      hipLaunchKernelGGL(green2d_fill_state, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0,
-                         s, c->gbuf, c->M0, c->M1, c->st, c->gate);
+  if (c->slab.slabs > 0) {  // grid, line density and deposit in one pass, no tile sort
+    const SlabDep D = slab_reserve(c, n);
+    launch_gdeposit(c, P, v, D);
+    if (c->plain) c->par ^= 1;
+    if (c->denoiser) {  // it changes rho before the moments and the solve
+      {
+        ProfScope ps_("sc2d_slab_rho");
+        hipLaunchKernelGGL(sc2d_slab_rho, dim3((c->nx * c->ny + 255) / 256), dim3(256), 0, s, D,
+                           c->nx, c->ny, c->st, c->rho);
+      }
+      dn_denoise_rho(c->denoiser, c->rho, c->nx, c->ny, &c->st->skip);
+      Tile2D tg{};
+      tg.zpart = D.zpart;
+      const PostArgs pa{P, tg, D.parts, 0};
+      launch_fft_pipeline(c, c->st, &pa);
+    } else {
+      launch_slab_solve(c, P, D);
     }
-    launch_rows_r2c(c, c->gbuf, c->M0, c->M1, c->M1, c->gate);
-    launch_cols<true>(c, c->M0, c->gate, 0.0);
-    c->par ^= 1;
-  }
-  // rb: the rho moments come from the deposit unless the denoiser changes rho after it
-  const int moments = (c->denoiser || c->plain) ? 0 : 1;
-  if (private_grid) {
-    static bool attr_done = false;
-    if (!attr_done) {
-      OB_HIP(hipFuncSetAttribute((const void*)sc2d_pdeposit,
-                                 hipFuncAttributeMaxDynamicSharedMemorySize,
-                                 (int)(sizeof(double) * kPrivNodes)));
-      attr_done = true;
-    }
-    const int64_t blocks = std::max<int64_t>(
-        1, std::min<int64_t>({(n + kPrivPerBlock - 1) / kPrivPerBlock,
-                              (int64_t)device_cu_count(), (int64_t)tg.max_items}));
-    const int64_t per = (n + blocks - 1) / blocks;
-    ProfScope ps_("sc2d_pdeposit");
-    hipLaunchKernelGGL(sc2d_pdeposit, dim3((unsigned)blocks), dim3(kPrivThreads),
-                       sizeof(double) * c->nx * c->ny, s, P, v, c->st, tg, per, c->rho,
-                       moments);
   } else {
-    {
-      ProfScope ps_("sc2d_scatter");
-      const int64_t per = std::max<int64_t>(2048, (n + 1023) / 1024);
-      hipLaunchKernelGGL(sc2d_scatter, dim3((unsigned)((n + per - 1) / per)),
-                         dim3(kDepositThreads), 2 * sizeof(uint32_t) * tg.ntiles, s, P, v,
-                         c->st, tg, per);
-    }
-    {
-      ProfScope ps_("sc2d_tdeposit");
-      hipLaunchKernelGGL(sc2d_tdeposit, dim3((unsigned)(n / tg.item + tg.ntiles + 1)),
-                         dim3(kDepositThreads), sizeof(double) * (tg.T + 2) * (tg.T + 2), s,
-                         P, c->st, tg, v.msize != nullptr ? 1 : 0, c->rho, moments);
-    }
-  }
-  if (c->denoiser) dn_denoise_rho(c->denoiser, c->rho, c->nx, c->ny, &c->st->skip);
-  if (c->plain || bnd) {  // their solve reads the post pass's results: it runs first
-    {
-      ProfScope ps_("sc2d_post");
-      hipLaunchKernelGGL(sc2d_post, dim3(1), dim3(kSetupThreads), 0, s, P, c->st, c->rho,
-                         c->zg, c->zd, tg, hb, moments);
-    }
-    launch_fft_pipeline(c, c->st);
-  } else {
-    const PostArgs pa{P, tg, hb, moments};
-    launch_fft_pipeline(c, c->st, &pa);
+    sc2d_tile_step(c, b, v, P, n);
   }
   if (bnd) boundary_add_potential(bnd, c->phi, c->nx, c->ny, c->st, s);  // :90-94
   OB_HIP(hipGetLastError());
