@@ -6,10 +6,9 @@
 // coefficients are the least-squares fit of phi on the boundary points, so that phi
 // minus that field is (nearly) constant on the boundary.  The projector
 // LSQ = (F^T F)^-1 F^T is set up once on the host (the reference's initializeBPs, a
-// (2M+1)^2 Gauss-Jordan inverse); every step then runs two kernels on the device:
-//   bnd_coef   one workgroup: phi interpolated at the points (Grid2D::getValue), then the
-//              2M+1 coefficients, each a dot product in point order;
-//   bnd_apply  one thread per node: the harmonic field from the coefficients, subtracted.
+// (2M+1)^2 Gauss-Jordan inverse); every step then runs one kernel on the device: every
+// workgroup interpolates phi at the points (Grid2D::getValue), forms the 2M+1 coefficients
+// (dot products over the points) in LDS and subtracts the harmonic field at its nodes.
 #include <cmath>
 #include <string>
 #include <utility>
@@ -26,7 +25,7 @@ struct ob_boundary2d {
   double xDim = 0., yDim = 0., p0 = 0., p1 = 0.;
   double xMin = DBL_MAX, xMax = -DBL_MAX, yMin = DBL_MAX, yMax = -DBL_MAX, rnorm = DBL_MAX;
   std::vector<double> bx, by, lsq;  // lsq: [(2 nm + 1)][np]
-  double *d_bx = nullptr, *d_by = nullptr, *d_lsq = nullptr, *d_work = nullptr;
+  double *d_bx = nullptr, *d_by = nullptr, *d_lsq = nullptr;
   double* d_work3 = nullptr;  // per-slice work of a stack of grids
   int64_t work3_cap = 0;
   ob::SC2DState* d_geo = nullptr;  // grid geometry of a user grid (add_potential)
@@ -57,41 +56,64 @@ __device__ __forceinline__ double grid2d_value(const double* __restrict__ a, int
          Wxp * Wyp * r2[1];
 }
 
-// work = [np] phi at the points, then [2 nm + 1] coefficients (BaseBoundary2D.cc:430-440).
-__global__ __launch_bounds__(kCoefThreads) void bnd_coef(const double* __restrict__ phi, int nx,
-                                                        int ny, const SC2DState* st,
-                                                        const double* __restrict__ bx,
-                                                        const double* __restrict__ by, int np,
-                                                        const double* __restrict__ lsq, int nf,
-                                                        double* __restrict__ work) {
-  if (st->skip) return;
-  const double xMin = st->xMin, dx = st->dx, yMin = st->yMin, dy = st->dy;
-  for (int j = threadIdx.x; j < np; j += blockDim.x)
-    work[j] = grid2d_value(phi, nx, ny, xMin, dx, yMin, dy, bx[j], by[j]);
-  __syncthreads();
-  for (int i = threadIdx.x; i < nf; i += blockDim.x) {
-    double c = 0.0;
-    const double* row = lsq + (size_t)i * np;
-    for (int j = 0; j < np; j++) c += row[j] * work[j];
-    work[np + i] = c;
+// coef[nf] = lsq[nf][np] . bphi[np] (BaseBoundary2D.cc:430-440) by all waves of a workgroup:
+// a wave takes kCoefRows rows at a time, its lanes the points, so the rows are read in whole
+// lines and their sums overlap (one thread per row read np strided values in turn, 14 us for
+// 33 x 128).  The sum runs lane by lane and then across the lanes.  coef may be LDS or global.
+constexpr int kCoefRows = 4;
+__device__ __forceinline__ void bnd_coefs(const double* __restrict__ lsq, int nf, int np,
+                                          const double* bphi, double* coef) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  for (int i0 = w * kCoefRows; i0 < nf; i0 += nw * kCoefRows) {
+    double c[kCoefRows];
+#pragma unroll
+    for (int u = 0; u < kCoefRows; u++) c[u] = 0.0;
+    for (int j = lane; j < np; j += 64) {
+      const double p = bphi[j];
+#pragma unroll
+      for (int u = 0; u < kCoefRows; u++)
+        c[u] += lsq[(size_t)(i0 + u < nf ? i0 + u : i0) * np + j] * p;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+      for (int u = 0; u < kCoefRows; u++) c[u] += __shfl_xor(c[u], o, 64);
+    if (lane == 0)
+#pragma unroll
+      for (int u = 0; u < kCoefRows; u++)
+        if (i0 + u < nf) coef[i0 + u] = c[u];
   }
 }
 
-// phi -= sum_k c_k f_k at every node (BaseBoundary2D.cc:442-457, functions :316-345).
-__global__ __launch_bounds__(256) void bnd_apply(double* __restrict__ phi, int nx, int ny,
-                                                 const SC2DState* st,
-                                                 const double* __restrict__ coef, int nm,
-                                                 double rnorm) {
+// dst = src - sum_k c_k f_k at every node (BaseBoundary2D.cc:430-457, functions :316-345).
+// Every workgroup computes the coefficients for itself: that is a few thousand products,
+// where a launch of its own for them made 14 us + a 4 us launch that waited for it; src and
+// dst differ because the points of other workgroups read src.  200k in a 128-point pipe,
+// 128 x 128: 20 us a step in two launches, 8.5 us so.  LDS: np + nf doubles.
+__global__ __launch_bounds__(kCoefThreads) void bnd_subtract(
+    const double* __restrict__ src, double* __restrict__ dst, int nx, int ny,
+    const SC2DState* st, const double* __restrict__ bx, const double* __restrict__ by, int np,
+    const double* __restrict__ lsq, int nm, double rnorm) {
   if (st->skip) return;
+  extern __shared__ double lds[];
+  const int nf = 2 * nm + 1;
+  double *bphi = lds, *coef = lds + np;
+  const double xMin = st->xMin, dx = st->dx, yMin = st->yMin, dy = st->dy;
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  const double own = src[t < nx * ny ? t : 0];
+  for (int j = threadIdx.x; j < np; j += blockDim.x)
+    bphi[j] = grid2d_value(src, nx, ny, xMin, dx, yMin, dy, bx[j], by[j]);
+  __syncthreads();
+  bnd_coefs(lsq, nf, np, bphi, coef);
+  __syncthreads();
   if (t >= nx * ny) return;
   const int i = t / ny, j = t - i * ny;
-  const double x = st->xMin + i * st->dx, y = st->yMin + j * st->dy;
+  const double x = xMin + i * dx, y = yMin + j * dy;
   const double r2 = x * x + y * y;
   double v = 0.;
   if (r2 == 0.) {
     v += coef[0] * 1.0;
-    for (int k = 1; k < 2 * nm + 1; k++) v += coef[k] * 0.0;
+    for (int k = 1; k < nf; k++) v += coef[k] * 0.0;
   } else {
     const double r = sqrt(r2);
     const double sn = y / r, cs = x / r, q = r / rnorm;
@@ -107,7 +129,7 @@ __global__ __launch_bounds__(256) void bnd_apply(double* __restrict__ phi, int n
       csk = c1;
     }
   }
-  phi[t] -= v;
+  dst[t] = own - v;
 }
 
 // A stack of z-fastest slices phi[(ix*ny + iy)*nz + iz]: one workgroup per slice iz.
@@ -135,13 +157,7 @@ __global__ __launch_bounds__(kCoefThreads) void bnd_coef_slices(
               Wxp * Wy0 * a(iX + 1, iY) + Wxp * Wyp * a(iX + 1, iY + 1);
   }
   __syncthreads();
-  double* coef = work + (size_t)nz * np + (size_t)iz * nf;
-  for (int i = threadIdx.x; i < nf; i += blockDim.x) {
-    double c = 0.0;
-    const double* row = lsq + (size_t)i * np;
-    for (int j = 0; j < np; j++) c += row[j] * bphi[j];
-    coef[i] = c;
-  }
+  bnd_coefs(lsq, nf, np, bphi, work + (size_t)nz * np + (size_t)iz * nf);
 }
 
 __global__ __launch_bounds__(256) void bnd_apply_slices(double* __restrict__ phi, int nx, int ny,
@@ -278,12 +294,11 @@ void initialize(ob_boundary2d* b) {
   hipStream_t s = stream();
   OB_HIP(hipStreamSynchronize(s));  // earlier steps may still read the old arrays
   if (b->d_np != b->np) {
-    for (void* p : {(void*)b->d_bx, (void*)b->d_by, (void*)b->d_lsq, (void*)b->d_work})
+    for (void* p : {(void*)b->d_bx, (void*)b->d_by, (void*)b->d_lsq})
       if (p) OB_HIP(hipFree(p));
     OB_HIP(hipMalloc((void**)&b->d_bx, sizeof(double) * b->np));
     OB_HIP(hipMalloc((void**)&b->d_by, sizeof(double) * b->np));
     OB_HIP(hipMalloc((void**)&b->d_lsq, sizeof(double) * nf * b->np));
-    OB_HIP(hipMalloc((void**)&b->d_work, sizeof(double) * (b->np + nf)));
     b->d_np = b->np;
   }
   OB_HIP(hipMemcpy(b->d_bx, b->bx.data(), sizeof(double) * b->np, hipMemcpyHostToDevice));
@@ -302,20 +317,21 @@ void set_point(ob_boundary2d* b, int i, double x, double y) {
 }
 }  // namespace
 
-void boundary_add_potential(ob_boundary2d* b, double* phi, int nx, int ny, const SC2DState* st,
-                            hipStream_t s) {
+void boundary_add_potential(ob_boundary2d* b, const double* src, double* dst, int nx, int ny,
+                            const SC2DState* st, hipStream_t s) {
   OB_REQUIRE(b->initialized,
              "Boundary2D addBoundaryPotential: the boundary was not initialized");
   const int nf = 2 * b->nm + 1;
+  const size_t lds = sizeof(double) * (b->np + nf);
+  OB_REQUIRE(lds <= 160 * 1024, "Boundary2D addBoundaryPotential: too many boundary points");
+  if (lds > 64 * 1024)
+    OB_HIP(hipFuncSetAttribute((const void*)bnd_subtract,
+                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   {
-    ProfScope ps("bnd_coef", s);
-    hipLaunchKernelGGL(bnd_coef, dim3(1), dim3(kCoefThreads), 0, s, phi, nx, ny, st, b->d_bx,
-                       b->d_by, b->np, b->d_lsq, nf, b->d_work);
-  }
-  {
-    ProfScope ps("bnd_apply", s);
-    hipLaunchKernelGGL(bnd_apply, dim3((nx * ny + 255) / 256), dim3(256), 0, s, phi, nx, ny, st,
-                       b->d_work + b->np, b->nm, b->rnorm);
+    ProfScope ps("bnd_subtract", s);
+    hipLaunchKernelGGL(bnd_subtract, dim3((nx * ny + kCoefThreads - 1) / kCoefThreads),
+                       dim3(kCoefThreads), lds, s, src, dst, nx, ny, st, b->d_bx, b->d_by, b->np,
+                       b->d_lsq, b->nm, b->rnorm);
   }
   OB_HIP(hipGetLastError());
 }
@@ -468,8 +484,8 @@ OB_API int ob_boundary2d_create_shaped(int nPoints, int nModes, const char* shap
 OB_API int ob_boundary2d_destroy(ob_boundary2d* b) {
   OB_TRY if (!b) return 0;
   (void)hipStreamSynchronize(ob::stream());  // queued steps may read its arrays
-  for (void* p : {(void*)b->d_bx, (void*)b->d_by, (void*)b->d_lsq, (void*)b->d_work,
-                  (void*)b->d_geo, (void*)b->d_work3})
+  for (void* p : {(void*)b->d_bx, (void*)b->d_by, (void*)b->d_lsq, (void*)b->d_geo,
+                  (void*)b->d_work3})
     if (p) (void)hipFree(p);
   delete b;
   OB_CATCH
@@ -535,12 +551,13 @@ OB_API int ob_boundary2d_add_potential(ob_boundary2d* b, double* phi, int nx, in
   g.dx = (lims[1] - lims[0]) / (nx - 1);  // Grid2D.cc:409-420
   g.dy = (lims[3] - lims[2]) / (ny - 1);
   double* d_phi = nullptr;
-  OB_HIP(hipMalloc((void**)&d_phi, sizeof(double) * nx * ny));
+  const size_t ng = (size_t)nx * ny;
+  OB_HIP(hipMalloc((void**)&d_phi, sizeof(double) * 2 * ng));
   try {
     OB_HIP(hipMemcpyAsync(b->d_geo, &g, sizeof(g), hipMemcpyHostToDevice, s));
     OB_HIP(hipMemcpyAsync(d_phi, phi, sizeof(double) * nx * ny, hipMemcpyHostToDevice, s));
-    ob::boundary_add_potential(b, d_phi, nx, ny, b->d_geo, s);
-    OB_HIP(hipMemcpyAsync(phi, d_phi, sizeof(double) * nx * ny, hipMemcpyDeviceToHost, s));
+    ob::boundary_add_potential(b, d_phi, d_phi + ng, nx, ny, b->d_geo, s);
+    OB_HIP(hipMemcpyAsync(phi, d_phi + ng, sizeof(double) * ng, hipMemcpyDeviceToHost, s));
     OB_HIP(hipStreamSynchronize(s));
   } catch (...) {
     (void)hipFree(d_phi);

@@ -249,10 +249,11 @@ void dn_denoise_rhos(const std::vector<DenoiseJob>& jobs);
 }  // namespace ob
 struct ob_boundary2d;
 namespace ob {
-// Boundary2D::addBoundaryPotential (BaseBoundary2D.cc:349-458) on a device phi grid whose
-// geometry is in st (skipped when st->skip); the boundary must be initialized.
-void boundary_add_potential(ob_boundary2d* b, double* phi, int nx, int ny, const SC2DState* st,
-                            hipStream_t s);
+// Boundary2D::addBoundaryPotential (BaseBoundary2D.cc:349-458) from the device phi grid src,
+// whose geometry is in st, into dst (not src; nothing is written when st->skip); the boundary
+// must be initialized.
+void boundary_add_potential(ob_boundary2d* b, const double* src, double* dst, int nx, int ny,
+                            const SC2DState* st, hipStream_t s);
 // The same for each z slice of a z-fastest [nx][ny][nz] stack (its own coefficients).
 void boundary_add_potential_slices(ob_boundary2d* b, double* phi, int nx, int ny, int nz,
                                    const SC2DState* st, hipStream_t s);

@@ -1501,6 +1501,7 @@ struct ob_sc2p5drb {
   double2* gspec = nullptr;         // M0 x H row transforms of a new Green function
   // grid-copy deposit (slabs 0: the grid is too large, tile sort)
   ob::SlabDep slab{};
+  double* phi0 = nullptr;           // potential before a boundary's correction
   int64_t copies_cap = 0;           // doubles of slab.copies
   ob::StatusBox status{nullptr, nullptr};  // set when a step finds a zero-extent bunch
 };
@@ -1565,7 +1566,8 @@ struct PostArgs {
   int zrows, moments;
 };
 
-void launch_rows_c2r(ob_sc2p5drb* c, SC2DState* st) {
+// The potential goes to c->phi, or before a boundary's correction to c->phi0.
+void launch_rows_c2r(ob_sc2p5drb* c, SC2DState* st, double* phi) {
   const double denom = 1.0 / (c->M0 * c->M1);
   dispatch_pow2(c->M1, [&](auto NC) {
     constexpr int N = decltype(NC)::value;
@@ -1577,14 +1579,15 @@ void launch_rows_c2r(ob_sc2p5drb* c, SC2DState* st) {
       }
       ob::ProfScope ps_("fft_rows_c2r");
       hipLaunchKernelGGL(fft_rows_c2r<N>, dim3((c->nx + 1) / 2), dim3(kFFTThreads), fft_lds<N>(),
-                         stream(), c->spec, c->nx, c->phi, c->ny, c->ny, denom, c->tw, c->nmax,
+                         stream(), c->spec, c->nx, phi, c->ny, c->ny, denom, c->tw, c->nmax,
                          st);
     }
   });
   OB_HIP(hipGetLastError());
 }
 
-void launch_fft_pipeline(ob_sc2p5drb* c, SC2DState* st, const PostArgs* post = nullptr) {
+void launch_fft_pipeline(ob_sc2p5drb* c, SC2DState* st, double* phi,
+                         const PostArgs* post = nullptr) {
   if (post) {
     dispatch_pow2(c->M1, [&](auto NC) {
       constexpr int N = decltype(NC)::value;
@@ -1606,12 +1609,12 @@ void launch_fft_pipeline(ob_sc2p5drb* c, SC2DState* st, const PostArgs* post = n
     launch_rows_r2c(c, c->rho, c->nx, c->ny, c->ny, st);
   }
   launch_cols<false>(c, c->nx, st, (double)c->M0 * (double)c->M1);
-  launch_rows_c2r(c, st);
+  launch_rows_c2r(c, st, phi);
 }
 
 // The solve after sc2d_gdeposit: row pass (adds the copies), column pass with the rest of the
 // post pass (and a rebuilt Green function's columns), inverse row pass.
-void launch_slab_solve(ob_sc2p5drb* c, const SC2DParams& P, const SlabDep& D) {
+void launch_slab_solve(ob_sc2p5drb* c, const SC2DParams& P, const SlabDep& D, double* phi) {
   dispatch_pow2(c->M1, [&](auto NC) {
     constexpr int N = decltype(NC)::value;
     if constexpr (N >= 8 && N <= 2 * kSlabMaxNy) {
@@ -1647,7 +1650,7 @@ void launch_slab_solve(ob_sc2p5drb* c, const SC2DParams& P, const SlabDep& D) {
     }
   });
   OB_HIP(hipGetLastError());
-  launch_rows_c2r(c, c->st);
+  launch_rows_c2r(c, c->st, phi);
 }
 
 void define_green(ob_sc2p5drb* c) {
@@ -1988,7 +1991,7 @@ void sc2d_destroy(ob_sc2p5drb* c) {
                   (void*)c->gate, (void*)c->gbuf, (void*)c->tg.counts, (void*)c->tg.items,
                   (void*)c->tg.sxy, (void*)c->tg.sm, (void*)c->tg.zpart,
                   (void*)c->tg.mpart, (void*)c->tg.icounts, (void*)c->gspec,
-                  (void*)c->slab.copies})
+                  (void*)c->slab.copies, (void*)c->phi0})
     if (p) (void)hipFree(p);
   delete c;
   OB_REQUIRE(err.empty(), err);
@@ -1997,7 +2000,7 @@ void sc2d_destroy(ob_sc2p5drb* c) {
 // Deposit and solve of a step on a grid too large for the slab copies: bin (grid, tile counts,
 // z line density), scatter (scan, counting sort), tile deposit, post pass and FFT passes.
 void sc2d_tile_step(ob_sc2p5drb* c, ob_bunch* b, const DeviceBunchView& v, const SC2DParams& P,
-                    int64_t n) {
+                    int64_t n, double* phi) {
   hipStream_t s = stream();
   const int hb = (int)std::max<int64_t>(
       1, std::min<int64_t>({(n + 2047) / 2048, (int64_t)4 * device_cu_count(),
@@ -2045,10 +2048,10 @@ void sc2d_tile_step(ob_sc2p5drb* c, ob_bunch* b, const DeviceBunchView& v, const
       hipLaunchKernelGGL(sc2d_post, dim3(1), dim3(kSetupThreads), 0, s, P, c->st, c->rho,
                          c->zg, c->zd, tg, hb, moments);
     }
-    launch_fft_pipeline(c, c->st);
+    launch_fft_pipeline(c, c->st, phi);
   } else {
     const PostArgs pa{P, tg, hb, moments};
-    launch_fft_pipeline(c, c->st, &pa);
+    launch_fft_pipeline(c, c->st, phi, &pa);
   }
 }
 
@@ -2075,6 +2078,9 @@ void sc2d_track(ob_sc2p5drb* c, ob_bunch* b, double length, double pipe_radius,
   P.par = c->par;
   for (int k = 0; k < 6; k++) P.bnd[k] = 0.0;
   P.bnd_type = bnd ? boundary_describe(bnd, P.bnd) : 0;
+  if (bnd && !c->phi0)
+    OB_HIP(hipMalloc((void**)&c->phi0, sizeof(double) * c->nx * c->ny));
+  double* phi = bnd ? c->phi0 : c->phi;
   if (c->slab.slabs > 0) {  // grid, line density and deposit in one pass, no tile sort
     const SlabDep D = slab_reserve(c, n);
     launch_gdeposit(c, P, v, D);
@@ -2089,14 +2095,14 @@ void sc2d_track(ob_sc2p5drb* c, ob_bunch* b, double length, double pipe_radius,
       Tile2D tg{};
       tg.zpart = D.zpart;
       const PostArgs pa{P, tg, D.parts, 0};
-      launch_fft_pipeline(c, c->st, &pa);
+      launch_fft_pipeline(c, c->st, phi, &pa);
     } else {
-      launch_slab_solve(c, P, D);
+      launch_slab_solve(c, P, D, phi);
     }
   } else {
-    sc2d_tile_step(c, b, v, P, n);
+    sc2d_tile_step(c, b, v, P, n, phi);
   }
-  if (bnd) boundary_add_potential(bnd, c->phi, c->nx, c->ny, c->st, s);  // :90-94
+  if (bnd) boundary_add_potential(bnd, phi, c->phi, c->nx, c->ny, c->st, s);  // :90-94
   OB_HIP(hipGetLastError());
   // kick (:146-167; 2p5D :105-119), fused into the next map kernel
   Op op;
@@ -2230,7 +2236,7 @@ OB_API int ob_sc2p5drb_find_potential(ob_sc2p5drb* c, const double* rho, double 
   h.scale_coeff = log(c->dx_solver / dx);  // :216
   OB_HIP(hipMemcpy(c->st, &h, sizeof(h), hipMemcpyHostToDevice));
   OB_HIP(hipMemcpyAsync(c->rho, rho, sizeof(double) * c->nx * c->ny, hipMemcpyHostToDevice, s));
-  ob::launch_fft_pipeline(c, c->st);
+  ob::launch_fft_pipeline(c, c->st, c->phi);
   OB_HIP(hipMemcpyAsync(phi, c->phi, sizeof(double) * c->nx * c->ny, hipMemcpyDeviceToHost, s));
   OB_HIP(hipStreamSynchronize(s));
   OB_CATCH
