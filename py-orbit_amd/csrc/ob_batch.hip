@@ -179,11 +179,7 @@ void flush(ob_batch* B, bool extrema) {
   bool first = true;
   do {
     OpProgram prog;
-    std::memset(&prog, 0, sizeof(prog));
-    const size_t take = std::min(B->queue.size() - pos, (size_t)kMaxOpsPerLaunch);
-    prog.nops = (int32_t)take;
-    for (size_t k = 0; k < take; k++) prog.ops[k] = B->queue[pos + k];
-    pos += take;
+    pos += program_encode(B->queue.data() + pos, B->queue.size() - pos, prog);
     const bool last = pos >= B->queue.size();
     prog.want_extrema = (last && extrema) ? 1 : 0;
     BatchKick k = first ? B->kick : BatchKick{};
@@ -245,7 +241,7 @@ void autotune(ob_batch* B) {
   OB_HIP(hipEventCreate(&e0));
   OB_HIP(hipEventCreate(&e1));
   OpProgram idp;
-  std::memset(&idp, 0, sizeof(idp));
+  program_encode(nullptr, 0, idp);
   idp.want_extrema = 1;
   float best = 1e30f;
   int best_chunk = B->chunk;

@@ -412,6 +412,23 @@ SyncInfo bunch_sync(ob_bunch* b) {
   return SyncInfo{b->mass, b->charge, b->r0, b->macrosize, b->T, b->p, b->beta, b->gamma, b->time};
 }
 
+namespace {
+// Launch the queue's front as one program: a leading 2.5D kick (the usual case: the previous
+// SC node's, which runs outside the program) and as many ops as fit.  Extrema only if the
+// queue ends there.  Returns the ops taken; *blocks = workgroups of the launch.
+size_t launch_front(ob_bunch* b, const DeviceBunchView& v, size_t pos, double* ext_partials,
+                    int* blocks) {
+  const size_t first = pos;
+  const Op* kick0 = nullptr;
+  if (pos < b->queue.size() && b->queue[pos].kind == OP_SC2P5DRB_KICK) kick0 = &b->queue[pos++];
+  OpProgram prog;
+  pos += program_encode(b->queue.data() + pos, b->queue.size() - pos, prog);
+  prog.want_extrema = (pos >= b->queue.size() && ext_partials) ? 1 : 0;
+  *blocks = launch_push(v, prog, kick0, prog.want_extrema ? ext_partials : nullptr, stream());
+  return pos - first;
+}
+}  // namespace
+
 int bunch_flush(ob_bunch* b, double* ext_partials) {
   if (b->owner) {  // maps and kicks of a batched bunch are the batch's
     OB_REQUIRE(ext_partials == nullptr,
@@ -424,15 +441,7 @@ int bunch_flush(ob_bunch* b, double* ext_partials) {
   size_t pos = 0;
   int blocks = 0;
   do {
-    OpProgram prog;
-    std::memset(&prog, 0, sizeof(prog));
-    size_t take = std::min(b->queue.size() - pos, (size_t)kMaxOpsPerLaunch);
-    prog.nops = (int32_t)take;
-    for (size_t k = 0; k < take; k++) prog.ops[k] = b->queue[pos + k];
-    pos += take;
-    const bool last = pos >= b->queue.size();
-    prog.want_extrema = (last && ext_partials) ? 1 : 0;
-    blocks = launch_push(v, prog, prog.want_extrema ? ext_partials : nullptr, stream());
+    pos += launch_front(b, v, pos, ext_partials, &blocks);
   } while (pos < b->queue.size());
   b->queue.clear();
   b->host_valid = false;
@@ -443,7 +452,12 @@ void bunch_queue(ob_bunch* b, const Op& op) {
   if (b->n == 0) return;  // maps over an empty bunch are no-ops
   b->queue.push_back(op);
   b->host_valid = false;
-  if (b->queue.size() >= 256 && !b->owner) bunch_flush(b, nullptr);
+  // two programs' worth waits: launch one full program, so that none goes out nearly empty
+  if (b->queue.size() >= 256 && !b->owner) {
+    int blocks = 0;
+    const size_t took = launch_front(b, bunch_device_view(b), 0, nullptr, &blocks);
+    b->queue.erase(b->queue.begin(), b->queue.begin() + (ptrdiff_t)took);
+  }
 }
 
 }  // namespace ob

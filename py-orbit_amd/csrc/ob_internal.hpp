@@ -98,6 +98,7 @@ enum OpKind : int32_t {
   OP_WEDGEBEND,  // wedgebend and wedgebendCF
   OP_SOLN,
   OP_RINGRF,
+  OP_ENV,  // (program words only) dpc, g2i
 };
 
 struct Op {
@@ -107,13 +108,29 @@ struct Op {
 };
 static_assert(sizeof(Op) == 112, "Op layout");
 
-constexpr int kMaxOpsPerLaunch = 24;
-struct OpProgram {
-  int32_t nops;
+// A map program as the push kernels read it: the ops one after another as 8-byte words in the
+// kernel arguments, so a launch takes what fits kProgWords (some 130 ops of a ring, where a
+// fixed 112-byte record per op held 24 in the same arguments) and each further pass over the
+// bunch does more work.  An op is a header word and its parameters:
+//   bits 0-7 kind, 8 kProgRecalc, 12-19 words of the op, 32-63 integer parameters;
+// 1/(p beta) and 1/gamma^2, which most maps share, are the program's dpc and g2i (changed by
+// an OP_ENV op).  kProgRecalc: dp/p and 1/(1 + dp/p) have to be computed anew before the op;
+// they depend on dE, dpc only, so between changes of those the ops share them.
+constexpr int kProgWords = 440;
+constexpr int kProgSmallWords = 48;
+constexpr uint32_t kProgRecalc = 1u << 8;
+template <int W>
+struct ProgramWords {
+  int32_t words;         // words used
   int32_t want_extrema;  // write per-block min/max of x, y, z after the last op
-  int32_t pad[2];
-  Op ops[kMaxOpsPerLaunch];
+  double dpc, g2i;
+  double data[W];
 };
+struct OpProgram : ProgramWords<kProgWords> {
+  int32_t level;  // kernel level (the highest of its ops)
+};
+// Encode ops[0 .. count) as far as they fit; returns how many were taken (at least one).
+size_t program_encode(const Op* ops, size_t count, OpProgram& prog);
 
 // Space-charge state shared between the 2.5D kernels and the kick op.
 struct SC2DState {
@@ -177,9 +194,10 @@ struct DeviceBunchView {
 };
 
 // Launch the fused map program over a bunch; partial extrema (6 per block) go to
-// ext_partials when prog.want_extrema.  Returns the number of blocks used.
-int launch_push(const DeviceBunchView& v, const OpProgram& prog, double* ext_partials,
-                hipStream_t s);
+// ext_partials when prog.want_extrema.  kick0: an OP_SC2P5DRB_KICK that runs before the
+// program, or null.  Returns the number of blocks used.
+int launch_push(const DeviceBunchView& v, const OpProgram& prog, const Op* kick0,
+                double* ext_partials, hipStream_t s);
 
 // Tile sort of a 2.5D deposit: T x T tiles of TSC centre nodes, work items of at most
 // `item` particles of one tile, scratch copies of the in-grid particles sorted by tile.

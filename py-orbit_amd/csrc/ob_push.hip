@@ -11,6 +11,10 @@
 // Arithmetic follows the reference routine of each map operation for operation
 // (cited per case), compiled with -ffp-contract=off so nothing is fused: results
 // are bit-identical to src/teapot/teapotbase.cc built with g++ for x86-64.
+#include <algorithm>
+#include <cstddef>
+#include <type_traits>
+
 #include "ob_internal.hpp"
 #include "ob_sc_device.hpp"
 
@@ -27,32 +31,43 @@ __device__ __forceinline__ cplx cmul(cplx a, cplx b) {  // std::complex<double> 
 __device__ __forceinline__ cplx cadd(cplx a, cplx b) { return {a.re + b.re, a.im + b.im}; }
 __device__ __forceinline__ cplx csub(cplx a, cplx b) { return {a.re - b.re, a.im - b.im}; }
 
-// teapotbase.cc:395-490 / 508-603.  p[0]=dp_p_coeff, p[1..2]=kk (+/-kterm), i0=pole.
-__device__ __forceinline__ void multpfringe(const Op& op, double& x, double& xp, double& y,
-                                            double& yp, double& z, double dE) {
-  const int lm1 = op.i0, l = op.i0 + 1, lp2 = op.i0 + 3;
-  const cplx rootm1 = {0.0, 1.0};
-  const cplx cxl = {(double)l, 0.0}, cxlp2 = {(double)lp2, 0.0};
-  const cplx kk = {op.p[1], op.p[2]};
+// teapotbase.cc:395-490 / 508-603.  kk = (kre, kim) = +/-kterm, pole; the reference's complex
+// products by real or imaginary constants (l, l + 2, i) without their zero terms, which add
+// +-0 to finite values: the same results, a third fewer operations.
+__device__ __forceinline__ void multpfringe(int pole, double kre, double kim, double KNL,
+                                            double& x, double& xp, double& y, double& yp,
+                                            double& z) {
+  const double l = (double)(pole + 1), lp2 = (double)(pole + 3);
   const double px = xp, py = yp;
-  const double dp_p = dE * op.p[0];
-  const double KNL = 1.0 / (1.0 + dp_p);
   const cplx zz = {x, y};
   cplx zlm1 = {1.0, 0.0};
-  for (int k = 0; k < lm1; k++) zlm1 = cmul(zlm1, zz);
-  const cplx zl = cmul(zlm1, zz);
+  if (pole > 0) zlm1 = zz;
+  for (int k = 1; k < pole; k++) zlm1 = cmul(zlm1, zz);
+  const cplx zl = pole > 0 ? cmul(zlm1, zz) : zz;
   const cplx fxterm = {l * x, -lp2 * y};
-  const cplx dxfxterm = cmul(cxl, cadd(fxterm, zz));
-  const cplx dyfxterm = cmul(rootm1, csub(cmul(cxl, fxterm), cmul(cxlp2, zz)));
+  const cplx fxz = cadd(fxterm, zz);
+  const cplx dxfxterm = {l * fxz.re, l * fxz.im};
+  const cplx w = {l * fxterm.re - lp2 * zz.re, l * fxterm.im - lp2 * zz.im};
+  const cplx dyfxterm = {-w.im, w.re};
   const cplx fyterm = {l * y, lp2 * x};
-  const cplx dxfyterm = cadd(cmul(cxl, fyterm), cmul(cmul(rootm1, cxlp2), zz));
-  const cplx dyfyterm = cmul(cxl, cadd(cmul(rootm1, fyterm), zz));
-  const cplx fxcx = cmul(cmul(kk, zl), fxterm);
-  const cplx dxfxcx = cmul(cmul(kk, zlm1), dxfxterm);
-  const cplx dyfxcx = cmul(cmul(kk, zlm1), dyfxterm);
-  const cplx fycx = cmul(cmul(kk, zl), fyterm);
-  const cplx dxfycx = cmul(cmul(kk, zlm1), dxfyterm);
-  const cplx dyfycx = cmul(cmul(kk, zlm1), dyfyterm);
+  const cplx dxfyterm = {l * fyterm.re - lp2 * zz.im, l * fyterm.im + lp2 * zz.re};
+  const cplx ify = {-fyterm.im + zz.re, fyterm.re + zz.im};
+  const cplx dyfyterm = {l * ify.re, l * ify.im};
+  cplx kzl, kzlm1;
+  if (kim == 0.0) {  // uniform: a normal multipole's coefficient is real
+    kzl = {kre * zl.re, kre * zl.im};
+    kzlm1 = {kre * zlm1.re, kre * zlm1.im};
+  } else {
+    const cplx kk = {kre, kim};
+    kzl = cmul(kk, zl);
+    kzlm1 = cmul(kk, zlm1);
+  }
+  const cplx fxcx = cmul(kzl, fxterm);
+  const cplx dxfxcx = cmul(kzlm1, dxfxterm);
+  const cplx dyfxcx = cmul(kzlm1, dyfxterm);
+  const cplx fycx = cmul(kzl, fyterm);
+  const cplx dxfycx = cmul(kzlm1, dxfyterm);
+  const cplx dyfycx = cmul(kzlm1, dyfyterm);
   x -= fxcx.re * KNL;
   y -= fycx.re * KNL;
   const double M11 = 1.0 - dxfxcx.re * KNL;
@@ -67,47 +82,38 @@ __device__ __forceinline__ void multpfringe(const Op& op, double& x, double& xp,
   z -= (pxnew * fxcx.re + pynew * fycx.re) * KNL * KNL;
 }
 
-// teapotbase.cc:784-835 (IN) / 854-905 (OUT).  p[0]=dp_p_coeff, p[1]=kq.
-template <bool OUT>
-__device__ __forceinline__ void quadfringe(const Op& op, double& x, double& xp, double& y,
-                                           double& yp, double& z, double dE) {
-  const double kq = op.p[1];
-  const double dp_p = dE * op.p[0];
-  const double KNL = 1.0 / (1.0 + dp_p);
+// teapotbase.cc:784-835 (IN) / 854-905 (OUT).
+__device__ __forceinline__ void quadfringe(bool out, double kq, double KNL, double& x, double& xp,
+                                           double& y, double& yp, double& z) {
   const double x0 = x, xp0 = xp, y0 = y, yp0 = yp;
   const double t = (kq * KNL / 4.) * (x0 * x0 - y0 * y0);
   const double detM = 1.0 - t * t;
-  const double dx = (kq * KNL / 12.) * x0 * (x0 * x0 + 3. * y0 * y0);
-  const double dxp = (kq * KNL / 4.) * (xp0 * (x0 * x0 + y0 * y0) - 2. * yp0 * x0 * y0);
-  const double dy = (kq * KNL / 12.) * y0 * (y0 * y0 + 3. * x0 * x0);
-  const double dyp = (kq * KNL / 4.) * (-yp0 * (x0 * x0 + y0 * y0) + 2. * xp0 * x0 * y0);
-  const double dz = (kq * KNL * KNL / 12.) *
-                    (xp0 * x0 * (x0 * x0 + 3. * y0 * y0) - yp0 * y0 * (y0 * y0 + 3. * x0 * x0));
-  if (!OUT) {
-    x += dx;
-    xp -= dxp;
-    xp /= detM;
-    y -= dy;
-    yp -= dyp;
-    yp /= detM;
-    z += dz;
-  } else {
-    x -= dx;
-    xp += dxp;
-    xp /= detM;
-    y += dy;
-    yp += dyp;
-    yp /= detM;
-    z -= dz;
+  double dx = (kq * KNL / 12.) * x0 * (x0 * x0 + 3. * y0 * y0);
+  double dxp = (kq * KNL / 4.) * (xp0 * (x0 * x0 + y0 * y0) - 2. * yp0 * x0 * y0);
+  double dy = (kq * KNL / 12.) * y0 * (y0 * y0 + 3. * x0 * x0);
+  double dyp = (kq * KNL / 4.) * (-yp0 * (x0 * x0 + y0 * y0) + 2. * xp0 * x0 * y0);
+  double dz = (kq * KNL * KNL / 12.) *
+              (xp0 * x0 * (x0 * x0 + 3. * y0 * y0) - yp0 * y0 * (y0 * y0 + 3. * x0 * x0));
+  if (out) {  // uniform; a - b and a + (-b) are the same value
+    dx = -dx;
+    dxp = -dxp;
+    dy = -dy;
+    dyp = -dyp;
+    dz = -dz;
   }
+  x += dx;
+  xp -= dxp;
+  xp /= detM;
+  y -= dy;
+  yp -= dyp;
+  yp /= detM;
+  z += dz;
 }
 
 // One particle's drift (drifti, teapotbase.cc:120-141).
-__device__ __forceinline__ void drift_one(double length, double gamma2i, double dp_p_coeff,
+__device__ __forceinline__ void drift_one(double length, double gamma2i, double dp_p, double KNL,
                                           double& x, double xp, double& y, double yp,
-                                          double& z, double dE) {
-  const double dp_p = dE * dp_p_coeff;
-  const double KNL = 1.0 / (1.0 + dp_p);
+                                          double& z) {
   x += KNL * length * xp;
   y += KNL * length * yp;
   double phifac = (xp * xp + yp * yp + dp_p * dp_p * gamma2i) / 2.0;
@@ -115,32 +121,34 @@ __device__ __forceinline__ void drift_one(double length, double gamma2i, double 
   z -= length * phifac;
 }
 
-// wedgebend / wedgebendCF (teapotbase.cc:1037-1080, 1447-1509).  p[0]=ct, p[1]=rho,
-// p[2]=dp_p_coeff, p[3]=gamma2i, p[4+l]=kl of multipole l; i0 = inout | n << 1 |
-// skew bits << 8, i1 = nst, i2 = poles, 4 bits each.  The multipole kick of each step is
-// multpi (:280-315) with kl * sm, divided by pole! per particle as there.
-__device__ __forceinline__ void wedgebend(const Op& op, double& x, double& xp, double& y,
-                                          double& yp, double& z, double dE) {
-  const double ct = op.p[0], rho = op.p[1], dpc = op.p[2], gamma2i = op.p[3];
-  const int inout = op.i0 & 1, nm = (op.i0 >> 1) & 15, skews = (op.i0 >> 8) & 255;
-  const int nst = op.i1;
+// wedgebend / wedgebendCF (teapotbase.cc:1037-1080, 1447-1509).  w: ct, rho, poles (4 bits
+// each), then kl of the nm multipoles; ia = inout | nm << 1 | skew bits << 8 | nst << 16.  The
+// multipole kick of each step is multpi (:280-315) with kl * sm, divided by pole! per particle
+// as there.
+template <typename W>
+__device__ __forceinline__ void wedgebend(W w, uint32_t ia, double gamma2i, double dp_p,
+                                          double KNL, double& x, double& xp, double& y,
+                                          double& yp, double& z) {
+  const double ct = w[0], rho = w[1];
+  const uint32_t poles = (uint32_t)__double_as_longlong(w[2]);
+  const int inout = ia & 1, nm = (ia >> 1) & 15, skews = (ia >> 8) & 255;
+  const int nst = (int)(ia >> 16);
   double s;
   if (inout == 0) {
     s = -x / ct;
   } else {
-    const double dp_p = dE * dpc;
     const double tn = xp / (1.0 + dp_p);
     s = -x / (ct + tn);
   }
   const double sm = s / nst, sm2 = sm / 2.0;
   for (int j = 0; j < nst; j++) {
-    drift_one(j == 0 ? sm2 : sm, gamma2i, dpc, x, xp, y, yp, z, dE);
+    drift_one(j == 0 ? sm2 : sm, gamma2i, dp_p, KNL, x, xp, y, yp, z);
     xp -= sm / rho;
     for (int l = 0; l < nm; l++) {
-      const int pole = (op.i2 >> (4 * l)) & 15;
+      const int pole = (poles >> (4 * l)) & 15;
       double fact = 1.0;  // teapotbase.cc:45-57
       for (int k = 1; k <= pole; k++) fact = k * fact;
-      const double kl1 = (op.p[4 + l] * sm) / fact;
+      const double kl1 = (w[3 + l] * sm) / fact;
       const cplx zz = {x, y};
       cplx zn = {1.0, 0.0};
       for (int k = 0; k < pole; k++) zn = cmul(zn, zz);
@@ -153,15 +161,13 @@ __device__ __forceinline__ void wedgebend(const Op& op, double& x, double& xp, d
       }
     }
   }
-  drift_one(sm2, gamma2i, dpc, x, xp, y, yp, z, dE);
+  drift_one(sm2, gamma2i, dp_p, KNL, x, xp, y, yp, z);
 }
 
-// soln (teapotbase.cc:1367-1425).  p: Bc, length, gamma2i, dp_p_coeff.
-__device__ __forceinline__ void soln(const Op& op, double& x, double& xp, double& y,
-                                     double& yp, double& z, double dE) {
-  const double Bc = op.p[0], length = op.p[1], gamma2i = op.p[2];
-  const double dp_p = dE * op.p[3];
-  const double KNL = 1.0 / (1.0 + dp_p);
+// soln (teapotbase.cc:1367-1425).
+__device__ __forceinline__ void soln(double Bc, double length, double gamma2i, double dp_p,
+                                     double KNL, double& x, double& xp, double& y, double& yp,
+                                     double& z) {
   const double cu = y / 2. - xp / Bc;
   const double cpu = x * Bc / 2. + yp;
   const double u_init = y / 2. + xp / Bc;
@@ -179,217 +185,207 @@ __device__ __forceinline__ void soln(const Op& op, double& x, double& xp, double
   z -= length * phifac;
 }
 
-// Kernel level an op kind needs: 0 = the lite kernels, 1 = with the multipole fringes
-// (a ring's sextupoles), 2 = with every register-hungry op (3D kick, wedge bend, solenoid,
-// ring RF).  Each level holds the ones below it; a lower level runs with fewer VGPRs and
-// so more waves per SIMD.
+// Kernel level an op kind needs: 0 = the lite kernels, 1 = with the multipole fringes (a
+// ring's sextupoles), 2 = with wedge bend, solenoid and ring RF, 3 = with space-charge kicks
+// inside a program (a calculator's kick leads its queue: 2.5D kicks run before the program, 3D
+// ones outside the deposit's tiles take this level).  Each level holds the ones below it; a
+// lower level runs with fewer VGPRs and so more waves per SIMD (maps only: 62, 70, 100, 214).
+constexpr int kLevels = 4;
 __host__ __device__ constexpr int op_level(int kind) {
-  return (kind == OP_MULTPFRINGE_IN || kind == OP_MULTPFRINGE_OUT)
-             ? 1
-             : ((kind == OP_SC3D_KICK || kind == OP_WEDGEBEND || kind == OP_SOLN ||
-                 kind == OP_RINGRF)
-                    ? 2
-                    : 0);
+  return (kind == OP_MULTPFRINGE_IN || kind == OP_MULTPFRINGE_OUT) ? 1
+         : (kind == OP_WEDGEBEND || kind == OP_SOLN || kind == OP_RINGRF) ? 2
+         : (kind == OP_SC2P5DRB_KICK || kind == OP_SC3D_KICK) ? 3
+                                                               : 0;
 }
 
-template <int LEVEL>
-__device__ __forceinline__ void apply_op(const Op& op, double& x, double& xp, double& y,
-                                         double& yp, double& z, double& dE) {
-  if (op_level(op.kind) > LEVEL) return;  // never reached: the host picks the level
-  switch (op.kind) {
-    case OP_DRIFT: {  // teapotbase.cc:158-183. p: length, gamma2i, dp_p_coeff
-      const double length = op.p[0], gamma2i = op.p[1];
-      const double dp_p = dE * op.p[2];
-      const double KNL = 1.0 / (1.0 + dp_p);
-      x += KNL * length * xp;
-      y += KNL * length * yp;
-      double phifac = (xp * xp + yp * yp + dp_p * dp_p * gamma2i) / 2.0;
-      phifac = (phifac * KNL - dp_p * gamma2i) * KNL;
-      z -= length * phifac;
-      break;
+// The whole program (ProgramWords) on one particle.  The next op's header is requested before
+// this op runs (all lanes run the same op: the words are scalar loads).
+template <int LEVEL, typename PROG>
+__device__ __forceinline__ void run_program(const PROG& prog, double& x, double& xp, double& y,
+                                            double& yp, double& z, double& dE) {
+  double dpc = prog.dpc, g2i = prog.g2i;
+  double dp_p = 0.0, KNL = 0.0;
+  const int words = prog.words;
+  uint64_t hdr = words > 0 ? (uint64_t)__double_as_longlong(prog.data[0]) : 0;
+  for (int pc = 0; pc < words;) {
+    const uint32_t h = (uint32_t)hdr, ia = (uint32_t)(hdr >> 32);
+    const double* w = prog.data + pc + 1;
+    pc += (int)((h >> 12) & 255u);
+    hdr = (uint64_t)__double_as_longlong(prog.data[pc < words ? pc : 0]);
+    if (h & kProgRecalc) {
+      dp_p = dE * dpc;
+      KNL = 1.0 / (1.0 + dp_p);
     }
-    case OP_QUAD1: {  // teapotbase.cc:686-699. p: m11 m12 m21 m22 m33 m34 m43 m44, gamma2i,
-                      // length, dp_p_coeff
-      const double dp_p = dE * op.p[10];
-      const double x0 = x, xp0 = xp, y0 = y, yp0 = yp;
-      x = x0 * op.p[0] + xp0 * op.p[1];
-      xp = x0 * op.p[2] + xp0 * op.p[3];
-      y = y0 * op.p[4] + yp0 * op.p[5];
-      yp = y0 * op.p[6] + yp0 * op.p[7];
-      z += dp_p * op.p[8] * op.p[9];
-      break;
-    }
-    case OP_QUAD2: {  // teapotbase.cc:719-745. p: length, gamma2i, dp_p_coeff
-      const double length = op.p[0], gamma2i = op.p[1];
-      const double dp_p = dE * op.p[2];
-      const double KNL = 1.0 / (1.0 + dp_p);
-      x -= KNL * length * dp_p * xp;
-      y -= KNL * length * dp_p * yp;
-      double phifac = (xp * xp + yp * yp + dp_p * dp_p * gamma2i) / 2.0;
-      phifac = (phifac * KNL + dp_p * dp_p * gamma2i) * KNL;
-      z -= length * phifac;
-      break;
-    }
-    case OP_QUADFRINGE_IN:
-      quadfringe<false>(op, x, xp, y, yp, z, dE);
-      break;
-    case OP_QUADFRINGE_OUT:
-      quadfringe<true>(op, x, xp, y, yp, z, dE);
-      break;
-    case OP_MULTP: {  // teapotbase.cc:336-372. p[0]=kl/pole!, i0=pole, i1=skew
-      const cplx zz = {x, y};
-      cplx zn = {1.0, 0.0};
-      for (int k = 0; k < op.i0; k++) zn = cmul(zn, zz);
-      const double kl1 = op.p[0];
-      if (op.i1) {
-        xp += kl1 * zn.im;
-        yp += kl1 * zn.re;
-      } else {
-        xp -= kl1 * zn.re;
-        yp += kl1 * zn.im;
+    switch (h & 255u) {
+      case OP_DRIFT:  // teapotbase.cc:158-183.  length
+        drift_one(w[0], g2i, dp_p, KNL, x, xp, y, yp, z);
+        break;
+      case OP_QUAD1: {  // teapotbase.cc:686-699.  m11 = m22, m12, m21, m33 = m44, m34, m43, length
+        const double x0 = x, xp0 = xp, y0 = y, yp0 = yp;
+        x = x0 * w[0] + xp0 * w[1];
+        xp = x0 * w[2] + xp0 * w[0];
+        y = y0 * w[3] + yp0 * w[4];
+        yp = y0 * w[5] + yp0 * w[3];
+        z += dp_p * g2i * w[6];
+        break;
       }
-      break;
-    }
-    case OP_MULTPFRINGE_IN:
-    case OP_MULTPFRINGE_OUT:
-      if constexpr (LEVEL >= 1) multpfringe(op, x, xp, y, yp, z, dE);
-      break;
-    case OP_WRAPBUNCH: {  // teapotbase.cc:202-211. p[0]=length
-      const double length = op.p[0];
-      if (z < -length / 2.0) z += length;
-      if (z > length / 2.0) z -= length;
-      break;
-    }
-    case OP_ROTATEXY: {  // teapotbase.cc:80-101. p: cos, sin
-      const double cs = op.p[0], sn = op.p[1];
-      const double xt = x, pxt = xp, yt = y, pyt = yp;
-      x = cs * xt - sn * yt;
-      xp = cs * pxt - sn * pyt;
-      y = sn * xt + cs * yt;
-      yp = sn * pxt + cs * pyt;
-      break;
-    }
-    case OP_KICK:  // teapotbase.cc:232-257. p: kx, ky, kE
-      if (op.p[0] != 0.) xp += op.p[0];
-      if (op.p[1] != 0.) yp += op.p[1];
-      if (op.p[2] != 0.) dE += op.p[2];
-      break;
-    case OP_SC2P5DRB_KICK:
-      sc2p5drb_kick(op, x, xp, y, yp, z, dE);
-      break;
-    case OP_SC3D_KICK:
-      if constexpr (LEVEL >= 2) sc3d_kick(op, x, xp, y, yp, z, dE);
-      break;
-    case OP_BEND1: {  // teapotbase.cc:1099-1145. p: m11 m12 m16 m21 m22 m26 m51 m52 m56,
-                      // length, dp_p_coeff
-      const double dp_p = dE * op.p[10];
-      const double x0 = x, xp0 = xp;
-      x = x0 * op.p[0] + xp0 * op.p[1] + dp_p * op.p[2];
-      xp = x0 * op.p[3] + xp0 * op.p[4] + dp_p * op.p[5];
-      y += op.p[9] * yp;
-      z += x0 * op.p[6] + xp0 * op.p[7] + dp_p * op.p[8];
-      break;
-    }
-    case OP_BEND3: {  // teapotbase.cc:1208-1233. p: th, gamma2i, dp_p_coeff
-      const double th = op.p[0], gamma2i = op.p[1];
-      const double dp_p = dE * op.p[2];
-      const double KNL = 1.0 / (1.0 + dp_p);
-      double phifac = (yp * yp + dp_p * dp_p * gamma2i) / 2.0;
-      xp -= phifac * KNL * th;
-      y += KNL * yp * x * th;
-      phifac = (phifac * KNL - dp_p * gamma2i) * KNL;
-      z -= th * phifac * x;
-      break;
-    }
-    case OP_BEND4: {  // teapotbase.cc:1251-1274. p: th, dp_p_coeff
-      const double th = op.p[0];
-      const double dp_p = dE * op.p[1];
-      const double KNL = 1.0 / (1.0 + dp_p);
-      const double xfac = 1.0 + KNL * xp * th / 2.0;
-      const double phifac = KNL * KNL * xp * xp / 2.0;
-      x *= xfac * xfac;
-      xp /= xfac;
-      z -= th * phifac * x;
-      break;
-    }
-    case OP_BENDFRINGE_IN:    // teapotbase.cc:1292-1311. p: rho, dp_p_coeff
-    case OP_BENDFRINGE_OUT: {  // teapotbase.cc:1329-1348
-      const double rho = op.p[0];
-      const double dp_p = dE * op.p[1];
-      const double KNL = 1.0 / (1.0 + dp_p);
-      if (op.kind == OP_BENDFRINGE_IN) {
-        x += KNL * y * y / (2. * rho);
-        yp -= KNL * xp * y / rho;
-        z += KNL * KNL * xp * y * y / (2. * rho);
-      } else {
-        x -= KNL * y * y / (2. * rho);
-        yp += KNL * xp * y / rho;
-        z -= KNL * KNL * xp * y * y / (2. * rho);
+      case OP_QUAD2: {  // teapotbase.cc:719-745.  length
+        const double length = w[0];
+        x -= KNL * length * dp_p * xp;
+        y -= KNL * length * dp_p * yp;
+        double phifac = (xp * xp + yp * yp + dp_p * dp_p * g2i) / 2.0;
+        phifac = (phifac * KNL + dp_p * dp_p * g2i) * KNL;
+        z -= length * phifac;
+        break;
       }
-      break;
-    }
-    case OP_WEDGEROTATE: {  // teapotbase.cc:923-966. p: cos e, sin e, dp_p_coeff; i0=frinout
-      const double cs = op.p[0], sn = op.p[1], dpc = op.p[2];
-      double dp_p, xp_temp, p0_temp, p0;
-      if (op.i0 == 0) {
-        dp_p = dE * dpc;
-        xp_temp = xp;
-        p0_temp = 1.0 + dp_p;
-        x /= cs;
-        xp = xp_temp * cs + p0_temp * sn;
-        p0 = -xp_temp * sn + p0_temp * cs;
-        dp_p = p0 - 1.0;
-        z = (-x * sn + z) * cs;
-      } else {
-        dp_p = dE * dpc;
-        p0 = 1.0 + dp_p;
-        z = x * sn + z / cs;
-        x *= cs;
-        xp_temp = xp * cs - p0 * sn;
-        p0_temp = xp * sn + p0 * cs;
-        xp = xp_temp;
-        dp_p = p0_temp - 1.0;
+      case OP_QUADFRINGE_IN:   // kq
+      case OP_QUADFRINGE_OUT:
+        quadfringe((h & 255u) == OP_QUADFRINGE_OUT, w[0], KNL, x, xp, y, yp, z);
+        break;
+      case OP_MULTP: {  // teapotbase.cc:336-372.  kl/pole!; ia = pole | skew << 8
+        const cplx zz = {x, y};
+        cplx zn = {1.0, 0.0};
+        const int pole = (int)(ia & 255u);
+        for (int k = 0; k < pole; k++) zn = cmul(zn, zz);
+        const double kl1 = w[0];
+        if (ia >> 8) {
+          xp += kl1 * zn.im;
+          yp += kl1 * zn.re;
+        } else {
+          xp -= kl1 * zn.re;
+          yp += kl1 * zn.im;
+        }
+        break;
       }
-      dE = dp_p / dpc;
-      break;
-    }
-    case OP_WEDGEDRIFT: {  // teapotbase.cc:986-1012. p: ct, dp_p_coeff, gamma2i; i0=inout
-      const double ct = op.p[0], dpc = op.p[1];
-      double s;
-      if (op.i0 == 0) {
-        const double dp_p = dE * dpc;
-        const double tn = xp / (1.0 + dp_p);
-        s = x / (ct - tn);
-      } else {
-        s = x / ct;
+      case OP_MULTPFRINGE_IN:
+      case OP_MULTPFRINGE_OUT:  // kre, kim; ia = pole
+        if constexpr (LEVEL >= 1) multpfringe((int)ia, w[0], w[1], KNL, x, xp, y, yp, z);
+        break;
+      case OP_WRAPBUNCH: {  // teapotbase.cc:202-211.  length
+        const double length = w[0];
+        if (z < -length / 2.0) z += length;
+        if (z > length / 2.0) z -= length;
+        break;
       }
-      drift_one(s, op.p[2], dpc, x, xp, y, yp, z, dE);
-      break;
-    }
-    case OP_WEDGEBEND:
-      if constexpr (LEVEL >= 2) wedgebend(op, x, xp, y, yp, z, dE);
-      break;
-    case OP_SOLN:
-      if constexpr (LEVEL >= 2) soln(op, x, xp, y, yp, z, dE);
-      break;
-    case OP_RINGRF:  // teapotbase.cc:1527-1566. p: h*2pi/L, phase_s, voltage, coeff, p_in/p_out
-      if constexpr (LEVEL >= 2) {
-        const double deltaV = op.p[2] * (sin(op.p[0] * z + op.p[1]));
-        dE += op.p[3] * deltaV;
-        xp *= op.p[4];
-        yp *= op.p[4];
+      case OP_ROTATEXY: {  // teapotbase.cc:80-101.  cos, sin
+        const double cs = w[0], sn = w[1];
+        const double xt = x, pxt = xp, yt = y, pyt = yp;
+        x = cs * xt - sn * yt;
+        xp = cs * pxt - sn * pyt;
+        y = sn * xt + cs * yt;
+        yp = sn * pxt + cs * pyt;
+        break;
       }
-      break;
-    default:
-      break;
+      case OP_KICK:  // teapotbase.cc:232-257.  kx, ky, kE
+        if (w[0] != 0.) xp += w[0];
+        if (w[1] != 0.) yp += w[1];
+        if (w[2] != 0.) dE += w[2];
+        break;
+      case OP_SC2P5DRB_KICK:  // p[0..5]; ia = nx, then a word with ny, nz
+        if constexpr (LEVEL >= 3) sc2p5drb_kick(w, (int)ia, x, xp, y, yp, z, dE);
+        break;
+      case OP_SC3D_KICK:  // p[0..11]; ia = nx, then a word with ny, nz
+        if constexpr (LEVEL >= 3) sc3d_kick(w, (int)ia, x, xp, y, yp, z, dE);
+        break;
+      case OP_BEND1: {  // teapotbase.cc:1099-1145.  m11 m12 m16 m21 m22 m26 m51 m52 m56, length
+        const double x0 = x, xp0 = xp;
+        x = x0 * w[0] + xp0 * w[1] + dp_p * w[2];
+        xp = x0 * w[3] + xp0 * w[4] + dp_p * w[5];
+        y += w[9] * yp;
+        z += x0 * w[6] + xp0 * w[7] + dp_p * w[8];
+        break;
+      }
+      case OP_BEND3: {  // teapotbase.cc:1208-1233.  th
+        const double th = w[0];
+        double phifac = (yp * yp + dp_p * dp_p * g2i) / 2.0;
+        xp -= phifac * KNL * th;
+        y += KNL * yp * x * th;
+        phifac = (phifac * KNL - dp_p * g2i) * KNL;
+        z -= th * phifac * x;
+        break;
+      }
+      case OP_BEND4: {  // teapotbase.cc:1251-1274.  th
+        const double th = w[0];
+        const double xfac = 1.0 + KNL * xp * th / 2.0;
+        const double phifac = KNL * KNL * xp * xp / 2.0;
+        x *= xfac * xfac;
+        xp /= xfac;
+        z -= th * phifac * x;
+        break;
+      }
+      case OP_BENDFRINGE_IN:     // teapotbase.cc:1292-1311.  rho
+      case OP_BENDFRINGE_OUT: {  // teapotbase.cc:1329-1348
+        const double rho = w[0];
+        if ((h & 255u) == OP_BENDFRINGE_IN) {
+          x += KNL * y * y / (2. * rho);
+          yp -= KNL * xp * y / rho;
+          z += KNL * KNL * xp * y * y / (2. * rho);
+        } else {
+          x -= KNL * y * y / (2. * rho);
+          yp += KNL * xp * y / rho;
+          z -= KNL * KNL * xp * y * y / (2. * rho);
+        }
+        break;
+      }
+      case OP_WEDGEROTATE: {  // teapotbase.cc:923-966.  cos e, sin e; ia = frinout
+        const double cs = w[0], sn = w[1];
+        double dp, xp_temp, p0_temp, p0;
+        if (ia == 0) {
+          dp = dE * dpc;
+          xp_temp = xp;
+          p0_temp = 1.0 + dp;
+          x /= cs;
+          xp = xp_temp * cs + p0_temp * sn;
+          p0 = -xp_temp * sn + p0_temp * cs;
+          dp = p0 - 1.0;
+          z = (-x * sn + z) * cs;
+        } else {
+          dp = dE * dpc;
+          p0 = 1.0 + dp;
+          z = x * sn + z / cs;
+          x *= cs;
+          xp_temp = xp * cs - p0 * sn;
+          p0_temp = xp * sn + p0 * cs;
+          xp = xp_temp;
+          dp = p0_temp - 1.0;
+        }
+        dE = dp / dpc;
+        break;
+      }
+      case OP_WEDGEDRIFT: {  // teapotbase.cc:986-1012.  ct; ia = inout
+        const double ct = w[0];
+        double s;
+        if (ia == 0) {
+          const double tn = xp / (1.0 + dp_p);
+          s = x / (ct - tn);
+        } else {
+          s = x / ct;
+        }
+        drift_one(s, g2i, dp_p, KNL, x, xp, y, yp, z);
+        break;
+      }
+      case OP_WEDGEBEND:
+        if constexpr (LEVEL >= 2) wedgebend(w, ia, g2i, dp_p, KNL, x, xp, y, yp, z);
+        break;
+      case OP_SOLN:  // Bc, length
+        if constexpr (LEVEL >= 2) soln(w[0], w[1], g2i, dp_p, KNL, x, xp, y, yp, z);
+        break;
+      case OP_RINGRF:  // teapotbase.cc:1527-1566.  h*2pi/L, phase_s, voltage, coeff, p_in/p_out
+        if constexpr (LEVEL >= 2) {
+          const double deltaV = w[2] * (sin(w[0] * z + w[1]));
+          dE += w[3] * deltaV;
+          xp *= w[4];
+          yp *= w[4];
+        }
+        break;
+      case OP_ENV:
+        dpc = w[0];
+        g2i = w[1];
+        break;
+      default:
+        break;
+    }
   }
-}
-
-// The kernel level a program needs (the highest of its ops).
-int program_level(const OpProgram& prog) {
-  int l = 0;
-  for (int k = 0; k < prog.nops; k++) l = std::max(l, op_level(prog.ops[k].kind));
-  return l;
 }
 
 constexpr int kPushThreads = 256;
@@ -414,12 +410,21 @@ __device__ __forceinline__ void load6(P a, P b, P c, P d, P e, P f, int64_t i, d
   q[5] = f[i];
 }
 
-// KICK0: the program's first op is a SpaceChargeCalc2p5Drb kick (the usual case: the
-// deferred kick of the previous SC node); it runs outside the op interpreter, with the
-// calculator's values read once, before any store (scalar loads).  Without it the kernel
-// keeps the interpreter's smaller register footprint.
-template <bool EXTREMA, int LEVEL, bool KICK0>
-__global__ __launch_bounds__(kPushThreads) void push_kernel(DeviceBunchView v, OpProgram prog,
+// KICK0: a SpaceChargeCalc2p5Drb kick comes before the program (the usual case: the deferred
+// kick of the previous SC node); it runs outside the op interpreter, with the calculator's
+// values read once, before any store (scalar loads).  Without it the kernel keeps the
+// interpreter's smaller register footprint.  W: the program's words in the kernel arguments; a
+// step's few maps take the small form, since every launch copies its arguments on the host
+// (2.7 KB 0.9 us more than a few hundred bytes).
+struct Kick0 {
+  const SC2DState* st;
+  const double *phi, *zg, *zd;
+  double p4, p5;
+  int32_t nx, ny, nz, pad;
+};
+template <bool EXTREMA, int LEVEL, bool KICK0, int W>
+__global__ __launch_bounds__(kPushThreads) void push_kernel(DeviceBunchView v,
+                                                            ProgramWords<W> prog, Kick0 k0,
                                                             double* __restrict__ partials) {
   double lo[3] = {DBL_MAX, DBL_MAX, DBL_MAX};
   double hi[3] = {-DBL_MAX, -DBL_MAX, -DBL_MAX};
@@ -430,9 +435,8 @@ __global__ __launch_bounds__(kPushThreads) void push_kernel(DeviceBunchView v, O
   const gptr<double> cyp = to_global(v.c[3]);
   const gptr<double> cz = to_global(v.c[4]);
   const gptr<double> cdE = to_global(v.c[5]);
-  const Op& k0 = prog.ops[0];
   SC2DKickParams kp;
-  if constexpr (KICK0) kp = sc2d_kick_params(op_ptr<const SC2DState*>(k0.p[0]));
+  if constexpr (KICK0) kp = sc2d_kick_params(k0.st);
   // The next particle's coordinates are loaded before this one is computed (after its
   // kick's loads), so their latency overlaps the kick and map arithmetic (few waves fit:
   // the map switch needs many VGPRs).
@@ -443,13 +447,11 @@ __global__ __launch_bounds__(kPushThreads) void push_kernel(DeviceBunchView v, O
     double x = q[0], xp = q[1], y = q[2], yp = q[3], z = q[4], dE = q[5];
     SC2DKickLoads L;
     if constexpr (KICK0)
-      sc2p5drb_kick_loads(kp, to_global(op_ptr<const double*>(k0.p[1])), k0.i0, k0.i1,
-                          to_global(op_ptr<const double*>(k0.p[2])),
-                          to_global(op_ptr<const double*>(k0.p[3])), k0.i2, x, y, z, L);
+      sc2p5drb_kick_loads(kp, to_global(k0.phi), k0.nx, k0.ny, to_global(k0.zg),
+                          to_global(k0.zd), k0.nz, x, y, z, L);
     if (i + stride < v.n) load6(cx, cxp, cy, cyp, cz, cdE, i + stride, q);
-    if constexpr (KICK0) sc2p5drb_kick_apply(kp, L, k0.i2, k0.p[4], k0.p[5], x, xp, y, yp, dE);
-    for (int k = KICK0 ? 1 : 0; k < prog.nops; k++)
-      apply_op<LEVEL>(prog.ops[k], x, xp, y, yp, z, dE);
+    if constexpr (KICK0) sc2p5drb_kick_apply(kp, L, k0.nz, k0.p4, k0.p5, x, xp, y, yp, dE);
+    run_program<LEVEL>(prog, x, xp, y, yp, z, dE);
     cx[i] = x;
     cxp[i] = xp;
     cy[i] = y;
@@ -499,7 +501,8 @@ constexpr int kBatchPhiLds = 4096;
 template <bool EXTREMA, int LEVEL>
 __device__ __forceinline__ void push_batch_body(const BatchBunch* __restrict__ bb,
                                                 const BatchItem* __restrict__ items,
-                                                const OpProgram& prog, const BatchKick& kick,
+                                                const ProgramWords<kProgWords>& prog,
+                                                const BatchKick& kick,
                                                 double* __restrict__ partials) {
   const BatchItem it = items[blockIdx.x];
   const BatchBunch& B = bb[it.bunch];
@@ -549,7 +552,7 @@ __device__ __forceinline__ void push_batch_body(const BatchBunch* __restrict__ b
       sc2p5drb_kick_loads(kp, gphi, nx, ny, zg, zd, nz, x, y, z, L);
     if (i + kPushThreads < it.end) load6(cx, cxp, cy, cyp, cz, cdE, i + kPushThreads, q);
     if (kick.active) sc2p5drb_kick_apply(kp, L, nz, kick.p4, kick.p5, x, xp, y, yp, dE);
-    for (int k = 0; k < prog.nops; k++) apply_op<LEVEL>(prog.ops[k], x, xp, y, yp, z, dE);
+    run_program<LEVEL>(prog, x, xp, y, yp, z, dE);
     cx[i] = x;
     cxp[i] = xp;
     cy[i] = y;
@@ -593,13 +596,13 @@ __device__ __forceinline__ void push_batch_body(const BatchBunch* __restrict__ b
 template <bool EXTREMA, int LEVEL>
 __global__ __launch_bounds__(kPushThreads) __attribute__((amdgpu_waves_per_eu(3))) void
 push_batch_kernel(const BatchBunch* __restrict__ bb, const BatchItem* __restrict__ items,
-                  OpProgram prog, BatchKick kick, double* __restrict__ partials) {
+                  ProgramWords<kProgWords> prog, BatchKick kick, double* __restrict__ partials) {
   push_batch_body<EXTREMA, LEVEL>(bb, items, prog, kick, partials);
 }
 template <bool EXTREMA>
 __global__ __launch_bounds__(kPushThreads) void push_batch_kernel_l2(
-    const BatchBunch* __restrict__ bb, const BatchItem* __restrict__ items, OpProgram prog,
-    BatchKick kick, double* __restrict__ partials) {
+    const BatchBunch* __restrict__ bb, const BatchItem* __restrict__ items,
+    ProgramWords<kProgWords> prog, BatchKick kick, double* __restrict__ partials) {
   push_batch_body<EXTREMA, 2>(bb, items, prog, kick, partials);
 }
 
@@ -610,11 +613,12 @@ void launch_push_batch(const BatchBunch* bb, const BatchItem* items, int nitems,
                        int threads, hipStream_t s) {
   OB_REQUIRE(threads == kPushThreads, "batch push: unsupported block size");
   if (nitems == 0) return;
-  const int level = program_level(prog);
+  const int level = prog.level;
+  OB_REQUIRE(level <= 2, "batch push: a space-charge kick inside a map program");
   const size_t lds = kick.active ? sizeof(double) * kBatchPhiLds : 0;
   auto go = [&](auto kernel, double* part) {
-    hipLaunchKernelGGL(kernel, dim3(nitems), dim3(kPushThreads), lds, s, bb, items, prog, kick,
-                       part);
+    hipLaunchKernelGGL(kernel, dim3(nitems), dim3(kPushThreads), lds, s, bb, items,
+                       static_cast<const ProgramWords<kProgWords>&>(prog), kick, part);
   };
   if (prog.want_extrema) {
     OB_REQUIRE(partials != nullptr, "batch push: extrema requested without a buffer");
@@ -626,7 +630,7 @@ void launch_push_batch(const BatchBunch* bb, const BatchItem* items, int nitems,
     else
       go(push_batch_kernel<true, 0>, partials);
   } else {
-    if (prog.nops == 0 && !kick.active) return;
+    if (prog.words == 0 && !kick.active) return;
     ProfScope ps("push_batch");
     if (level == 2)
       go(push_batch_kernel_l2<false>, nullptr);
@@ -645,38 +649,190 @@ int push_grid_blocks(int64_t n) {
   return (int)b;
 }
 
-int launch_push(const DeviceBunchView& v, const OpProgram& prog, double* ext_partials,
-                hipStream_t s) {
+int launch_push(const DeviceBunchView& v, const OpProgram& prog, const Op* kick0,
+                double* ext_partials, hipStream_t s) {
   const int blocks = push_grid_blocks(v.n);
-  const int level = program_level(prog);
-  // levels 0 and 1 take a leading 2.5D kick out of the interpreter
-  const bool kick0 = level < 2 && prog.nops > 0 && prog.ops[0].kind == OP_SC2P5DRB_KICK;
-  auto go = [&](auto kernel, double* part) {
-    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kPushThreads), 0, s, v, prog, part);
+  const bool ext = prog.want_extrema != 0;
+  OB_REQUIRE(!ext || ext_partials != nullptr, "push: extrema requested without a buffer");
+  if (!ext && ((prog.words == 0 && !kick0) || v.n == 0)) return 0;
+  Kick0 k{};
+  if (kick0)
+    k = Kick0{op_ptr<const SC2DState*>(kick0->p[0]), op_ptr<const double*>(kick0->p[1]),
+              op_ptr<const double*>(kick0->p[2]), op_ptr<const double*>(kick0->p[3]),
+              kick0->p[4], kick0->p[5], kick0->i0, kick0->i1, kick0->i2, 0};
+  ProgramWords<kProgSmallWords> small;
+  const bool fits = prog.words <= kProgSmallWords;
+  if (fits) std::memcpy(&small, &prog, offsetof(ProgramWords<kProgSmallWords>, data) +
+                                           sizeof(double) * prog.words);
+  ProfScope ps(ext ? "push_extrema" : "push");
+  auto go = [&](auto ce, auto cl, auto ck) {
+    constexpr bool E = decltype(ce)::value != 0, K = decltype(ck)::value != 0;
+    constexpr int L = decltype(cl)::value;
+    if (fits)
+      hipLaunchKernelGGL((push_kernel<E, L, K, kProgSmallWords>), dim3(blocks),
+                         dim3(kPushThreads), 0, s, v, small, k, ext_partials);
+    else
+      hipLaunchKernelGGL((push_kernel<E, L, K, kProgWords>), dim3(blocks), dim3(kPushThreads), 0,
+                         s, v, static_cast<const ProgramWords<kProgWords>&>(prog), k,
+                         ext_partials);
   };
-  if (prog.want_extrema) {
-    OB_REQUIRE(ext_partials != nullptr, "push: extrema requested without a buffer");
-    ProfScope ps("push_extrema");
-    if (level == 2)
-      go(push_kernel<true, 2, false>, ext_partials);
-    else if (level == 1)
-      kick0 ? go(push_kernel<true, 1, true>, ext_partials)
-            : go(push_kernel<true, 1, false>, ext_partials);
+  auto by_level = [&](auto ce, auto ck) {
+    if (prog.level == 0)
+      go(ce, std::integral_constant<int, 0>{}, ck);
+    else if (prog.level == 1)
+      go(ce, std::integral_constant<int, 1>{}, ck);
+    else if (prog.level == 2)
+      go(ce, std::integral_constant<int, 2>{}, ck);
     else
-      kick0 ? go(push_kernel<true, 0, true>, ext_partials)
-            : go(push_kernel<true, 0, false>, ext_partials);
-  } else {
-    if (prog.nops == 0 || v.n == 0) return 0;
-    ProfScope ps("push");
-    if (level == 2)
-      go(push_kernel<false, 2, false>, nullptr);
-    else if (level == 1)
-      kick0 ? go(push_kernel<false, 1, true>, nullptr) : go(push_kernel<false, 1, false>, nullptr);
-    else
-      kick0 ? go(push_kernel<false, 0, true>, nullptr) : go(push_kernel<false, 0, false>, nullptr);
-  }
+      go(ce, std::integral_constant<int, 3>{}, ck);
+  };
+  using No = std::integral_constant<int, 0>;
+  using Yes = std::integral_constant<int, 1>;
+  if (ext)
+    kick0 ? by_level(Yes{}, Yes{}) : by_level(Yes{}, No{});
+  else
+    kick0 ? by_level(No{}, Yes{}) : by_level(No{}, No{});
   OB_HIP(hipGetLastError());
   return blocks;
+}
+
+namespace {
+double word_of(uint32_t lo, uint32_t hi) {
+  const uint64_t u = (uint64_t)lo | ((uint64_t)hi << 32);
+  double d;
+  std::memcpy(&d, &u, sizeof(d));
+  return d;
+}
+// What an op takes from the program and does to it: the coefficients dpc and g2i it was queued
+// with (0: none), whether it reads dp/p or 1/(1 + dp/p), whether it changes dE.
+struct OpUse {
+  double dpc = 0.0, g2i = 0.0;
+  bool has_dpc = false, has_g2i = false, reads = false, moves_dE = false;
+};
+}  // namespace
+
+size_t program_encode(const Op* ops, size_t count, OpProgram& prog) {
+  prog.words = 0;
+  prog.want_extrema = 0;
+  prog.level = 0;
+  prog.dpc = prog.g2i = 0.0;
+  double cur_dpc = 0.0, cur_g2i = 0.0;
+  bool has_dpc = false, has_g2i = false, env_used = false, fresh = false;
+  auto same = [](double a, double b) { return std::memcmp(&a, &b, sizeof(a)) == 0; };
+  int n = 0;
+  size_t k = 0;
+  for (; k < count; k++) {
+    const Op& o = ops[k];
+    OpUse u;
+    double q[16];
+    int nq = 0;
+    uint32_t ia = 0;
+    auto put = [&](double v) { q[nq++] = v; };
+    auto dpc = [&](double v) { u.dpc = v; u.has_dpc = true; u.reads = true; };
+    auto g2i = [&](double v) { u.g2i = v; u.has_g2i = true; };
+    switch (o.kind) {
+      case OP_DRIFT: put(o.p[0]); g2i(o.p[1]); dpc(o.p[2]); break;
+      case OP_QUAD1:  // m11 = m22 and m33 = m44 are one value each
+        for (int j : {0, 1, 2, 4, 5, 6, 9}) put(o.p[j]);
+        g2i(o.p[8]);
+        dpc(o.p[10]);
+        break;
+      case OP_QUAD2: put(o.p[0]); g2i(o.p[1]); dpc(o.p[2]); break;
+      case OP_QUADFRINGE_IN:
+      case OP_QUADFRINGE_OUT: put(o.p[1]); dpc(o.p[0]); break;
+      case OP_MULTP:
+        put(o.p[0]);
+        ia = (uint32_t)o.i0 | (o.i1 ? 256u : 0u);
+        break;
+      case OP_MULTPFRINGE_IN:
+      case OP_MULTPFRINGE_OUT:
+        put(o.p[1]); put(o.p[2]); dpc(o.p[0]);
+        ia = (uint32_t)o.i0;
+        break;
+      case OP_WRAPBUNCH: put(o.p[0]); break;
+      case OP_ROTATEXY: put(o.p[0]); put(o.p[1]); break;
+      case OP_KICK:
+        for (int j = 0; j < 3; j++) put(o.p[j]);
+        u.moves_dE = o.p[2] != 0.;
+        break;
+      case OP_SC2P5DRB_KICK:
+        for (int j = 0; j < 6; j++) put(o.p[j]);
+        put(word_of((uint32_t)o.i1, (uint32_t)o.i2));
+        ia = (uint32_t)o.i0;
+        u.moves_dE = true;
+        break;
+      case OP_SC3D_KICK:
+        for (int j = 0; j < 12; j++) put(o.p[j]);
+        put(word_of((uint32_t)o.i1, (uint32_t)o.i2));
+        ia = (uint32_t)o.i0;
+        u.moves_dE = true;
+        break;
+      case OP_BEND1:
+        for (int j = 0; j < 10; j++) put(o.p[j]);
+        dpc(o.p[10]);
+        break;
+      case OP_BEND3: put(o.p[0]); g2i(o.p[1]); dpc(o.p[2]); break;
+      case OP_BEND4: put(o.p[0]); dpc(o.p[1]); break;
+      case OP_BENDFRINGE_IN:
+      case OP_BENDFRINGE_OUT: put(o.p[0]); dpc(o.p[1]); break;
+      case OP_WEDGEROTATE:
+        put(o.p[0]); put(o.p[1]);
+        u.dpc = o.p[2];
+        u.has_dpc = true;
+        ia = (uint32_t)o.i0;
+        u.moves_dE = true;
+        break;
+      case OP_WEDGEDRIFT:
+        put(o.p[0]); dpc(o.p[1]); g2i(o.p[2]);
+        ia = (uint32_t)o.i0;
+        break;
+      case OP_WEDGEBEND: {
+        const int nm = (o.i0 >> 1) & 15;
+        OB_REQUIRE(o.i1 < 65536, "wedgebend: more than 131071 steps");
+        put(o.p[0]); put(o.p[1]);
+        put(word_of((uint32_t)o.i2, 0u));
+        for (int l = 0; l < nm; l++) put(o.p[4 + l]);
+        dpc(o.p[2]); g2i(o.p[3]);
+        ia = (uint32_t)(o.i0 & 0xFFFF) | ((uint32_t)o.i1 << 16);
+        break;
+      }
+      case OP_SOLN: put(o.p[0]); put(o.p[1]); g2i(o.p[2]); dpc(o.p[3]); break;
+      case OP_RINGRF:
+        for (int j = 0; j < 5; j++) put(o.p[j]);
+        u.moves_dE = true;
+        break;
+      default: throw Error{"map program: unknown op"};
+    }
+    // the program's coefficients are the first ones; others are set by an OP_ENV before the op
+    const bool env = (u.has_dpc && (has_dpc || env_used) && !same(u.dpc, cur_dpc)) ||
+                     (u.has_g2i && (has_g2i || env_used) && !same(u.g2i, cur_g2i));
+    if (n + (env ? 3 : 0) + 1 + nq > kProgWords) break;
+    if (env) {
+      if (u.has_dpc && !same(u.dpc, cur_dpc)) fresh = false;
+      if (u.has_dpc) cur_dpc = u.dpc;
+      if (u.has_g2i) cur_g2i = u.g2i;
+      prog.data[n++] = word_of((uint32_t)OP_ENV | (3u << 12), 0u);
+      prog.data[n++] = cur_dpc;
+      prog.data[n++] = cur_g2i;
+      env_used = true;
+    } else if (!env_used) {
+      if (u.has_dpc) prog.dpc = cur_dpc = u.dpc;
+      if (u.has_g2i) prog.g2i = cur_g2i = u.g2i;
+    }
+    has_dpc = has_dpc || u.has_dpc;
+    has_g2i = has_g2i || u.has_g2i;
+    uint32_t h = (uint32_t)o.kind | ((uint32_t)(1 + nq) << 12);
+    if (u.reads && !fresh) {
+      h |= kProgRecalc;
+      fresh = true;
+    }
+    if (u.moves_dE) fresh = false;
+    prog.data[n++] = word_of(h, ia);
+    for (int j = 0; j < nq; j++) prog.data[n++] = q[j];
+    prog.level = std::max(prog.level, op_level(o.kind));
+  }
+  prog.words = n;
+  return k;
 }
 
 }  // namespace ob

@@ -13,8 +13,10 @@
 namespace ob {
 
 template <typename T>
-__device__ __forceinline__ T op_ptr(double d) {
-  return reinterpret_cast<T>(__double_as_longlong(d));
+__host__ __device__ __forceinline__ T op_ptr(double d) {
+  uint64_t u;
+  __builtin_memcpy(&u, &d, sizeof(u));
+  return reinterpret_cast<T>(u);
 }
 
 // Every buffer of the library is global memory, but a pointer read from a struct in device
@@ -357,37 +359,43 @@ __device__ __forceinline__ void sc2p5drb_kick_apply(const SC2DKickParams& k,
   dE += ez * long_coef * coeff;
 }
 
-// The whole kick of one particle (the op-program interpreter's form).
-__device__ __forceinline__ void sc2p5drb_kick(const Op& op, double x, double& xp, double y,
-                                              double& yp, double z, double& dE) {
-  const SC2DKickParams k = sc2d_kick_params(op_ptr<const SC2DState*>(op.p[0]));
+// The whole kick of one particle (the op-program interpreter's form): p = the op's p[0..5],
+// then a word with ny (low half) and nz.
+__device__ __forceinline__ void sc2p5drb_kick(const double* p, int nx, double x, double& xp,
+                                              double y, double& yp, double z, double& dE) {
+  const SC2DKickParams k = sc2d_kick_params(op_ptr<const SC2DState*>(p[0]));
+  const uint64_t u = (uint64_t)__double_as_longlong(p[6]);
+  const int ny = (int)(uint32_t)u, nz = (int)(u >> 32);
   SC2DKickLoads L;
-  sc2p5drb_kick_loads(k, to_global(op_ptr<const double*>(op.p[1])), op.i0, op.i1,
-                      to_global(op_ptr<const double*>(op.p[2])),
-                      to_global(op_ptr<const double*>(op.p[3])), op.i2, x, y, z, L);
-  sc2p5drb_kick_apply(k, L, op.i2, op.p[4], op.p[5], x, xp, y, yp, dE);
+  sc2p5drb_kick_loads(k, to_global(op_ptr<const double*>(p[1])), nx, ny,
+                      to_global(op_ptr<const double*>(p[2])),
+                      to_global(op_ptr<const double*>(p[3])), nz, x, y, z, L);
+  sc2p5drb_kick_apply(k, L, nz, p[4], p[5], x, xp, y, yp, dE);
 }
 
 // SpaceChargeCalc3D kick loop body (SpaceChargeCalc3D.cc:132-147).
 // op: p[0]=phi (z-fastest), p[1..6]=xMin,dx,yMin,dy,zMin,dz of the rest-frame phi grid,
 //     p[7]=z_center, p[8]=gamma, p[9]=trans_factor, p[10]=long_factor, p[11]=spacing of
 //     external bunches in the rest frame (0: none); i0=nx, i1=ny, i2=nz | kSC3DWrapBit when
-//     the potential grid wraps periodically in z (Grid3D longWrapping).
+//     the potential grid wraps periodically in z (Grid3D longWrapping).  In the program's
+//     words: p[0..11], then a word with i1 (low half) and i2.
 constexpr int kSC3DWrapBit = 1 << 30;
 constexpr int kSC3DNzMask = kSC3DWrapBit - 1;
-__device__ __forceinline__ void sc3d_kick(const Op& op, double x, double& xp, double y,
+__device__ __forceinline__ void sc3d_kick(const double* p, int nx, double x, double& xp, double y,
                                           double& yp, double z, double& dE) {
-  const double zc = op.p[7], gamma = op.p[8], lambda_cm = op.p[11];
+  const double zc = p[7], gamma = p[8], lambda_cm = p[11];
+  const uint64_t u = (uint64_t)__double_as_longlong(p[12]);
+  const int ny = (int)(uint32_t)u, i2 = (int)(u >> 32);
   double zr = (z - zc) * gamma + zc;
   if (lambda_cm != 0.0) zr = remainder(zr, lambda_cm);  // external bunches (:138-140)
   double ex, ey, ez;
-  const int nz = op.i2 & kSC3DNzMask;
-  const bool wrap = (op.i2 & kSC3DWrapBit) != 0;
-  grid3d_gradient(op_ptr<const double*>(op.p[0]), op.i0, op.i1, nz, op.p[1], op.p[2], op.p[3],
-                  op.p[4], op.p[5], op.p[6], x, y, zr, ex, ey, ez, wrap);
-  xp += -ex * op.p[9];
-  yp += -ey * op.p[9];
-  dE += -ez * op.p[10];
+  const int nz = i2 & kSC3DNzMask;
+  const bool wrap = (i2 & kSC3DWrapBit) != 0;
+  grid3d_gradient(op_ptr<const double*>(p[0]), nx, ny, nz, p[1], p[2], p[3], p[4], p[5], p[6], x,
+                  y, zr, ex, ey, ez, wrap);
+  xp += -ex * p[9];
+  yp += -ey * p[9];
+  dE += -ez * p[10];
 }
 
 // Exclusive block scan of two counters (blockDim.x a multiple of 64, at most 1024).
