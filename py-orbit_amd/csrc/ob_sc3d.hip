@@ -79,47 +79,52 @@ __device__ __forceinline__ double green3d(int i, int j, int k, const GreenGeom& 
   return (ii != 0 || jj != 0 || kk != 0) ? 1. / rTot + externalPhi : externalPhi;
 }
 
-// ---- extrema reduction (one block) -------------------------------------------
+// ---- extrema reduction (one workgroup) ------------------------------------------------
 // Writes the six extrema to out (pinned host memory) and then seq to *seq_out with a
 // system-scope release, all from one thread, so a host that reads *seq_out == seq (with
-// acquire) reads the extrema of this launch.
-__global__ __launch_bounds__(1024) void reduce_extrema(const double* __restrict__ partials,
-                                                       int nblk, double* __restrict__ out,
-                                                       uint64_t* __restrict__ seq_out,
-                                                       uint64_t seq) {
-  __shared__ double red[16][6];
+// acquire) reads the extrema of this launch.  The host waits for it, so its latency counts:
+// four waves with four rows in flight each take 4.4 us for the 196 rows of 50k particles
+// (sixteen waves, whose results one thread walked, 8.4 us).
+constexpr int kExtThreads = 256;
+__global__ __launch_bounds__(kExtThreads) void reduce_extrema(const double* __restrict__ partials,
+                                                              int nblk, double* __restrict__ out,
+                                                              uint64_t* __restrict__ seq_out,
+                                                              uint64_t seq) {
+  __shared__ double red[6][kExtThreads / 64];
   double r[6] = {DBL_MAX, -DBL_MAX, DBL_MAX, -DBL_MAX, DBL_MAX, -DBL_MAX};
-  // four rows per thread and round, their loads in flight together
-  constexpr int U = 4;
-  for (int b0 = threadIdx.x; b0 < nblk; b0 += U * blockDim.x) {
+  constexpr int U = 4;  // rows in flight; a row past the last repeats the first
+  for (int b = threadIdx.x; b < nblk; b += U * kExtThreads) {
     double v[U][6];
 #pragma unroll
-    for (int u = 0; u < U; u++) {
-      const int b = b0 + u * (int)blockDim.x;
+    for (int u = 0; u < U; u++)
 #pragma unroll
-      for (int k = 0; k < 6; k++) v[u][k] = b < nblk ? partials[b * 6 + k] : r[k];
-    }
+      for (int k = 0; k < 6; k++)
+        v[u][k] = partials[(b + u * kExtThreads < nblk ? b + u * kExtThreads : b) * 6 + k];
 #pragma unroll
     for (int u = 0; u < U; u++)
 #pragma unroll
       for (int k = 0; k < 6; k++) r[k] = (k & 1) ? fmax(r[k], v[u][k]) : fmin(r[k], v[u][k]);
   }
-  for (int k = 0; k < 6; k++)
-    for (int o = 32; o > 0; o >>= 1) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+    for (int k = 0; k < 6; k++) {
       const double v = __shfl_xor(r[k], o, 64);
       r[k] = (k & 1) ? fmax(r[k], v) : fmin(r[k], v);
     }
   if ((threadIdx.x & 63) == 0)
-    for (int k = 0; k < 6; k++) red[threadIdx.x >> 6][k] = r[k];
+#pragma unroll
+    for (int k = 0; k < 6; k++) red[k][threadIdx.x >> 6] = r[k];
   __syncthreads();
   if (threadIdx.x == 0) {
-    double acc[6];
+#pragma unroll
     for (int k = 0; k < 6; k++) {
-      acc[k] = red[0][k];
-      for (int w = 1; w < (int)(blockDim.x >> 6); w++)
-        acc[k] = (k & 1) ? fmax(acc[k], red[w][k]) : fmin(acc[k], red[w][k]);
+      double acc = red[k][0];
+#pragma unroll
+      for (int w = 1; w < kExtThreads / 64; w++)
+        acc = (k & 1) ? fmax(acc, red[k][w]) : fmin(acc, red[k][w]);
+      out[k] = acc;
     }
-    for (int k = 0; k < 6; k++) out[k] = acc[k];
     __hip_atomic_store(seq_out, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
@@ -152,7 +157,7 @@ const double* extrema_to_host(ExtremaLink& e, const double* partials, int nblk, 
   uint64_t* seq_host = reinterpret_cast<uint64_t*>(e.host + 6);
   {
     ProfScope ps_("reduce_extrema");
-    hipLaunchKernelGGL(reduce_extrema, dim3(1), dim3(1024), 0, s, partials, nblk, e.dev,
+    hipLaunchKernelGGL(reduce_extrema, dim3(1), dim3(kExtThreads), 0, s, partials, nblk, e.dev,
                        reinterpret_cast<uint64_t*>(e.dev + 6), want);
   }
   OB_HIP(hipGetLastError());
@@ -1003,11 +1008,6 @@ OB_API int ob_sc3d_track(ob_sc3d* c, ob_bunch* b, double length) {
     g.zMin = center - width; g.zMax = center + width; g.dz = (g.zMax - g.zMin) / c->nz;
   }
   // deposit in lab z
-  const int64_t ng = (int64_t)c->nx * c->ny * c->nz;
-  {
-    ob::ProfScope ps_("fill_zero");
-    hipLaunchKernelGGL(ob::fill_zero, dim3(1024), dim3(256), 0, s, c->rho, ng);
-  }
   const ob::TileGeom tg = ob::make_tile_geom(g.nx, g.ny, g.nz, g.xMin, g.xMax, g.yMin, g.yMax,
                                              g.zMin, g.zMax, g.dx, g.dy, g.dz, c->lds_budget);
   const bool tiled = c->tiled && tg.T > 0 && !wrapped;
@@ -1018,6 +1018,11 @@ OB_API int ob_sc3d_track(ob_sc3d* c, ob_bunch* b, double length) {
     int dblk = (int)((n + ob::kThreads - 1) / ob::kThreads);
     const int cap = 16 * ob::device_cu_count();
     if (dblk > cap) dblk = cap;
+    {
+      ob::ProfScope ps_("fill_zero");
+      hipLaunchKernelGGL(ob::fill_zero, dim3(1024), dim3(256), 0, s, c->rho,
+                         (int64_t)c->nx * c->ny * c->nz);
+    }
     ob::ProfScope ps_("deposit3d");
     hipLaunchKernelGGL(ob::deposit3d, dim3(dblk), dim3(ob::kThreads), 0, s, v, g, sy.macrosize,
                        lambda, c->rho);
@@ -1319,11 +1324,6 @@ void slice_track(ob_slice2d* c, ob_bunch* b, double length, ob_boundary2d* bnd) 
   c->g[0] = g.xMin; c->g[1] = g.xMax; c->g[2] = g.yMin; c->g[3] = g.yMax;
   c->g[4] = g.zMin; c->g[5] = g.zMax; c->g[6] = g.dx; c->g[7] = g.dy; c->g[8] = g.dz;
   // Grid3D::binBunch (Grid3D.cc:281-305)
-  const int64_t ng = (int64_t)c->nx * c->ny * c->nz;
-  {
-    ProfScope ps_("fill_zero");
-    hipLaunchKernelGGL(fill_zero, dim3(1024), dim3(256), 0, s, c->rho, ng);
-  }
   const TileGeom tg = make_tile_geom(g.nx, g.ny, g.nz, g.xMin, g.xMax, g.yMin, g.yMax, g.zMin,
                                      g.zMax, g.dx, g.dy, g.dz, c->lds_budget);
   const bool tiled = tg.T > 0;
@@ -1336,6 +1336,11 @@ void slice_track(ob_slice2d* c, ob_bunch* b, double length, ob_boundary2d* bnd) 
     int dblk = (int)((n + kThreads - 1) / kThreads);
     const int cap = 16 * device_cu_count();
     if (dblk > cap) dblk = cap;
+    {
+      ProfScope ps_("fill_zero");
+      hipLaunchKernelGGL(fill_zero, dim3(1024), dim3(256), 0, s, c->rho,
+                         (int64_t)c->nx * c->ny * c->nz);
+    }
     ProfScope ps_("deposit3d");
     hipLaunchKernelGGL(deposit3d, dim3(dblk), dim3(kThreads), 0, s, v, g, sy.macrosize, 0.0,
                        c->rho);

@@ -91,15 +91,30 @@ struct TileBox {
   }
 };
 
+// Workgroups past hist_blocks clear rho, which the deposit needs: the histogram waits for
+// particle loads and LDS, so the stores cost next to nothing beside it (a launch of their own
+// took 3.3 us at 64 x 64 x 64 nodes and 12.5 us at 128 x 128 x 256, and the gap before it).
 __global__ __launch_bounds__(1024) void tile_hist(const double* __restrict__ cur, int64_t cap,
                                                       int64_t n, TileGeom g,
                                                       uint32_t* __restrict__ key,
-                                                      uint32_t* __restrict__ counts) {
+                                                      uint32_t* __restrict__ counts,
+                                                      uint32_t* __restrict__ cursor,
+                                                      int hist_blocks,
+                                                      double* __restrict__ rho) {
   extern __shared__ uint32_t lh[];
+  if ((int)blockIdx.x >= hist_blocks) {
+    const int64_t ng = (int64_t)g.nx * g.ny * g.nz;
+    const int64_t step = (int64_t)(gridDim.x - hist_blocks) * 1024;
+    for (int64_t c = (int64_t)(blockIdx.x - hist_blocks) * 1024 + threadIdx.x; c < ng; c += step)
+      rho[c] = 0.0;
+    return;
+  }
   const int nb = g.ntiles + 1;
+  if (cursor && blockIdx.x == 0)  // (scan in the scatter: its positions start at 0)
+    for (int t = threadIdx.x; t < nb; t += blockDim.x) cursor[t] = 0;
   for (int t = threadIdx.x; t < nb; t += blockDim.x) lh[t] = 0;
   __syncthreads();
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  const int64_t stride = (int64_t)hist_blocks * blockDim.x;
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   // four particles per round: their 12 loads are in flight together
   constexpr int U = 4;
@@ -196,15 +211,58 @@ __global__ __launch_bounds__(1024) void tile_scan(uint32_t* __restrict__ counts,
   }
 }
 
+// SCAN: few tiles (kScanTiles): every workgroup scans the counts itself and workgroup 0 writes
+// the offsets and work items; cursor then counts from 0 in each tile and the deposit clears
+// the counts.  Otherwise tile_scan has written offsets and cursor = offsets.  At 840 tiles
+// (96 x 80 x 100 nodes, 700k particles) the scatter goes from 21.3 to 23.4 us and the scan's
+// 5.0 us and the gap before it go; at 8192 tiles it would go from 153 to 267 us against the
+// scan's 26, its LDS too large for the workgroups a CU needs.
+constexpr int kScanTiles = 1024;
+struct ScatterScan {
+  const uint32_t* counts;
+  uint32_t* offsets;
+  int4* items;
+  uint32_t* nitems;
+};
+template <bool SCAN>
 __global__ __launch_bounds__(kThreads) void tile_scatter(
     const double* __restrict__ cur, double* __restrict__ alt, int64_t cap, int64_t n,
     const uint32_t* __restrict__ key, int ntiles, uint32_t* __restrict__ cursor,
     const int32_t* __restrict__ perm, int32_t* __restrict__ perm_alt,
-    const double* __restrict__ msize, double* __restrict__ msize_alt, int64_t per_block) {
+    const double* __restrict__ msize, double* __restrict__ msize_alt, int64_t per_block,
+    ScatterScan sc) {
   extern __shared__ uint32_t sh[];
   uint32_t* lc = sh;               // local counts, then running destinations
   const int nb = ntiles + 1;
+  uint32_t* loff = sh + nb;        // SCAN: tile offsets
   for (int t = threadIdx.x; t < nb; t += blockDim.x) lc[t] = 0;
+  if constexpr (SCAN) {
+    const int per = (nb + kThreads - 1) / kThreads;
+    const int a = min(nb, (int)threadIdx.x * per), e = min(nb, a + per);
+    uint32_t off = 0, item = 0;
+    for (int t = a; t < e; t++) {
+      const uint32_t k = sc.counts[t];
+      loff[t] = k;
+      off += k;
+      if (t < ntiles) item += (k + kChunk - 1) / kChunk;
+    }
+    uint32_t total, total_items;
+    block_scan2(off, item, total, total_items);
+    const bool writer = blockIdx.x == 0;
+    for (int t = a; t < e; t++) {  // each thread rewrites only the entries it alone has read
+      const uint32_t k = loff[t];
+      loff[t] = off;
+      if (writer) {
+        sc.offsets[t] = off;
+        if (t < ntiles)
+          for (uint32_t b0 = 0; b0 < k; b0 += kChunk)
+            sc.items[item++] =
+                make_int4(t, (int)(off + b0), (int)(off + min(k, b0 + (uint32_t)kChunk)), 0);
+      }
+      off += k;
+    }
+    if (writer && threadIdx.x == 0) *sc.nitems = total_items;
+  }
   __syncthreads();
   const int64_t lo = (int64_t)blockIdx.x * per_block;
   const int64_t hi = min(n, lo + per_block);
@@ -212,7 +270,7 @@ __global__ __launch_bounds__(kThreads) void tile_scatter(
   __syncthreads();
   for (int t = threadIdx.x; t < nb; t += blockDim.x) {
     const uint32_t c = lc[t];
-    lc[t] = c ? atomicAdd(&cursor[t], c) : 0u;
+    lc[t] = c ? (SCAN ? loff[t] : 0u) + atomicAdd(&cursor[t], c) : 0u;
   }
   __syncthreads();
   // U particles per thread and round: all their loads are issued before any store
@@ -303,7 +361,10 @@ __global__ __launch_bounds__(kThreads) void tile_deposit(const double* __restric
                                                          double macrosize, TileGeom g,
                                                          const int4* __restrict__ items,
                                                          const uint32_t* __restrict__ nitems,
-                                                         double* __restrict__ rho) {
+                                                         double* __restrict__ rho,
+                                                         uint32_t* __restrict__ counts) {
+  if (counts && blockIdx.x == 0)  // (scan in the scatter: zero for the next step)
+    for (int t = threadIdx.x; t <= g.ntiles; t += blockDim.x) counts[t] = 0;
   if (blockIdx.x >= *nitems) return;
   extern __shared__ double acc[];
   __shared__ uint32_t rcount[kBankWords], roff[kBankWords], rmax;
@@ -629,7 +690,7 @@ void sort_and_deposit_3d(ob_bunch* b, const TileGeom& g, double macrosize, doubl
                                hipFuncAttributeMaxDynamicSharedMemorySize, 159 * 1024));
     OB_HIP(hipFuncSetAttribute((const void*)tile_hist,
                                hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-    OB_HIP(hipFuncSetAttribute((const void*)tile_scatter,
+    OB_HIP(hipFuncSetAttribute((const void*)tile_scatter<false>,
                                hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
     OB_HIP(hipFuncSetAttribute((const void*)tile_scan,
                                hipFuncAttributeMaxDynamicSharedMemorySize, 136 * 1024));
@@ -648,16 +709,20 @@ void sort_and_deposit_3d(ob_bunch* b, const TileGeom& g, double macrosize, doubl
   hipStream_t s = stream();
   SortBuffers sb = bunch_sort_begin(b);
   const size_t hl = sizeof(uint32_t) * (g.ntiles + 1);
+  const bool scan = n > 0 && g.ntiles <= kScanTiles;  // (no scatter without particles)
   // one workgroup of 1024 threads per CU: each merges up to ntiles + 1 counters into the
   // global counts, so fewer, larger workgroups mean fewer global atomics (measured 38 -> 32 us)
   int hb = (int)std::min<int64_t>((n + 1023) / 1024, device_cu_count());
   if (hb < 1) hb = 1;
   {
     ProfScope ps("tile_hist");
-    hipLaunchKernelGGL(tile_hist, dim3(hb), dim3(1024), hl, s, sb.cur, sb.cap, n, g, w.key,
-                       w.counts);
+    // (four nodes per thread, at most one clearing workgroup per CU)
+    const int64_t ng = (int64_t)g.nx * g.ny * g.nz;
+    const int cb = (int)std::min<int64_t>((ng + 4095) / 4096, device_cu_count());
+    hipLaunchKernelGGL(tile_hist, dim3(hb + cb), dim3(1024), hl, s, sb.cur, sb.cap, n, g, w.key,
+                       w.counts, scan ? w.cursor : nullptr, hb, rho);
   }
-  {
+  if (!scan) {
     ProfScope ps("tile_scan");
     hipLaunchKernelGGL(tile_scan, dim3(1), dim3(1024), sizeof(uint32_t) * 2 * (g.ntiles + 2), s,
                        w.counts, g.ntiles, w.offsets,
@@ -668,9 +733,15 @@ void sort_and_deposit_3d(ob_bunch* b, const TileGeom& g, double macrosize, doubl
   const int sb_blocks = (int)((n + per - 1) / per);
   if (n) {
     ProfScope ps("tile_scatter");
-    hipLaunchKernelGGL(tile_scatter, dim3(sb_blocks), dim3(kThreads), hl, s, sb.cur, sb.alt,
-                       sb.cap, n, w.key, g.ntiles, w.cursor, sb.perm, sb.perm_alt, sb.msize,
-                       sb.msize_alt, per);
+    const ScatterScan sc{w.counts, w.offsets, w.items, w.nitems};
+    if (scan)
+      hipLaunchKernelGGL(tile_scatter<true>, dim3(sb_blocks), dim3(kThreads), 2 * hl, s, sb.cur,
+                         sb.alt, sb.cap, n, w.key, g.ntiles, w.cursor, sb.perm, sb.perm_alt,
+                         sb.msize, sb.msize_alt, per, sc);
+    else
+      hipLaunchKernelGGL(tile_scatter<false>, dim3(sb_blocks), dim3(kThreads), hl, s, sb.cur,
+                         sb.alt, sb.cap, n, w.key, g.ntiles, w.cursor, sb.perm, sb.perm_alt,
+                         sb.msize, sb.msize_alt, per, sc);
   }
   OB_HIP(hipGetLastError());
   bunch_sort_commit(b);
@@ -681,7 +752,7 @@ void sort_and_deposit_3d(ob_bunch* b, const TileGeom& g, double macrosize, doubl
     hipLaunchKernelGGL(tile_deposit, dim3((unsigned)max_items), dim3(kThreads),
                        tile_deposit_lds_bytes(g),
                        s, v.c[0], (int64_t)(v.c[1] - v.c[0]), v.msize, macrosize, g, w.items,
-                       w.nitems, rho);
+                       w.nitems, rho, scan ? w.counts : nullptr);
   }
   OB_HIP(hipGetLastError());
 }

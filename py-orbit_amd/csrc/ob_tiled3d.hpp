@@ -33,7 +33,7 @@ struct TileWork {
 };
 
 // Sort the bunch by tile (device order only) and deposit its charge into rho, a
-// z-fastest [nx][ny][nz] array that must already be zero.  The work items stay valid for
+// z-fastest [nx][ny][nz] array (cleared first).  The work items stay valid for
 // tile_kick_3d until the particles move.
 void sort_and_deposit_3d(ob_bunch* b, const TileGeom& g, double macrosize, double* rho,
                          TileWork& w);

@@ -1,0 +1,58 @@
+"""The tile sort of the 3D calculators where its path changes: tile counts around the limit
+of the scan inside the scatter, bunches around one workgroup's and one work item's particles,
+one z node, and the way back to user order, with and without macrosizes.  The tiled deposit
+against the particle-order one of the same calculator: the same terms in another order, so rho
+agrees to n eps / 2 of the largest node at worst and to sqrt(n) eps in the mean."""
+import numpy as np
+import pytest
+
+from test_gpu_sc import _bunches
+
+pytestmark = pytest.mark.gpu
+
+
+def _coords(n, seed):
+    r = np.random.default_rng(seed)
+    return r.standard_normal((6, n)) * np.array([3e-3, 1e-3, 2.5e-3, 1e-3, 0.3, 1e-3])[:, None]
+
+
+# 8 x 8 x 16 boxes: 64 x 64 x 256 nodes are 1024 tiles (scan in the scatter), 64 x 64 x 257
+# and 72 x 64 x 256 more (scan launch)
+GRIDS = [(64, 64, 256), (64, 64, 257), (72, 64, 256), (3, 3, 1), (9, 17, 2), (33, 8, 40)]
+
+
+@pytest.mark.parametrize("weights", [False, True])
+@pytest.mark.parametrize("n", [2, 511, 513, 1025, 40_011])
+@pytest.mark.parametrize("grid", GRIDS)
+def test_sorted_deposit_and_order(grid, n, weights):
+    import spacecharge
+    c = _coords(n, n)
+    b, _ = _bunches(c)
+    if weights:
+        b.setMacroSizes(np.random.default_rng(2).uniform(0.5e8, 1.5e8, n))
+    calc, plain = spacecharge.SpaceChargeCalc3D(*grid), spacecharge.SpaceChargeCalc3D(*grid)
+    plain.setDepositMode(False)
+    for _ in range(3):  # (counters and rho are left clear for the next step)
+        calc.trackBunch(b, 0.0)
+    # a kick of length 0 leaves the bunch as it was, back in user order
+    assert np.array_equal(b.getCoordinates(), c)
+    if weights:
+        assert np.array_equal(b.getMacroSizes(),
+                              np.random.default_rng(2).uniform(0.5e8, 1.5e8, n))
+    plain.trackBunch(b, 0.0)
+    rho, ref = calc.getRhoGrid().array(), plain.getRhoGrid().array()
+    assert np.abs(rho - ref).max() <= n * 1.2e-16 * np.abs(ref).max() + 4e-16 * np.abs(ref).max()
+    assert np.isclose(rho.sum(), ref.sum(), rtol=1e-13)
+
+
+def test_rho_is_kept_when_a_step_is_refused():
+    import spacecharge
+    c = _coords(500, 1)
+    b, _ = _bunches(c)
+    calc = spacecharge.SpaceChargeCalc3D(16, 16, 16)
+    calc.trackBunch(b, 0.0)
+    rho = calc.getRhoGrid().array().copy()
+    flat, _ = _bunches(c * np.array([0, 1, 1, 1, 1, 1.])[:, None])
+    with pytest.raises(Exception, match="zero extent"):
+        calc.trackBunch(flat, 0.0)
+    assert np.array_equal(calc.getRhoGrid().array(), rho)
