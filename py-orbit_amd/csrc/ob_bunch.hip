@@ -12,6 +12,7 @@
 #include <mutex>
 
 #include "ob_internal.hpp"
+#include "ob_tiled3d.hpp"
 
 namespace ob {
 
@@ -170,6 +171,8 @@ struct ob_bunch {
   bool has_msize = false;
   bool host_valid = true, dev_valid = true;
 
+  ob::TileKick tile_kick;      // waits before the queue's ops if has_tile_kick
+  bool has_tile_kick = false;
   std::vector<ob::Op> queue;
   ob_batch* owner = nullptr;  // batch applying this bunch's maps, if any
   ob::DiagWork diag;
@@ -412,23 +415,25 @@ void bunch_set_owner(ob_bunch* b, ob_batch* owner) { b->owner = owner; }
 
 std::vector<ob_bunch*> g_live_bunches;
 
-// A calculator is about to free its buffers: apply every queued space-charge kick that
+// A calculator is about to write or free its buffers: apply every waiting space-charge kick that
 // reads them (the kick belongs to a trackBunch call that has already happened).
 void flush_kicks_reading(const void* state) {
+  const double want = ptr_bits(state);
   for (ob_bunch* b : g_live_bunches) {
-    for (const Op& op : b->queue) {
-      const double want = ptr_bits(state);
-      if ((op.kind == OP_SC2P5DRB_KICK || op.kind == OP_SC3D_KICK) &&
-          std::memcmp(&op.p[0], &want, sizeof(double)) == 0) {
-        try {
-          bunch_flush(b, nullptr);
-        } catch (const Error&) {
-          // The kick cannot be applied; it must not outlive the buffers it reads.
-          b->queue.clear();
-          throw;
-        }
-        break;
-      }
+    bool reads = b->has_tile_kick && b->tile_kick.k.phi == state;
+    for (size_t j = 0; j < b->queue.size() && !reads; j++) {
+      const Op& op = b->queue[j];
+      reads = (op.kind == OP_SC2P5DRB_KICK || op.kind == OP_SC3D_KICK) &&
+              std::memcmp(&op.p[0], &want, sizeof(double)) == 0;
+    }
+    if (!reads) continue;
+    try {
+      bunch_flush(b, nullptr);
+    } catch (const Error&) {
+      // The kick cannot be applied; it must not outlive the buffers it reads.
+      b->has_tile_kick = false;
+      b->queue.clear();
+      throw;
     }
   }
 }
@@ -438,8 +443,11 @@ SyncInfo bunch_sync(ob_bunch* b) {
 }
 
 namespace {
-// Launch the queue's front as one program: a leading 2.5D kick (the usual case: the previous
-// SC node's, which runs outside the program) and as many ops as fit.  Extrema only if the
+// Launch the queue's front as one program: a waiting tile kick or a leading 2.5D kick (the usual
+// case: the previous SC node's, which runs outside the program) and as many ops as fit.  A tile
+// kick takes the program along if that is short and of level 0 or 1 (drifts to dipoles: the
+// maps between two SC nodes); the registers of the higher levels would cost the kick its
+// third wave per SIMD, so then the kick goes first by itself.  Extrema only if the
 // queue ends there.  Returns the ops taken; *blocks = workgroups of the launch.
 size_t launch_front(ob_bunch* b, const DeviceBunchView& v, size_t pos, double* ext_partials,
                     int* blocks) {
@@ -449,6 +457,17 @@ size_t launch_front(ob_bunch* b, const DeviceBunchView& v, size_t pos, double* e
   OpProgram prog;
   pos += program_encode(b->queue.data() + pos, b->queue.size() - pos, prog);
   prog.want_extrema = (pos >= b->queue.size() && ext_partials) ? 1 : 0;
+  if (b->has_tile_kick) {
+    b->has_tile_kick = false;
+    if (!kick0 && prog.level <= 1 && prog.words <= kProgSmallWords) {
+      *blocks = launch_tile_push(v, b->tile_kick, prog,
+                                 prog.want_extrema ? ext_partials : nullptr, stream());
+      return pos - first;
+    }
+    OpProgram none;
+    program_encode(nullptr, 0, none);
+    launch_tile_push(v, b->tile_kick, none, nullptr, stream());
+  }
   *blocks = launch_push(v, prog, kick0, prog.want_extrema ? ext_partials : nullptr, stream());
   return pos - first;
 }
@@ -461,7 +480,7 @@ int bunch_flush(ob_bunch* b, double* ext_partials) {
     batch_flush_owner(b->owner);
     return 0;
   }
-  if (b->queue.empty() && ext_partials == nullptr) return 0;
+  if (b->queue.empty() && !b->has_tile_kick && ext_partials == nullptr) return 0;
   DeviceBunchView v = bunch_device_view(b);
   size_t pos = 0;
   int blocks = 0;
@@ -471,6 +490,13 @@ int bunch_flush(ob_bunch* b, double* ext_partials) {
   b->queue.clear();
   b->host_valid = false;
   return blocks;
+}
+
+void bunch_queue_tile_kick(ob_bunch* b, const TileKick& t) {
+  OB_REQUIRE(b->queue.empty() && !b->has_tile_kick, "tile kick: the bunch has waiting maps");
+  b->tile_kick = t;
+  b->has_tile_kick = true;
+  b->host_valid = false;
 }
 
 void bunch_queue(ob_bunch* b, const Op& op) {
@@ -665,6 +691,7 @@ OB_API int ob_bunch_set_coords(ob_bunch* b, int64_t n, const double* x, const do
                                const double* dE) {
   OB_TRY OB_CHECK_B(b);
   OB_REQUIRE(n >= 0, "negative particle count");
+  b->has_tile_kick = false;
   b->queue.clear();
   const double* src[6] = {x, xp, y, yp, z, dE};
   for (int k = 0; k < 6; k++) OB_REQUIRE(n == 0 || src[k] != nullptr, "null coordinate array");

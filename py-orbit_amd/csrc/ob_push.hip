@@ -17,6 +17,8 @@
 
 #include "ob_internal.hpp"
 #include "ob_sc_device.hpp"
+#include "ob_tiled3d.hpp"
+#include "ob_tiled3d_device.hpp"
 
 namespace ob {
 
@@ -400,6 +402,28 @@ __device__ __forceinline__ double wave_max(double v) {
   return v;
 }
 
+// Extrema of a workgroup's x, y, z (each thread's in lo, hi) to its row of partials.
+__device__ __forceinline__ void block_extrema(const double lo[3], const double hi[3],
+                                              double* __restrict__ partials) {
+  __shared__ double red[kPushThreads / 64][6];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  double r[6];
+  for (int k = 0; k < 3; k++) {
+    r[2 * k] = wave_min(lo[k]);
+    r[2 * k + 1] = wave_max(hi[k]);
+  }
+  if (lane == 0)
+    for (int k = 0; k < 6; k++) red[w][k] = r[k];
+  __syncthreads();
+  if (threadIdx.x < 6) {
+    const int k = threadIdx.x;
+    double acc = red[0][k];
+    for (int j = 1; j < kPushThreads / 64; j++)
+      acc = (k & 1) ? fmax(acc, red[j][k]) : fmin(acc, red[j][k]);
+    partials[(int64_t)blockIdx.x * 6 + k] = acc;
+  }
+}
+
 template <typename P>
 __device__ __forceinline__ void load6(P a, P b, P c, P d, P e, P f, int64_t i, double q[6]) {
   q[0] = a[i];
@@ -467,25 +491,99 @@ __global__ __launch_bounds__(kPushThreads) void push_kernel(DeviceBunchView v,
       hi[2] = fmax(hi[2], z);
     }
   }
-  if (EXTREMA) {
-    __shared__ double red[kPushThreads / 64][6];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    double r[6];
-    for (int k = 0; k < 3; k++) {
-      r[2 * k] = wave_min(lo[k]);
-      r[2 * k + 1] = wave_max(hi[k]);
+  if (EXTREMA) block_extrema(lo, hi, partials);
+}
+
+// The kick of a tile-sorted bunch (ob_tiled3d.hip) and the program of the maps after it, one pass
+// over the particles.  Workgroups walk the work items: a tile's block of phi goes to LDS, its
+// particles are kicked from it; item nitems is the particles outside the grid (last in the
+// sorted order, from offsets[ntiles]), kicked from the whole grid like the reference.  MAPS:
+// false without a program and extrema (three of the six coordinates are written).
+// As two launches the kick and the push moved 72 + 96 bytes per particle; here 96.
+// At least 3 waves per SIMD: the kick with the next particle's prefetch takes 157 VGPRs
+// without spills.  Bounded to 4 waves (128 VGPRs) the prefetch spills and the kick ran
+// 133 us against 113; without the prefetch, 119.
+template <bool BND, bool EXTREMA, int LEVEL, bool MAPS>
+__global__ __launch_bounds__(kTileThreads, 3) void tile_push(
+    double* __restrict__ cur, int64_t cap, TileKick t, ProgramWords<kProgSmallWords> prog,
+    double* __restrict__ partials) {
+  const TileGeom& g = t.g;
+  const Kick3D& k = t.k;
+  const uint32_t ni = *t.nitems;
+  extern __shared__ double sphi[];
+  double lo[3] = {DBL_MAX, DBL_MAX, DBL_MAX};
+  double hi[3] = {-DBL_MAX, -DBL_MAX, -DBL_MAX};
+  auto finish = [&](int64_t i, double x, double xp, double y, double yp, double z, double dE) {
+    if constexpr (MAPS) {
+      run_program<LEVEL>(prog, x, xp, y, yp, z, dE);
+      cur[i] = x;
+      cur[2 * cap + i] = y;
+      cur[4 * cap + i] = z;
     }
-    if (lane == 0)
-      for (int k = 0; k < 6; k++) red[w][k] = r[k];
+    cur[cap + i] = xp;
+    cur[3 * cap + i] = yp;
+    cur[5 * cap + i] = dE;
+    if constexpr (EXTREMA) {
+      lo[0] = fmin(lo[0], x);
+      hi[0] = fmax(hi[0], x);
+      lo[1] = fmin(lo[1], y);
+      hi[1] = fmax(hi[1], y);
+      lo[2] = fmin(lo[2], z);
+      hi[2] = fmax(hi[2], z);
+    }
+  };
+  const int64_t gsx = (int64_t)g.ny * g.nz;
+  for (uint32_t item = blockIdx.x; item <= ni; item += gridDim.x) {
+    const bool rest = item == ni;
+    const int4 it = rest ? make_int4(0, (int)t.offsets[g.ntiles], (int)t.n, 0) : t.items[item];
+    TileBox box(g, it.x);
+    if (rest) box.x0 = 1 << 30;  // no block: holds no node
+    const int cells = box.cells();
+    // The first particle's coordinates are requested with the block of phi, and all of a
+    // thread's block loads are issued before any is stored (a masked lane loads phi[0] and
+    // stores 0), so these latencies overlap instead of adding up.
+    const int i0 = it.y + (int)threadIdx.x;
+    const int ia = i0 < it.z ? i0 : 0;
+    double q[6] = {cur[ia], cur[2 * cap + ia], cur[4 * cap + ia],
+                   cur[cap + ia], cur[3 * cap + ia], cur[5 * cap + ia]};
+    constexpr int KB = 8;  // cells <= KB * kTileThreads for blocks of up to 16 KiB
+    double bv[KB];
+    uint32_t inmask = 0;
+    CellWalk w((int)threadIdx.x, box.W, box.Wz);
+#pragma unroll
+    for (int u = 0; u < KB; u++, w.next()) {
+      const int c = (int)threadIdx.x + u * kTileThreads;
+      const int gx = box.x0 + w.lx, gy = box.y0 + w.ly, gz = box.z0 + w.lz;
+      const bool in = c < cells && gx >= 0 && gx < g.nx && gy >= 0 && gy < g.ny && gz >= 0 &&
+                      gz < g.nz;
+      bv[u] = k.phi[in ? gx * gsx + (int64_t)gy * g.nz + gz : 0];
+      inmask |= (in ? 1u : 0u) << u;
+    }
+    if (item != blockIdx.x) __syncthreads();  // the last item's block is no longer read
+#pragma unroll
+    for (int u = 0; u < KB; u++) {
+      const int c = (int)threadIdx.x + u * kTileThreads;
+      if (c < cells) sphi[c] = ((inmask >> u) & 1u) ? bv[u] : 0.0;
+    }
+    for (int c = (int)threadIdx.x + KB * kTileThreads; c < cells; c += kTileThreads, w.next()) {
+      // larger blocks: the walk continues from cell threadIdx.x + KB * kTileThreads
+      const int gx = box.x0 + w.lx, gy = box.y0 + w.ly, gz = box.z0 + w.lz;
+      const bool in = gx >= 0 && gx < g.nx && gy >= 0 && gy < g.ny && gz >= 0 && gz < g.nz;
+      sphi[c] = in ? k.phi[gx * gsx + (int64_t)gy * g.nz + gz] : 0.0;
+    }
     __syncthreads();
-    if (threadIdx.x < 6) {
-      const int k = threadIdx.x;
-      double acc = red[0][k];
-      for (int j = 1; j < kPushThreads / 64; j++)
-        acc = (k & 1) ? fmax(acc, red[j][k]) : fmin(acc, red[j][k]);
-      partials[(int64_t)blockIdx.x * 6 + k] = acc;
+    // The next particle's coordinates are loaded before this one is kicked.
+    for (int i = i0; i < it.z; i += kTileThreads) {
+      const int in = i + kTileThreads < it.z ? i + kTileThreads : i;
+      const double nq[6] = {cur[in], cur[2 * cap + in], cur[4 * cap + in],
+                            cur[cap + in], cur[3 * cap + in], cur[5 * cap + in]};
+      tile_kick_particle<BND>(g, k, sphi, box, q[0], q[1], q[2], q[3], q[4], q[5]);
+      finish(i, q[0], q[3], q[1], q[4], q[2], q[5]);
+#pragma unroll
+      for (int c = 0; c < 6; c++) q[c] = nq[c];
     }
   }
+  if constexpr (EXTREMA) block_extrema(lo, hi, partials);
 }
 
 // Potentials of at most this many nodes (64 x 64) are copied into LDS by each workgroup
@@ -568,25 +666,7 @@ __device__ __forceinline__ void push_batch_body(const BatchBunch* __restrict__ b
       hi[2] = fmax(hi[2], z);
     }
   }
-  if (EXTREMA) {
-    __shared__ double red[kPushThreads / 64][6];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    double r[6];
-    for (int k = 0; k < 3; k++) {
-      r[2 * k] = wave_min(lo[k]);
-      r[2 * k + 1] = wave_max(hi[k]);
-    }
-    if (lane == 0)
-      for (int k = 0; k < 6; k++) red[w][k] = r[k];
-    __syncthreads();
-    if (threadIdx.x < 6) {
-      const int k = threadIdx.x;
-      double acc = red[0][k];
-      for (int j = 1; j < kPushThreads / 64; j++)
-        acc = (k & 1) ? fmax(acc, red[j][k]) : fmin(acc, red[j][k]);
-      partials[(int64_t)blockIdx.x * 6 + k] = acc;
-    }
-  }
+  if (EXTREMA) block_extrema(lo, hi, partials);
 }
 
 
@@ -692,6 +772,44 @@ int launch_push(const DeviceBunchView& v, const OpProgram& prog, const Op* kick0
     kick0 ? by_level(Yes{}, Yes{}) : by_level(Yes{}, No{});
   else
     kick0 ? by_level(No{}, Yes{}) : by_level(No{}, No{});
+  OB_HIP(hipGetLastError());
+  return blocks;
+}
+
+int launch_tile_push(const DeviceBunchView& v, const TileKick& t, const OpProgram& prog,
+                     double* ext_partials, hipStream_t s) {
+  OB_REQUIRE(v.n == t.n, "tile kick: the bunch has changed since its sort");
+  OB_REQUIRE(prog.level <= 1 && prog.words <= kProgSmallWords, "tile kick: program too long");
+  const bool ext = prog.want_extrema != 0;
+  OB_REQUIRE(!ext || ext_partials != nullptr, "push: extrema requested without a buffer");
+  const size_t lds = tile_lds_bytes(t.g);
+  const int blocks = (int)std::min<int64_t>(t.max_items + 1, kMaxPushBlocks);
+  ProgramWords<kProgSmallWords> small;
+  std::memcpy(&small, &prog, offsetof(ProgramWords<kProgSmallWords>, data) +
+                                 sizeof(double) * prog.words);
+  ProfScope ps(prog.words || ext ? (ext ? "tile_push_extrema" : "tile_push") : "tile_kick");
+  auto go = [&](auto cb, auto ce, auto cl, auto cm) {
+    constexpr bool B = decltype(cb)::value != 0, E = decltype(ce)::value != 0;
+    constexpr bool M = decltype(cm)::value != 0;
+    constexpr int L = decltype(cl)::value;
+    static bool ready = false;
+    if (!ready) {  // (extrema: 192 static bytes beside the block of phi)
+      OB_HIP(hipFuncSetAttribute((const void*)tile_push<B, E, L, M>,
+                                 hipFuncAttributeMaxDynamicSharedMemorySize, 159 * 1024));
+      ready = true;
+    }
+    hipLaunchKernelGGL((tile_push<B, E, L, M>), dim3(blocks), dim3(kTileThreads), lds, s, v.c[0],
+                       (int64_t)(v.c[1] - v.c[0]), t, small, ext_partials);
+  };
+  using No = std::integral_constant<int, 0>;
+  using Yes = std::integral_constant<int, 1>;
+  auto by_bnd = [&](auto... r) { t.k.bnd_type ? go(Yes{}, r...) : go(No{}, r...); };
+  if (!ext && prog.words == 0)
+    by_bnd(No{}, No{}, No{});
+  else if (prog.level == 1)
+    ext ? by_bnd(Yes{}, Yes{}, Yes{}) : by_bnd(No{}, Yes{}, Yes{});
+  else
+    ext ? by_bnd(Yes{}, No{}, Yes{}) : by_bnd(No{}, No{}, Yes{});
   OB_HIP(hipGetLastError());
   return blocks;
 }

@@ -941,6 +941,7 @@ OB_API int ob_sc3d_track(ob_sc3d* c, ob_bunch* b, double length) {
   if (n < 2) return 0;  // :102-103
   hipStream_t s = ob::stream();
   const int nblk = ob::bunch_flush(b, c->partials);
+  ob::flush_kicks_reading(c->phi);  // (other bunches' waiting kicks)
   const double* ext = ob::extrema_to_host(c->ext, c->partials, nblk, s);
   const ob::SyncInfo sy = ob::bunch_sync(b);
   const double gamma = sy.gamma, beta = sy.beta;
@@ -1273,6 +1274,7 @@ void slice_track(ob_slice2d* c, ob_bunch* b, double length, ob_boundary2d* bnd) 
   if (n < 2) return;  // :69-70
   hipStream_t s = stream();
   const int nblk = bunch_flush(b, c->partials);
+  flush_kicks_reading(c->phi);  // (other bunches' waiting kicks)
   const double* ext = extrema_to_host(c->ext, c->partials, nblk, s);
   const SyncInfo sy = bunch_sync(b);
   double xMin = ext[0], xMax = ext[1], yMin = ext[2];

@@ -13,19 +13,21 @@
 //   4. tile_deposit one workgroup per work item accumulates its particles into an LDS
 //                   block of the box plus a one-node halo, then adds the block to rho with
 //                   atomics;
-//   5. tile_kick    after the Poisson solve, one workgroup per work item copies the same
-//                   block of phi into LDS and computes its particles' kicks from it.
+//   5. the kick     after the Poisson solve, workgroups copy the same block of phi into LDS
+//                   and compute their particles' kicks from it.  It waits on the bunch and
+//                   runs in the launch of the maps that follow it (tile_push in ob_push.hip).
 // The blocks are small (~14 KiB for 8 x 8 x 16 boxes), so many workgroups share a CU.
 // Weights, indices and the kick arithmetic are the reference's (same device helpers as
 // the unsorted path); only the FP64 summation order of rho differs.
 #include "ob_internal.hpp"
 #include "ob_sc_device.hpp"
 #include "ob_tiled3d.hpp"
+#include "ob_tiled3d_device.hpp"
 
 namespace ob {
 namespace {
 
-constexpr int kThreads = 256;
+constexpr int kThreads = kTileThreads;
 constexpr int kChunk = 1024;
 constexpr int kMaxTiles = 16383;  // (ntiles + 1) 32-bit counters in 64 KiB of LDS (the scan: 2x)
 
@@ -42,54 +44,6 @@ __device__ __forceinline__ uint32_t tile_key(const TileGeom& g, double x, double
   grid3d_z_ind_frac(z, g.zMin, g.dz, g.nz, iZ, zF);
   return (uint32_t)(((iX / g.T) * g.ty + (iY / g.T)) * g.tz + iZ / g.Tz);
 }
-
-// Cell c = (lx*W + ly)*Wz + lz of a tile block, advanced by kThreads cells per step with
-// carries instead of a division per cell (the divisions are done once per thread).
-struct CellWalk {
-  int lx, ly, lz, sx, sy, sz, W, Wz;
-  __device__ __forceinline__ CellWalk(int c, int W_, int Wz_) : W(W_), Wz(Wz_) {
-    lz = c % Wz;
-    const int r = c / Wz;
-    ly = r % W;
-    lx = r / W;
-    sz = kThreads % Wz;
-    const int sr = kThreads / Wz;
-    sy = sr % W;
-    sx = sr / W;
-  }
-  __device__ __forceinline__ void next() {
-    lz += sz;
-    int carry = lz >= Wz ? 1 : 0;
-    lz -= carry * Wz;
-    ly += sy + carry;  // < 2W
-    carry = ly >= W ? 1 : 0;
-    ly -= carry * W;
-    lx += sx + carry;
-  }
-};
-
-// Tile t's LDS block: nodes x0..x0+W-1, y0..y0+W-1, z0..z0+Wz-1, z fastest.
-struct TileBox {
-  int x0, y0, z0, W, Wz;
-  __device__ __forceinline__ TileBox(const TileGeom& g, int t) {
-    const int tzi = t % g.tz, r = t / g.tz;
-    const int tyi = r % g.ty, txi = r / g.ty;
-    W = g.T + 2;
-    Wz = g.Tz + 2 * g.zh;
-    x0 = txi * g.T - 1;
-    y0 = tyi * g.T - 1;
-    z0 = tzi * g.Tz - g.zh;
-  }
-  __device__ __forceinline__ int cells() const { return W * W * Wz; }
-  __device__ __forceinline__ int idx(int gx, int gy, int gz) const {
-    return ((gx - x0) * W + (gy - y0)) * Wz + (gz - z0);
-  }
-  // nodes gx-1..gx+1, gy-1..gy+1, zlo..zhi inside the block
-  __device__ __forceinline__ bool holds(int gx, int gy, int zlo, int zhi) const {
-    return gx - 1 >= x0 && gx + 1 < x0 + W && gy - 1 >= y0 && gy + 1 < y0 + W && zlo >= z0 &&
-           zhi < z0 + Wz;
-  }
-};
 
 // Workgroups past hist_blocks clear rho, which the deposit needs: the histogram waits for
 // particle loads and LDS, so the stores cost next to nothing beside it (a launch of their own
@@ -469,146 +423,6 @@ __global__ __launch_bounds__(kThreads) void tile_deposit(const double* __restric
   }
 }
 
-// SpaceChargeCalc3D kick of particle i, gathering phi through view v (which must hold the
-// 27 nodes) or the whole grid.
-// BND: particles outside the boundary in k are not kicked.
-// The kick of particle i at (x, y, z) with momenta (xp, yp, dE) already read: writes
-// xp, yp, dE (the rest of kick_particle).
-template <bool BND>
-__device__ __forceinline__ void kick_particle_all(double* __restrict__ cur, int64_t cap,
-                                                  int64_t i, double x, double y, double z,
-                                                  double xp, double yp, double dE,
-                                                  const TileGeom& g, const Kick3D& k,
-                                                  const double* lds, const TileBox* box);
-
-template <bool BND>
-__device__ __forceinline__ void kick_particle_xyz(double* __restrict__ cur, int64_t cap,
-                                                  int64_t i, double x, double y, double z,
-                                                  const TileGeom& g, const Kick3D& k,
-                                                  const double* lds, const TileBox* box) {
-  if (BND && !boundary_inside(k.bnd_type, k.bnd, x, y)) return;
-  const double zr = (z - k.zc) * k.gamma + k.zc;
-  int iX, iY, iZ;
-  double xF, yF, zF;
-  node_ind_frac(x, g.xMin, g.dx, g.nx, iX, xF);
-  node_ind_frac(y, g.yMin, g.dy, g.ny, iY, yF);
-  grid3d_z_ind_frac(zr, k.rzMin, k.rdz, g.nz, iZ, zF);
-  const int zlo = g.nz >= 3 ? iZ - 1 : 0, zhi = g.nz >= 3 ? iZ + 1 : g.nz - 1;
-  double ex, ey, ez;
-  if (box && box->holds(iX, iY, zlo, zhi)) {
-    const Grid3View v{lds, (int64_t)box->W * box->Wz, box->Wz, box->x0, box->y0, box->z0};
-    grid3d_gradient_at(v, g.nz, iX, iY, iZ, xF, yF, zF, g.dx, g.dy, k.rdz, ex, ey, ez);
-  } else {
-    const Grid3View v{k.phi, (int64_t)g.ny * g.nz, g.nz, 0, 0, 0};
-    grid3d_gradient_at(v, g.nz, iX, iY, iZ, xF, yF, zF, g.dx, g.dy, k.rdz, ex, ey, ez);
-  }
-  cur[cap + i] += -ex * k.trans_factor;
-  cur[3 * cap + i] += -ey * k.trans_factor;
-  cur[5 * cap + i] += -ez * k.long_factor;
-}
-
-template <bool BND>
-__device__ __forceinline__ void kick_particle_all(double* __restrict__ cur, int64_t cap,
-                                                  int64_t i, double x, double y, double z,
-                                                  double xp, double yp, double dE,
-                                                  const TileGeom& g, const Kick3D& k,
-                                                  const double* lds, const TileBox* box) {
-  if (BND && !boundary_inside(k.bnd_type, k.bnd, x, y)) return;
-  const double zr = (z - k.zc) * k.gamma + k.zc;
-  int iX, iY, iZ;
-  double xF, yF, zF;
-  node_ind_frac(x, g.xMin, g.dx, g.nx, iX, xF);
-  node_ind_frac(y, g.yMin, g.dy, g.ny, iY, yF);
-  grid3d_z_ind_frac(zr, k.rzMin, k.rdz, g.nz, iZ, zF);
-  const int zlo = g.nz >= 3 ? iZ - 1 : 0, zhi = g.nz >= 3 ? iZ + 1 : g.nz - 1;
-  double ex, ey, ez;
-  if (box->holds(iX, iY, zlo, zhi)) {
-    const Grid3View v{lds, (int64_t)box->W * box->Wz, box->Wz, box->x0, box->y0, box->z0};
-    grid3d_gradient_at(v, g.nz, iX, iY, iZ, xF, yF, zF, g.dx, g.dy, k.rdz, ex, ey, ez);
-  } else {
-    const Grid3View v{k.phi, (int64_t)g.ny * g.nz, g.nz, 0, 0, 0};
-    grid3d_gradient_at(v, g.nz, iX, iY, iZ, xF, yF, zF, g.dx, g.dy, k.rdz, ex, ey, ez);
-  }
-  cur[cap + i] = xp + -ex * k.trans_factor;
-  cur[3 * cap + i] = yp + -ey * k.trans_factor;
-  cur[5 * cap + i] = dE + -ez * k.long_factor;
-}
-
-template <bool BND>
-__device__ __forceinline__ void kick_particle(double* __restrict__ cur, int64_t cap, int64_t i,
-                                              const TileGeom& g, const Kick3D& k,
-                                              const double* lds, const TileBox* box) {
-  kick_particle_xyz<BND>(cur, cap, i, cur[i], cur[2 * cap + i], cur[4 * cap + i], g, k, lds,
-                         box);
-}
-
-// Blocks 0..nitems-1: work items; block nitems: the particles outside the grid (last in the
-// sorted order, from offsets[ntiles]), kicked from the whole grid like the reference.
-// At least 3 waves per SIMD: the kick with the next particle's prefetch takes 157 VGPRs
-// without spills.  Bounded to 4 waves (128 VGPRs) the prefetch spills and the kick ran
-// 133 us against 113; without the prefetch, 119.
-template <bool BND>
-__global__ __launch_bounds__(kThreads, 3) void tile_kick(double* __restrict__ cur, int64_t cap,
-                                                      int64_t n, TileGeom g, Kick3D k,
-                                                      const int4* __restrict__ items,
-                                                      const uint32_t* __restrict__ nitems,
-                                                      const uint32_t* __restrict__ offsets) {
-  const uint32_t ni = *nitems;
-  if (blockIdx.x > ni) return;
-  if (blockIdx.x == ni) {
-    for (int64_t i = (int64_t)offsets[g.ntiles] + threadIdx.x; i < n; i += blockDim.x)
-      kick_particle<BND>(cur, cap, i, g, k, nullptr, nullptr);
-    return;
-  }
-  extern __shared__ double sphi[];
-  const int4 it = items[blockIdx.x];
-  const TileBox box(g, it.x);
-  const int cells = box.cells();
-  const int64_t gsx = (int64_t)g.ny * g.nz;
-  // The first particle's coordinates are requested with the block of phi, and all of a
-  // thread's block loads are issued before any is stored (a masked lane loads phi[0] and
-  // stores 0), so these latencies overlap instead of adding up.
-  const int i0 = it.y + (int)threadIdx.x;
-  const int ia = i0 < it.z ? i0 : it.y;
-  const double px = cur[ia], py = cur[2 * cap + ia], pz = cur[4 * cap + ia];
-  const double pxp = cur[cap + ia], pyp = cur[3 * cap + ia], pdE = cur[5 * cap + ia];
-  constexpr int KB = 8;  // cells <= KB * kThreads for blocks of up to 16 KiB
-  double bv[KB];
-  uint32_t inmask = 0;
-  CellWalk w((int)threadIdx.x, box.W, box.Wz);
-#pragma unroll
-  for (int u = 0; u < KB; u++, w.next()) {
-    const int c = (int)threadIdx.x + u * kThreads;
-    const int gx = box.x0 + w.lx, gy = box.y0 + w.ly, gz = box.z0 + w.lz;
-    const bool in = c < cells && gx >= 0 && gx < g.nx && gy >= 0 && gy < g.ny && gz >= 0 &&
-                    gz < g.nz;
-    bv[u] = k.phi[in ? gx * gsx + (int64_t)gy * g.nz + gz : 0];
-    inmask |= (in ? 1u : 0u) << u;
-  }
-#pragma unroll
-  for (int u = 0; u < KB; u++) {
-    const int c = (int)threadIdx.x + u * kThreads;
-    if (c < cells) sphi[c] = ((inmask >> u) & 1u) ? bv[u] : 0.0;
-  }
-  for (int c = (int)threadIdx.x + KB * kThreads; c < cells; c += kThreads, w.next()) {
-    // larger blocks: the walk continues from cell threadIdx.x + KB * kThreads
-    const int gx = box.x0 + w.lx, gy = box.y0 + w.ly, gz = box.z0 + w.lz;
-    const bool in = gx >= 0 && gx < g.nx && gy >= 0 && gy < g.ny && gz >= 0 && gz < g.nz;
-    sphi[c] = in ? k.phi[gx * gsx + (int64_t)gy * g.nz + gz] : 0.0;
-  }
-  __syncthreads();
-  // The next particle's coordinates are loaded before this one is kicked.
-  double q[6] = {px, py, pz, pxp, pyp, pdE};
-  for (int i = i0; i < it.z; i += kThreads) {
-    const int in = i + kThreads < it.z ? i + kThreads : i;
-    const double nq[6] = {cur[in], cur[2 * cap + in], cur[4 * cap + in],
-                          cur[cap + in], cur[3 * cap + in], cur[5 * cap + in]};
-    kick_particle_all<BND>(cur, cap, i, q[0], q[1], q[2], q[3], q[4], q[5], g, k, sphi, &box);
-#pragma unroll
-    for (int c = 0; c < 6; c++) q[c] = nq[c];
-  }
-}
-
 }  // namespace
 
 TileGeom make_tile_geom(int nx, int ny, int nz, double xMin, double xMax, double yMin,
@@ -694,10 +508,6 @@ void sort_and_deposit_3d(ob_bunch* b, const TileGeom& g, double macrosize, doubl
                                hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
     OB_HIP(hipFuncSetAttribute((const void*)tile_scan,
                                hipFuncAttributeMaxDynamicSharedMemorySize, 136 * 1024));
-    OB_HIP(hipFuncSetAttribute((const void*)tile_kick<false>,
-                               hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-    OB_HIP(hipFuncSetAttribute((const void*)tile_kick<true>,
-                               hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
     attr_done = true;
   }
   const int64_t n = bunch_size(b);
@@ -760,21 +570,11 @@ void sort_and_deposit_3d(ob_bunch* b, const TileGeom& g, double macrosize, doubl
 void tile_kick_3d(ob_bunch* b, const TileGeom& g, const Kick3D& k, TileWork& w) {
   const int64_t n = bunch_size(b);
   if (n == 0) return;
-  DeviceBunchView v = bunch_device_view(b);
-  const int64_t max_items = n / kChunk + g.ntiles + 1;
-  {
-    ProfScope ps("tile_kick");
-    if (k.bnd_type)
-      hipLaunchKernelGGL(tile_kick<true>, dim3((unsigned)(max_items + 1)), dim3(kThreads),
-                         tile_lds_bytes(g), stream(), v.c[0], (int64_t)(v.c[1] - v.c[0]), n, g, k,
-                         w.items, w.nitems, w.offsets);
-    else
-      hipLaunchKernelGGL(tile_kick<false>, dim3((unsigned)(max_items + 1)), dim3(kThreads),
-                         tile_lds_bytes(g), stream(), v.c[0], (int64_t)(v.c[1] - v.c[0]), n, g, k,
-                         w.items, w.nitems, w.offsets);
-  }
-  OB_HIP(hipGetLastError());
-  bunch_device_written(b);
+  TileKick t{g, k, w.items, w.nitems, w.offsets, n, n / kChunk + g.ntiles + 1};
+  t.k.fx = k.trans_factor / g.dx;
+  t.k.fy = k.trans_factor / g.dy;
+  t.k.fz = k.long_factor / k.rdz;
+  bunch_queue_tile_kick(b, t);
 }
 
 }  // namespace ob

@@ -48,7 +48,27 @@ struct Kick3D {
   // (SpaceChargeCalcSliceBySlice2D.cc:104); type 0 = no boundary (SC2DState::bnd_type).
   int bnd_type;
   double bnd[6];
+  double fx, fy, fz;  // the factors over the grid steps (set by tile_kick_3d)
 };
+// The kick waits on the bunch (bunch_queue_tile_kick) and is applied, before any queued map, by
+// the bunch's next flush: with the maps that follow it, in one pass over the particles.  What
+// it reads (phi and the work items, the calculator's) is not written while a kick waits:
+// flush_kicks_reading(phi) comes before the calculator's next step and before its end.
 void tile_kick_3d(ob_bunch* b, const TileGeom& g, const Kick3D& k, TileWork& w);
+
+// A waiting kick.
+struct TileKick {
+  TileGeom g;
+  Kick3D k;
+  const int4* items;
+  const uint32_t *nitems, *offsets;
+  int64_t n, max_items;
+};
+void bunch_queue_tile_kick(ob_bunch* b, const TileKick& t);
+
+// The kick of a bunch sorted for it, then prog (level 0 or 1, at most kProgSmallWords words);
+// extrema as launch_push.  Returns the workgroups (rows of ext_partials, at most 4096).
+int launch_tile_push(const DeviceBunchView& v, const TileKick& t, const OpProgram& prog,
+                     double* ext_partials, hipStream_t s);
 
 }  // namespace ob
