@@ -29,6 +29,14 @@ namespace {
 
 constexpr int kThreads = kTileThreads;
 constexpr int kChunk = 1024;
+
+// Particles of a work item at most.  A step of few particles has too few items of 1024 for 256
+// CUs: at 50k particles on 32 x 32 x 32 nodes items of 256 take the deposit from 15.4 to 12.0
+// us, the kick from 13.0 to 8.4 and a step from 72 to 63 (items of 512: 65); at 100k on 64 x 64
+// x 64 nodes the step takes 85 with 256 or 512 and 90 with 1024, at 200k 104, 93 and 97, at
+// 300k 124, 106 and 103 (a tile's copies then cost more than the CUs give).
+int64_t tile_chunk(int64_t n) { return n <= 1 << 16 ? 256 : n <= 1 << 18 ? 512 : kChunk; }
+
 constexpr int kMaxTiles = 16383;  // (ntiles + 1) 32-bit counters in 64 KiB of LDS (the scan: 2x)
 
 __device__ __forceinline__ bool inside(const TileGeom& g, double x, double y, double z) {
@@ -108,7 +116,8 @@ __global__ __launch_bounds__(1024) void tile_scan(uint32_t* __restrict__ counts,
                                                   uint32_t* __restrict__ offsets,
                                                   uint32_t* __restrict__ cursor,
                                                   int4* __restrict__ items,
-                                                  uint32_t* __restrict__ nitems) {
+                                                  uint32_t* __restrict__ nitems,
+                                                  uint32_t chunk) {
   extern __shared__ uint32_t ls[];
   const int nb = ntiles + 1;
   uint32_t* loff = ls;            // [nb + 1]: counts, then exclusive particle offsets
@@ -132,7 +141,7 @@ __global__ __launch_bounds__(1024) void tile_scan(uint32_t* __restrict__ counts,
   for (int t = lo; t < hi; t++) {
     const uint32_t k = loff[t];
     off += k;
-    if (t < ntiles) item += (k + kChunk - 1) / kChunk;
+    if (t < ntiles) item += (k + chunk - 1) / chunk;
   }
   uint32_t total, total_items;
   block_scan2(off, item, total, total_items);
@@ -142,7 +151,7 @@ __global__ __launch_bounds__(1024) void tile_scan(uint32_t* __restrict__ counts,
     loff[t] = off;
     litem[t] = item;
     off += k;
-    if (t < ntiles) item += (k + kChunk - 1) / kChunk;
+    if (t < ntiles) item += (k + chunk - 1) / chunk;
   }
   if (threadIdx.x == 0) {
     loff[nb] = total;
@@ -159,8 +168,8 @@ __global__ __launch_bounds__(1024) void tile_scan(uint32_t* __restrict__ counts,
     counts[t] = 0;
     if (t < ntiles) {
       uint32_t j = litem[t];
-      for (uint32_t b0 = o; b0 < e; b0 += kChunk)
-        items[j++] = make_int4(t, (int)b0, (int)min(e, b0 + kChunk), 0);
+      for (uint32_t b0 = o; b0 < e; b0 += chunk)
+        items[j++] = make_int4(t, (int)b0, (int)min(e, b0 + chunk), 0);
     }
   }
 }
@@ -177,6 +186,7 @@ struct ScatterScan {
   uint32_t* offsets;
   int4* items;
   uint32_t* nitems;
+  uint32_t chunk;
 };
 template <bool SCAN>
 __global__ __launch_bounds__(kThreads) void tile_scatter(
@@ -186,6 +196,7 @@ __global__ __launch_bounds__(kThreads) void tile_scatter(
     const double* __restrict__ msize, double* __restrict__ msize_alt, int64_t per_block,
     ScatterScan sc) {
   extern __shared__ uint32_t sh[];
+  const uint32_t chunk = sc.chunk;
   uint32_t* lc = sh;               // local counts, then running destinations
   const int nb = ntiles + 1;
   uint32_t* loff = sh + nb;        // SCAN: tile offsets
@@ -198,7 +209,7 @@ __global__ __launch_bounds__(kThreads) void tile_scatter(
       const uint32_t k = sc.counts[t];
       loff[t] = k;
       off += k;
-      if (t < ntiles) item += (k + kChunk - 1) / kChunk;
+      if (t < ntiles) item += (k + chunk - 1) / chunk;
     }
     uint32_t total, total_items;
     block_scan2(off, item, total, total_items);
@@ -209,9 +220,9 @@ __global__ __launch_bounds__(kThreads) void tile_scatter(
       if (writer) {
         sc.offsets[t] = off;
         if (t < ntiles)
-          for (uint32_t b0 = 0; b0 < k; b0 += kChunk)
+          for (uint32_t b0 = 0; b0 < k; b0 += chunk)
             sc.items[item++] =
-                make_int4(t, (int)(off + b0), (int)(off + min(k, b0 + (uint32_t)kChunk)), 0);
+                make_int4(t, (int)(off + b0), (int)(off + min(k, b0 + chunk)), 0);
       }
       off += k;
     }
@@ -470,7 +481,7 @@ void TileWork::reserve(int64_t n, int ntiles) {
     OB_HIP(hipMalloc((void**)&key, sizeof(uint32_t) * c));
     n_cap = c;
   }
-  const int64_t want_items = n_cap / kChunk + ntiles + 2;
+  const int64_t want_items = n_cap / kChunk + ntiles + 2;  // (tile_chunk: at most 512 more)
   if (ntiles + 1 > t_cap || want_items > i_cap) {
     for (void* p : {(void*)counts, (void*)offsets, (void*)cursor, (void*)items, (void*)nitems})
       if (p) OB_HIP(hipFree(p));
@@ -536,14 +547,14 @@ void sort_and_deposit_3d(ob_bunch* b, const TileGeom& g, double macrosize, doubl
     ProfScope ps("tile_scan");
     hipLaunchKernelGGL(tile_scan, dim3(1), dim3(1024), sizeof(uint32_t) * 2 * (g.ntiles + 2), s,
                        w.counts, g.ntiles, w.offsets,
-                       w.cursor, w.items, w.nitems);
+                       w.cursor, w.items, w.nitems, (uint32_t)tile_chunk(n));
   }
   // about 4096 workgroups: measured fastest for the scatter and for the deposit after it
   const int64_t per = std::max<int64_t>(512, (n + 4095) / 4096);
   const int sb_blocks = (int)((n + per - 1) / per);
   if (n) {
     ProfScope ps("tile_scatter");
-    const ScatterScan sc{w.counts, w.offsets, w.items, w.nitems};
+    const ScatterScan sc{w.counts, w.offsets, w.items, w.nitems, (uint32_t)tile_chunk(n)};
     if (scan)
       hipLaunchKernelGGL(tile_scatter<true>, dim3(sb_blocks), dim3(kThreads), 2 * hl, s, sb.cur,
                          sb.alt, sb.cap, n, w.key, g.ntiles, w.cursor, sb.perm, sb.perm_alt,
@@ -556,7 +567,7 @@ void sort_and_deposit_3d(ob_bunch* b, const TileGeom& g, double macrosize, doubl
   OB_HIP(hipGetLastError());
   bunch_sort_commit(b);
   DeviceBunchView v = bunch_device_view(b);
-  const int64_t max_items = n / kChunk + g.ntiles + 1;
+  const int64_t max_items = n / tile_chunk(n) + g.ntiles + 1;
   {
     ProfScope ps("tile_deposit");
     hipLaunchKernelGGL(tile_deposit, dim3((unsigned)max_items), dim3(kThreads),
@@ -570,7 +581,7 @@ void sort_and_deposit_3d(ob_bunch* b, const TileGeom& g, double macrosize, doubl
 void tile_kick_3d(ob_bunch* b, const TileGeom& g, const Kick3D& k, TileWork& w) {
   const int64_t n = bunch_size(b);
   if (n == 0) return;
-  TileKick t{g, k, w.items, w.nitems, w.offsets, n, n / kChunk + g.ntiles + 1};
+  TileKick t{g, k, w.items, w.nitems, w.offsets, n, n / tile_chunk(n) + g.ntiles + 1};
   t.k.fx = k.trans_factor / g.dx;
   t.k.fy = k.trans_factor / g.dy;
   t.k.fz = k.long_factor / k.rdz;

@@ -96,3 +96,22 @@ def test_kick_waits_for_the_maps(calc_name, grid, maps):
             assert np.abs(o1[k] - o2[k]).max() <= 1e-12 * np.abs(o2[k]).max(), k
             if k in (1, 3):  # (one node in z and slices: no dE kick)
                 assert not np.array_equal(o1[k], c[k])
+
+
+@pytest.mark.parametrize("n", [65_536, 65_537, 262_144, 262_145])
+def test_item_sizes(n):
+    """Work items of 256, 512 and 1024 particles, at the limits between them, most particles in
+    one tile."""
+    import spacecharge
+    c = _coords(n, 8) * np.where(np.random.default_rng(9).random(n) < 0.9, 0.05, 1.0)
+    b, _ = _bunches(c)
+    calc, plain = spacecharge.SpaceChargeCalc3D(40, 40, 40), spacecharge.SpaceChargeCalc3D(40, 40, 40)
+    plain.setDepositMode(False)
+    b2, _ = _bunches(c)
+    calc.trackBunch(b, 0.3)
+    plain.trackBunch(b2, 0.3)
+    rho, ref = calc.getRhoGrid().array(), plain.getRhoGrid().array()
+    assert np.abs(rho - ref).max() <= n * 1.2e-16 * np.abs(ref).max()
+    o1, o2 = b.getCoordinates(), b2.getCoordinates()
+    for k in range(6):
+        assert np.abs(o1[k] - o2[k]).max() <= 1e-12 * np.abs(o2[k]).max(), k
