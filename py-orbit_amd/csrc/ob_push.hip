@@ -392,6 +392,7 @@ __device__ __forceinline__ void run_program(const PROG& prog, double& x, double&
 
 constexpr int kPushThreads = 256;
 constexpr int kMaxPushBlocks = 4096;
+constexpr int kKickPushBlocks = 1024;
 
 __device__ __forceinline__ double wave_min(double v) {
   for (int o = 32; o > 0; o >>= 1) v = fmin(v, __shfl_xor(v, o, 64));
@@ -731,7 +732,12 @@ int push_grid_blocks(int64_t n) {
 
 int launch_push(const DeviceBunchView& v, const OpProgram& prog, const Op* kick0,
                 double* ext_partials, hipStream_t s) {
-  const int blocks = push_grid_blocks(v.n);
+  // With a leading 2.5D kick, four waves per SIMD fit and 1024 workgroups are resident at once:
+  // more only wait, each with the latency of its first loads and a row of extrema for the
+  // next kernel to read (1M particles, 200 x 150 nodes: push 34.5 us with 3907 workgroups, 31.7
+  // with 1024, 33.8 with 512; the deposit that reads the rows 26.9, 25.7, 25.6).  Maps alone
+  // fit more waves: a ring's programs take 208 us with 3907 workgroups, 244 with 1024.
+  const int blocks = std::min(push_grid_blocks(v.n), kick0 ? kKickPushBlocks : kMaxPushBlocks);
   const bool ext = prog.want_extrema != 0;
   OB_REQUIRE(!ext || ext_partials != nullptr, "push: extrema requested without a buffer");
   if (!ext && ((prog.words == 0 && !kick0) || v.n == 0)) return 0;
