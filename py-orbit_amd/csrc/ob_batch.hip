@@ -6,7 +6,9 @@
 //   push     one workgroup per work item (a chunk of one bunch's particles): deferred SC
 //            kick, the map program, per-item extrema;
 //   setup    one workgroup per bunch (extrema of its items, grid sizing, clearing);
-//   deposit  tile sort per bunch: hist and scatter one workgroup per work item, then one
+//   deposit  where every grid fits and nothing changes rho, LDS copies of the grids (three
+//            passes with the solve, see sc2d_gdeposit_batch); otherwise setup and a tile sort
+//            per bunch: hist and scatter one workgroup per work item, then one
 //            workgroup per tile work item accumulating rho in LDS;
 //   post     one workgroup per bunch; FFT row / column / row passes over all bunches'
 //            rows and columns (the FFT length is dispatched per workgroup).
@@ -80,7 +82,9 @@ void build_records(ob_batch* B, bool force) {
     if (same && (B->seen_n[b] != views[b].n || B->seen_ptr[b] != views[b].c[0])) same = false;
     // the calculator's tile buffers move if it tracked a larger bunch on its own
     if (same && !B->calcs.empty() &&
-        !sc2d_tile_same(B->calcs[b], B->h_bb[b].tg, views[b].n, views[b].msize != nullptr))
+        !(B->h_bb[b].sd.slabs
+              ? sc2d_slab_same(B->calcs[b], B->h_bb[b].sd)
+              : sc2d_tile_same(B->calcs[b], B->h_bb[b].tg, views[b].n, views[b].msize != nullptr)))
       same = false;
     if (same) {  // RingRF changed the synchronous momentum: new kick factors
       const SyncInfo sy = bunch_sync(B->bunches[b]);
@@ -96,7 +100,14 @@ void build_records(ob_batch* B, bool force) {
   B->h_bb.assign(nb, BatchBunch{});
   B->h_items.clear();
   int rows = 0, cols = 0, max_M = 16, slots = 0;
-  size_t hist_lds = 0, dep_lds = 0;
+  size_t hist_lds = 0, dep_lds = 0, slab_lds = 0, srow_lds = 0;
+  int slabs = 0, srows = 0, scols = 0;
+  std::vector<SlabDep> split;
+  if (!B->calcs.empty()) {
+    std::vector<int64_t> n;
+    for (const DeviceBunchView& v : views) n.push_back(v.n);
+    if (!sc2d_batch_slabs(B->calcs, n, split)) split.clear();
+  }
   for (int b = 0; b < nb; b++) {
     BatchBunch& r = B->h_bb[b];
     std::memset(&r, 0, sizeof(r));
@@ -117,6 +128,18 @@ void build_records(ob_batch* B, bool force) {
       rows += (r.nx + 1) / 2;
       cols += r.H;
       max_M = std::max(max_M, std::max(r.M0, r.M1));
+      if (!split.empty()) {
+        r.sd = split[b];
+        r.slab_begin = slabs;
+        r.srows_begin = srows;
+        r.scols_begin = scols;
+        slabs += r.sd.slabs * r.sd.parts;
+        srows += r.nx;
+        scols += r.H + 2;
+        slab_lds = std::max(slab_lds, sc2d_slab_lds(r));
+        srow_lds = std::max(srow_lds, sc2d_row_lds(r));
+        continue;
+      }
       r.tg = sc2d_tile_reserve(B->calcs[b], r.v.n, r.v.msize != nullptr, B->item, 1,
                                r.item_end - r.item_begin);
       r.slot_begin = slots;
@@ -148,7 +171,8 @@ void build_records(ob_batch* B, bool force) {
     OB_HIP(hipMemcpyAsync(B->d_items, B->h_items.data(), sizeof(BatchItem) * ni,
                           hipMemcpyHostToDevice, s));
   OB_HIP(hipStreamSynchronize(s));  // host vectors may change before the copies run
-  B->shape = BatchShape{nb, ni, rows, cols, max_M, slots, hist_lds, dep_lds};
+  B->shape = BatchShape{nb,    ni,    rows,  cols,     max_M,   slots, hist_lds, dep_lds,
+                        slabs, srows, scols, slab_lds, srow_lds};
   B->seen_n.resize(nb);
   B->seen_ptr.resize(nb);
   for (int b = 0; b < nb; b++) {
@@ -262,7 +286,7 @@ void autotune(ob_batch* B) {
     }
   }
   B->chunk = best_chunk;
-  if (!B->calcs.empty()) {
+  if (!B->calcs.empty() && !B->shape.slab_blocks) {
     best = 1e30f;
     int best_item = B->item;
     for (int item : {256, 1024, 4096}) {

@@ -219,6 +219,21 @@ struct Tile2D {
 struct ob_denoiser;
 namespace ob {
 // ---- batches of bunches, each with its own SpaceChargeCalc2p5Drb ----------------------
+// Grid-copy deposit: workgroup s * parts + p deposits the particles of part p whose TSC
+// centre row lies in slab s (centre rows 1 + s * rows .. (s + 1) * rows) into its own LDS
+// copy of the slab's nodes (rows s * rows .. s * rows + rows + 1, R = rows + 2 of them) and
+// stores it as copy s * parts + p.
+struct SlabDep {
+  int slabs, parts, rows, R;
+  int64_t per;     // particles per part
+  double* copies;  // [slabs * parts][R * ny]
+  double* zpart;   // [parts][nz] z line densities
+  double* mrows;   // [nx][5] rho moments of the grid rows, written by the row pass
+  int green_blocks;  // SpaceChargeCalc2p5D: workgroups after the deposit's that transform
+  double2* gspec;    // the rows of a new Green function into gspec ([M0][H]); 0 otherwise
+  int M0;
+};
+
 // Device-resident record of one bunch of a batch.
 struct BatchBunch {
   DeviceBunchView v;
@@ -233,6 +248,8 @@ struct BatchBunch {
   Tile2D tg;                      // deposit tile sort (buffers owned by the calculator)
   int32_t slot_begin, slot_end;   // its blocks of the batched tile-deposit pass
   int32_t moments_from_rho, pad;  // 1: rho changes after the deposit (denoiser)
+  SlabDep sd;  // grid-copy deposit (slabs 0: the batch deposits through the tile sort)
+  int32_t slab_begin, srows_begin, scols_begin, pad2;  // its first blocks of those passes
 };
 struct BatchItem {  // particles [begin, end) of one bunch
   int32_t bunch, pad;
@@ -250,6 +267,8 @@ void launch_push_batch(const BatchBunch* bb, const BatchItem* items, int nitems,
 struct BatchShape {
   int nb, nitems, row_blocks, col_blocks, max_M, dep_slots;
   size_t hist_lds, dep_lds;  // dynamic LDS of the hist/scatter and tile-deposit passes
+  int slab_blocks, srow_blocks, scol_blocks;  // grid-copy deposit (slab_blocks 0: tile sort)
+  size_t slab_lds, srow_lds;
 };
 // Denoiser applied to one bunch's rho between the deposit and the moments.
 struct DenoiseJob {
@@ -291,6 +310,14 @@ Tile2D sc2d_tile_reserve(ob_sc2p5drb* c, int64_t n, bool per_particle_m, int ite
                          int zrows = 1, int hist_rows = 0);
 // Whether `t` still describes the calculator's tile buffers and fits such a bunch.
 bool sc2d_tile_same(ob_sc2p5drb* c, const Tile2D& t, int64_t n, bool per_particle_m);
+// Grid-copy deposit of a batch: the split of every bunch (n particles each), or false if a
+// grid does not fit it or a calculator has a denoiser.  sc2d_slab_same: D's buffers are still
+// the calculator's.
+bool sc2d_batch_slabs(const std::vector<ob_sc2p5drb*>& calcs, const std::vector<int64_t>& n,
+                      std::vector<SlabDep>& out);
+bool sc2d_slab_same(ob_sc2p5drb* c, const SlabDep& D);
+size_t sc2d_slab_lds(const BatchBunch& r);
+size_t sc2d_row_lds(const BatchBunch& r);
 void sc2d_mark_tracked(ob_sc2p5drb* c);
 int sc2d_read_status(ob_sc2p5drb* c);
 int push_grid_blocks(int64_t n);
