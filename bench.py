@@ -39,7 +39,8 @@ TRAFFIC_FILES = {"ring3d": "profiles/ring3d_hbm_traffic.md",
 # profiler label -> kernel name (prefix) in the rocprofv3 summaries
 ROCPROF_NAME = {"fft3_strided_conv": "fft3_strided<2,", "fft3_strided_fwd": "fft3_strided<0,",
                 "fft3_strided_inv": "fft3_strided<1,", "push_extrema": "push_kernel<true,",
-                "push": "push_kernel<false,", "fft_cols": "fft_cols<false,",
+                "push": "push_kernel<false,", "tile_push_extrema": "tile_push<false, true,",
+                "fft_cols": "fft_cols<false,", "sc2d_gdeposit": "sc2d_gdeposit<",
                 "fft3_z_r2c": "fft3_z_r2c<", "fft3_z_c2r": "fft3_z_c2r<"}
 
 
@@ -156,7 +157,8 @@ def kernel_bytes(workload, n, grid):
         qx, qy = M0 // 2 + 1, M1 // 2 + 1
         b.update({
             "deposit3d": 24 * n + 8 * ng,
-            "fill_zero": 8 * ng,
+            "tile_push_extrema": 96 * n + 8 * ng,
+            "tile_push": 96 * n + 8 * ng,
             "fft3_z_r2c": 8 * ng + 16 * nx * ny * H2,
             "fft3_strided_fwd": 16 * nx * ny * H2 + 16 * nx * M1 * H2,
             "fft3_strided_conv": 32 * nx * M1 * H2 + 8 * qx * qy * H2,
@@ -166,11 +168,9 @@ def kernel_bytes(workload, n, grid):
     else:
         H = M1 // 2 + 1
         b.update({
-            "sc2d_bin": 24 * n + 8 * nx * ny,
-            "sc2d_scatter": 32 * n,
-            "sc2d_tdeposit": 16 * n + 8 * nx * ny,
-            "fft_rows_r2c": 8 * nx * ny + 16 * nx * H,
-            "fft_cols": 32 * nx * H + 16 * M0 * H,
+            "sc2d_gdeposit": 24 * n + 8 * nx * ny,
+            "fft_rows_sum_post": 8 * nx * ny + 16 * nx * H,
+            "fft_cols_post": 32 * nx * H + 16 * M0 * H,
             "fft_rows_c2r": 16 * nx * H + 8 * nx * ny,
         })
     return b
@@ -352,7 +352,8 @@ def main_batch(args):
     grid_nodes = sum(sp["grid"][0] * sp["grid"][1] for sp in specs)
     kb = {"push_batch_extrema": 96 * n, "push_batch": 96 * n,
           "sc2d_hist_batch": 24 * n, "sc2d_scatter_batch": 32 * n,
-          "sc2d_tdeposit_batch": 16 * n + 8 * grid_nodes}
+          "sc2d_tdeposit_batch": 16 * n + 8 * grid_nodes,
+          "sc2d_gdeposit_batch": 24 * n + 8 * grid_nodes}
     dom = max((k for k in prof if k in kb), key=lambda k: prof[k][1])
     cnt, tot, _, _ = prof[dom]
     avg_s = tot / cnt / 1e3
