@@ -168,6 +168,7 @@ struct ob_bunch {
   std::vector<double> h[6];   // host mirror
   std::vector<double> h_msize;
   std::vector<uint8_t> alive; // host-side flags for deleteParticle/compress
+  int64_t dead = 0;           // zeros among them
   bool has_msize = false;
   bool host_valid = true, dev_valid = true;
 
@@ -706,6 +707,7 @@ OB_API int ob_bunch_set_coords(ob_bunch* b, int64_t n, const double* x, const do
   OB_HIP(hipStreamSynchronize(s));
   for (int k = 0; k < 6; k++) b->h[k].clear();
   b->alive.assign(n, 1);
+  b->dead = 0;
   b->has_msize = false;
   b->h_msize.clear();
   b->dev_valid = true;
@@ -762,7 +764,11 @@ OB_API int ob_bunch_get_size(ob_bunch* b, int64_t* n) {
 OB_API int ob_bunch_delete_particle(ob_bunch* b, int64_t i) {
   OB_TRY OB_CHECK_B(b);
   OB_REQUIRE(i >= 0 && i < b->n, "particle index out of range");
-  if ((int64_t)b->alive.size() != b->n) b->alive.assign(b->n, 1);
+  if ((int64_t)b->alive.size() != b->n) {
+    b->alive.assign(b->n, 1);
+    b->dead = 0;
+  }
+  if (b->alive[i]) b->dead++;
   b->alive[i] = 0;
   OB_CATCH
 }
@@ -771,11 +777,12 @@ OB_API int ob_bunch_compress(ob_bunch* b) {  // Bunch.cc:704-763 (order kept)
   OB_TRY OB_CHECK_B(b);
   if ((int64_t)b->alive.size() != b->n) {
     b->alive.assign(b->n, 1);
+    b->dead = 0;
     return 0;
   }
-  bool any_dead = false;
-  for (int64_t i = 0; i < b->n; i++) any_dead |= (b->alive[i] == 0);
-  if (!any_dead) return 0;
+  // (the count of dead particles is kept: the diagnostics compress first, and going through the
+  // flags of 1M particles three times took 31 us of 281 us for the diagnostics of a turn)
+  if (b->dead == 0) return 0;
   ob::host_write(b);
   int64_t w = 0;
   for (int64_t i = 0; i < b->n; i++) {
@@ -788,6 +795,7 @@ OB_API int ob_bunch_compress(ob_bunch* b) {  // Bunch.cc:704-763 (order kept)
   if (b->has_msize) b->h_msize.resize(w);
   b->n = w;
   b->alive.assign(w, 1);
+  b->dead = 0;
   OB_CATCH
 }
 

@@ -100,3 +100,26 @@ def test_profile_of_every_width(n, nz):
         np.add.at(ref, ip, 1 - w0)
     # weights from the same formulas; a bin adds up to n of them in another order
     assert np.abs(a - ref).max() <= 1e-12 * max(1.0, ref.max())
+
+
+def test_deleted_particles_are_counted():
+    """Deleting twice, adding after a deletion, deleting all: compress removes what was deleted
+    and nothing more, however often it is called."""
+    from workloads import make_bunch
+    c = np.random.default_rng(1).standard_normal((6, 9)) * 1e-3
+    b = make_bunch(c)
+    for i in (3, 3, 7):
+        b.deleteParticleFast(i)
+    b.addParticle(*[1e-3] * 6)
+    b.compress()
+    b.compress()
+    keep = [0, 1, 2, 4, 5, 6, 8]
+    assert b.getSize() == 8
+    assert np.array_equal(b.getCoordinates()[:, :7], c[:, keep])
+    for i in range(8):
+        b.deleteParticleFast(i)
+    b.compress()
+    assert b.getSize() == 0
+    b.addParticle(*[1e-3] * 6)
+    b.compress()
+    assert b.getSize() == 1
