@@ -13,7 +13,7 @@
 //   post     one workgroup per bunch; FFT row / column / row passes over all bunches'
 //            rows and columns (the FFT length is dispatched per workgroup).
 // The per-bunch records and the work items live in device memory and change only when a
-// bunch changes size, so a stretch of tracking (a lattice cell) can be captured once into
+// bunch changes size, weights or constants, so a stretch of tracking (a lattice cell) can be captured once into
 // a hipGraph and replayed.  The work-item size and the tile-deposit item size are chosen
 // by timing the candidates on the batch's own data (autotune).
 //
@@ -71,6 +71,14 @@ void check_same_species(const std::vector<ob_bunch*>& bs) {
   }
 }
 
+// Whether what a record took from its bunch, other than size and coordinates, still holds: the
+// macrosize attribute (set, removed, or its buffer exchanged when the bunch went back to user
+// order), the bunch macrosize, and the kick's constants (RingRF changes the momentum).
+bool record_holds(const BatchBunch& r, const DeviceBunchView& v, const SyncInfo& sy) {
+  return r.v.msize == v.msize && r.macrosize == sy.macrosize && r.r0 == sy.r0 &&
+         r.mass == sy.mass && r.gamma_D == (sy.beta * sy.beta) * pow(sy.gamma, 3);
+}
+
 // (Re)build the device records when the bunches or the tuning changed.
 void build_records(ob_batch* B, bool force) {
   const int nb = (int)B->bunches.size();
@@ -86,9 +94,11 @@ void build_records(ob_batch* B, bool force) {
               ? sc2d_slab_same(B->calcs[b], B->h_bb[b].sd)
               : sc2d_tile_same(B->calcs[b], B->h_bb[b].tg, views[b].n, views[b].msize != nullptr)))
       same = false;
-    if (same) {  // RingRF changed the synchronous momentum: new kick factors
-      const SyncInfo sy = bunch_sync(B->bunches[b]);
-      if (B->h_bb[b].gamma_D != (sy.beta * sy.beta) * pow(sy.gamma, 3)) same = false;
+    if (same && !record_holds(B->h_bb[b], views[b], bunch_sync(B->bunches[b]))) same = false;
+    if (same && !B->calcs.empty()) {
+      BatchBunch now{};
+      sc2d_batch_record(B->calcs[b], now);
+      if (now.n_long_avg != B->h_bb[b].n_long_avg) same = false;
     }
     DenoiseJob dj;  // a denoiser set or cleared since: the moments come from elsewhere
     if (same && !B->calcs.empty() &&
@@ -96,7 +106,7 @@ void build_records(ob_batch* B, bool force) {
       same = false;
   }
   if (same) return;
-  OB_REQUIRE(!B->capturing, "batch: bunch sizes changed during a graph capture");
+  OB_REQUIRE(!B->capturing, "batch: bunch sizes, weights or constants changed during a graph capture");
   B->h_bb.assign(nb, BatchBunch{});
   B->h_items.clear();
   int rows = 0, cols = 0, max_M = 16, slots = 0;
@@ -537,7 +547,8 @@ OB_API int ob_batch_replay(ob_batch* B, int count) {
   OB_REQUIRE(count >= 0, "negative replay count");
   ob::flush(B, false);
   OB_REQUIRE(B->version == B->graph_version,
-             "batch: bunch sizes or buffers changed since the capture; capture again");
+             "batch: bunch sizes, weights, constants or buffers changed since the capture; "
+             "capture again");
   for (int k = 0; k < count; k++) OB_HIP(hipGraphLaunch(B->exec, ob::stream()));
   const double t = ob::bunch_sync(B->leader).time + count * B->graph_dt;
   for (ob_bunch* b : B->bunches) {

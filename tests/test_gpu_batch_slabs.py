@@ -70,3 +70,93 @@ def test_replays_and_a_moved_buffer(weights):
     for a, b in zip(*outs):
         for j in range(6):
             assert rel_l2(a[j], b[j]) < 1e-9, j
+
+
+def _weights(n, seed):
+    return np.random.default_rng(seed).uniform(0.5e8, 1.5e8, n)
+
+
+def _set_weights(bunches, calcs):
+    for k, b in enumerate(bunches):
+        b.setMacroSizes(_weights(b.getSize(), 60 + k))
+
+
+def _drop_weights(bunches, calcs):
+    bunches[1].removePartAttr("macrosize")
+
+
+def _macrosize(bunches, calcs):
+    bunches[0].macroSize(3 * bunches[0].macroSize())
+
+
+def _long_avg(bunches, calcs):
+    calcs[1].setLongAveragingPointsN(7)
+
+
+CHANGES = {"set": _set_weights, "removed": _drop_weights, "macrosize": _macrosize,
+           "long_avg": _long_avg}
+
+
+@pytest.mark.parametrize("grids", [[(64, 64, 32), (200, 150, 16)], [(64, 64, 32), (400, 400, 16)]])
+@pytest.mark.parametrize("change", sorted(CHANGES))
+def test_attributes_changed_between_steps(change, grids):
+    """What a step reads of its bunches and calculators beside the coordinates, changed after
+    the batch has tracked: the next cell is that of the bunches alone, a cell captured before
+    the change is refused, one captured after it repeats the direct one."""
+    from batch import BunchBatch
+    from _obnative import OrbitError
+    sizes = [20_000, 50_001]
+    weighted = change == "removed"
+    alone, acalcs = _setup(sizes, grids)
+    batched, bcalcs = _setup(sizes, grids)
+    if weighted:
+        _set_weights(alone, acalcs)
+        _set_weights(batched, bcalcs)
+    lats = [_lattice(c, 1) for c in acalcs]
+    bb = BunchBatch(batched, bcalcs)
+    lat = _lattice(bb.calculator(), 1)
+    lat.trackBunch(bb.bunch())
+    bb.capture(lambda: lat.trackBunch(bb.bunch()))
+    for b, la in zip(alone, lats):
+        la.trackBunch(b)
+    for bunches, calcs in ((alone, acalcs), (batched, bcalcs)):
+        CHANGES[change](bunches, calcs)
+    with pytest.raises(OrbitError, match="capture again"):
+        bb.replay(1)
+    lat.trackBunch(bb.bunch())
+    bb.capture(lambda: lat.trackBunch(bb.bunch()))
+    bb.replay(1)
+    bb.synchronize()
+    for k, (a, b, la) in enumerate(zip(alone, batched, lats)):
+        la.trackBunch(a)
+        la.trackBunch(a)
+        ref, out = a.getCoordinates(), b.getCoordinates()
+        for j in range(6):
+            assert rel_l2(out[j], ref[j]) < 1e-9, (k, j)
+
+
+def test_weights_of_a_bunch_brought_back_to_user_order():
+    """A weighted bunch that a 3D calculator has left sorted joins a batch; a read puts it back
+    in user order between two cells: coordinates and weights stay together."""
+    import spacecharge
+    from batch import BunchBatch
+    sizes, grids = [30_011, 9000], [(64, 64, 32), (33, 20, 5)]
+    outs = []
+    for read in (False, True):
+        bunches, calcs = _setup(sizes, grids)
+        for k, b in enumerate(bunches):
+            b.setMacroSizes(_weights(sizes[k], k) ** 2 * 1e-8)
+            # (a kick of length 0 sorts the bunch and changes nothing else)
+            spacecharge.SpaceChargeCalc3D(32, 32, 16).trackBunch(b, 0.0)
+        bb = BunchBatch(bunches, calcs)
+        lat = _lattice(bb.calculator(), 1)
+        lat.trackBunch(bb.bunch())
+        if read:
+            for b in bunches:
+                b.getCoordinates()
+        lat.trackBunch(bb.bunch())
+        bb.synchronize()
+        outs.append([b.getCoordinates() for b in bunches])
+    for a, b in zip(*outs):
+        for j in range(6):
+            assert rel_l2(b[j], a[j]) < 1e-9, j
