@@ -83,6 +83,7 @@ class BunchBatch:
 
     def capture(self, fn):
         """Record the batch work done by fn() as a hipGraph (not run: replay runs it)."""
+        self._push_attrs()  # (not possible while the capture runs)
         N.call("ob_batch_capture_begin", self._h)
         try:
             fn()
@@ -90,7 +91,14 @@ class BunchBatch:
             N.call("ob_batch_capture_end", self._h)
 
     def replay(self, count=1):
+        self._push_attrs()
         N.call("ob_batch_replay", self._h, int(count))
+
+
+    def _push_attrs(self):
+        """Particle attributes set one by one (partAttrValue) reach the device."""
+        for b in self.bunches:
+            b._push_attrs()
 
 
 class _BatchBunch:
@@ -134,4 +142,5 @@ class _BatchCalc:
     def trackBunch(self, bunch, length, pipe_radius):
         if bunch is not self._batch._proxy:
             raise ValueError("the batch calculator tracks its own batch only")
+        self._batch._push_attrs()
         N.call("ob_batch_sc2p5drb_track", self._batch._h, float(length), float(pipe_radius))

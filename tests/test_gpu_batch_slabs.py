@@ -135,6 +135,33 @@ def test_attributes_changed_between_steps(change, grids):
             assert rel_l2(out[j], ref[j]) < 1e-9, (k, j)
 
 
+def test_weights_set_one_by_one():
+    """partAttrValue keeps the values on the host until the next step, as for a bunch alone."""
+    from batch import BunchBatch
+    sizes, grids = [3000, 5000], [(32, 32, 16), (16, 16, 8)]
+    alone, acalcs = _setup(sizes, grids)
+    batched, bcalcs = _setup(sizes, grids)
+    lats = [_lattice(c, 1) for c in acalcs]
+    bb = BunchBatch(batched, bcalcs)
+    lat = _lattice(bb.calculator(), 1)
+    for replayed in (False, True):
+        for bunches in (alone, batched):
+            bunches[0].addPartAttr("macrosize")
+            for i in range(sizes[0]):
+                bunches[0].partAttrValue("macrosize", i, 0, 1e7 * (1 + (i + replayed) % 5))
+        if replayed:  # (the attribute is there already: the captured cell takes new values)
+            bb.replay(1)
+        else:
+            lat.trackBunch(bb.bunch())
+            bb.capture(lambda: lat.trackBunch(bb.bunch()))
+        bb.synchronize()
+        for k, (a, b, la) in enumerate(zip(alone, batched, lats)):
+            la.trackBunch(a)
+            ref, out = a.getCoordinates(), b.getCoordinates()
+            for j in range(6):
+                assert rel_l2(out[j], ref[j]) < 1e-9, (replayed, k, j)
+
+
 def test_weights_of_a_bunch_brought_back_to_user_order():
     """A weighted bunch that a 3D calculator has left sorted joins a batch; a read puts it back
     in user order between two cells: coordinates and weights stay together."""
