@@ -262,12 +262,12 @@ __device__ __forceinline__ void lds_fft(double* __restrict__ re, double* __restr
 // Stockham stage (a radix-2 stage at the end for odd powers) serves every stage and both
 // directions, between two LDS buffers with one barrier per stage.
 //   a, b   N points each; the input in a, ready before the caller's barrier;
-//   tw     exp(-2 pi i q / N) at tw[q << tshift] (LDS or global), q < N / 2;
+//   tw     exp(-2 pi i q / N) at tw[q], q < N / 2 (LDS);
 //   sign   +1 forward (exponent -1), -1 inverse.
 // Returns the buffer that holds the result, after a barrier; the other is free.
 template <int N, int NT>
 __device__ __forceinline__ double2* line_fft(double2* a, double2* b, const double2* tw,
-                                             int tshift, double sign) {
+                                             double sign) {
 #pragma clang fp contract(fast)
   constexpr int L = clog2(N);
   static_assert(N >= 8, "line_fft: at least 8 points");
@@ -278,7 +278,7 @@ __device__ __forceinline__ double2* line_fft(double2* a, double2* b, const doubl
     for (int j = threadIdx.x; j < N / 4; j += NT) {
       const int k = j & (Ns - 1);
       const double2 v0 = a[j], x1 = a[j + N / 4], x2 = a[j + N / 2], x3 = a[j + 3 * (N / 4)];
-      double2 w = tw[(k << (L - 2 - ls)) << tshift];
+      double2 w = tw[k << (L - 2 - ls)];
       w.y *= sign;
       const double2 w2 = make_double2(w.x * w.x - w.y * w.y, 2.0 * w.x * w.y);
       const double2 w3 = make_double2(w2.x * w.x - w2.y * w.y, w2.x * w.y + w2.y * w.x);
@@ -305,7 +305,7 @@ __device__ __forceinline__ double2* line_fft(double2* a, double2* b, const doubl
 #pragma unroll 1
     for (int j = threadIdx.x; j < N / 2; j += NT) {
       const double2 v0 = a[j], x1 = a[j + N / 2];
-      double2 w = tw[j << tshift];
+      double2 w = tw[j];
       w.y *= sign;
       const double2 v1 = make_double2(x1.x * w.x - x1.y * w.y, x1.x * w.y + x1.y * w.x);
       b[j] = make_double2(v0.x + v1.x, v0.y + v1.y);
@@ -319,52 +319,76 @@ __device__ __forceinline__ double2* line_fft(double2* a, double2* b, const doubl
   return a;
 }
 
-// The LDS of a line_fft kernel: two line buffers and, up to 1024 points, the twiddles, loaded
-// beside the kernel's data at its start and stored with it (commit, before the barrier).
-__host__ __device__ constexpr bool line_tw_in_lds(int n) { return n <= 1024; }
-__host__ __device__ constexpr size_t line_lds_bytes(int n) {
-  return sizeof(double2) * (2 * n + (line_tw_in_lds(n) ? n / 2 : 0));
+// The line of a one-line kernel.  Up to kLineTwoBuffers points it is transformed by line_fft
+// between two buffers, with the twiddles in LDS (loaded beside the kernel's data at its start
+// and stored with it: commit, before the barrier); longer lines by lds_fft in place, real and
+// imaginary parts apart, in less than half the LDS.  The line lies where two buffers leave a
+// CU one workgroup and the solve has more of them than the chip has CUs: a step on 1000 x 1000
+// nodes (2048 points) took 140 us with two buffers and takes 116 in place, on 600 x 520 124 and
+// 103; on 500 x 500 (1024 points) both take 80.7.  Two buffers of 4096 points beside the post
+// pass would be more LDS than a workgroup has.
+constexpr int kLineTwoBuffers = 1024;
+__host__ __device__ constexpr bool line_two_buffers(int n) { return n <= kLineTwoBuffers; }
+__host__ __device__ constexpr size_t line_lds_bytes(int n, bool two) {
+  return two ? sizeof(double2) * (2 * n + n / 2) : sizeof(double) * 2 * fft_line(n);
 }
-template <int N, int NT>
+__host__ __device__ constexpr size_t line_lds_bytes(int n) {
+  return line_lds_bytes(n, line_two_buffers(n));
+}
+template <int N, int NT, bool TWO = line_two_buffers(N)>
 struct LineFft {
-  static constexpr bool LDS = line_tw_in_lds(N);
-  static constexpr int CNT = N / 2, IT = LDS ? (CNT + NT - 1) / NT : 1;
+  static constexpr int CNT = N / 2, IT = (CNT + NT - 1) / NT;
   double2 *a, *b;
   const double2* tw;
-  int tshift;
   double2 v[IT];
   __device__ __forceinline__ LineFft(double* lds, const double2* __restrict__ tw_, int nmax)
-      : a((double2*)lds), b((double2*)lds + N), tw(tw_) {
-    tshift = 0;
+      : a((double2*)lds), b((double2*)lds + N) {
+    int tshift = 0;
     while ((N << tshift) < nmax) tshift++;
-    if constexpr (LDS) {
 #pragma unroll
-      for (int u = 0; u < IT; u++) {
-        const int i = (int)threadIdx.x + u * NT;
-        v[u] = tw_[(i < CNT ? i : 0) << tshift];
-      }
+    for (int u = 0; u < IT; u++) {
+      const int i = (int)threadIdx.x + u * NT;
+      v[u] = tw_[(i < CNT ? i : 0) << tshift];
     }
   }
+  __device__ __forceinline__ void set(int i, double2 z) { a[i] = z; }
+  __device__ __forceinline__ double2 get(int i) const { return a[i]; }
   __device__ __forceinline__ void commit() {
-    if constexpr (LDS) {
-      double2* t = b + N;
+    double2* t = b + N;
 #pragma unroll
-      for (int u = 0; u < IT; u++) {
-        const int i = (int)threadIdx.x + u * NT;
-        if (i < CNT) t[i] = v[u];
-      }
-      tw = t;
-      tshift = 0;
+    for (int u = 0; u < IT; u++) {
+      const int i = (int)threadIdx.x + u * NT;
+      if (i < CNT) t[i] = v[u];
     }
+    tw = t;
   }
-  // The transform of the line in a (see line_fft); afterwards a holds the result.
+  // The transform of the line, between the caller's barrier and one of its own.
+  __device__ __forceinline__ void forward() { run(1.0); }
+  __device__ __forceinline__ void inverse() { run(-1.0); }
   __device__ __forceinline__ void run(double sign) {
-    double2* r = line_fft<N, NT>(a, b, tw, tshift, sign);
+    double2* r = line_fft<N, NT>(a, b, tw, sign);
     if (r != a) {
       b = a;
       a = r;
     }
   }
+};
+template <int N, int NT>
+struct LineFft<N, NT, false> {
+  static constexpr int LINE = fft_line(N);  // evaluated at compile time
+  double *re, *im;
+  const double2* tw;
+  int nmax;
+  __device__ __forceinline__ LineFft(double* lds, const double2* __restrict__ tw_, int nmax_)
+      : re(lds), im(lds + LINE), tw(tw_), nmax(nmax_) {}
+  __device__ __forceinline__ void set(int i, double2 z) {
+    re[i] = z.x;
+    im[i] = z.y;
+  }
+  __device__ __forceinline__ double2 get(int i) const { return make_double2(re[i], im[i]); }
+  __device__ __forceinline__ void commit() {}
+  __device__ __forceinline__ void forward() { lds_fft<N, 1, NT, -1>(re, im, 1, N, tw, nmax); }
+  __device__ __forceinline__ void inverse() { lds_fft<N, 1, NT, +1>(re, im, 1, N, tw, nmax); }
 };
 
 // ---- transforms with register-resident ends ------------------------------------------

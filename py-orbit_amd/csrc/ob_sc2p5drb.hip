@@ -1063,7 +1063,7 @@ __global__ __launch_bounds__(kSetupThreads) void sc2d_post(SC2DParams P, SC2DSta
 // (a) two real rows per complex FFT along y, r2c split.  rows >= nrows_in are zero;
 // columns >= ncols_in are zero (padding).  out: spectrum [*][H] complex (H = N/2+1).
 // blk: row pair (rows 2 blk, 2 blk + 1).
-template <int N>
+template <int N, bool TWO = line_two_buffers(N)>
 __device__ __forceinline__ void rows_r2c_body(const double* __restrict__ in, int nrows_in,
                                               int ncols_in, int ld_in,
                                               double2* __restrict__ out,
@@ -1071,17 +1071,17 @@ __device__ __forceinline__ void rows_r2c_body(const double* __restrict__ in, int
                                               const SC2DState* st, int blk) {
   if (st && st->skip) return;
   extern __shared__ double sm[];
-  LineFft<N, kFFTThreads> F(sm, tw, nmax);
+  LineFft<N, kFFTThreads, TWO> F(sm, tw, nmax);
   const int r0 = 2 * blk, r1 = r0 + 1;
   for (int j = threadIdx.x; j < N; j += kFFTThreads)
-    F.a[j] = make_double2((j < ncols_in) ? in[(int64_t)r0 * ld_in + j] : 0.0,
-                          (j < ncols_in && r1 < nrows_in) ? in[(int64_t)r1 * ld_in + j] : 0.0);
+    F.set(j, make_double2((j < ncols_in) ? in[(int64_t)r0 * ld_in + j] : 0.0,
+                          (j < ncols_in && r1 < nrows_in) ? in[(int64_t)r1 * ld_in + j] : 0.0));
   F.commit();
   __syncthreads();
-  F.run(1.0);
+  F.forward();
   constexpr int H = N / 2 + 1;
   for (int k = threadIdx.x; k < H; k += kFFTThreads) {
-    const double2 z = F.a[k], n = F.a[(N - k) & (N - 1)];
+    const double2 z = F.get(k), n = F.get((N - k) & (N - 1));
     out[(int64_t)r0 * H + k] = make_double2((z.x + n.x) * 0.5, (z.y - n.y) * 0.5);
     if (r1 < nrows_in)
       out[(int64_t)r1 * H + k] = make_double2((z.y + n.y) * 0.5, -(z.x - n.x) * 0.5);
@@ -1102,7 +1102,10 @@ __global__ __launch_bounds__(kFFTThreads) void fft_rows_r2c(const double* __rest
 // independent halves side by side (z line density and derivative; rho moments and kick
 // factors).  All only read rho; the post pass writes the state's kick factors, z line
 // density and derivative, which the column pass after this launch (scale_coeff) and the
-// next map kernel read.  One launch fewer per step.
+// next map kernel read.  One launch fewer per step.  1024 points go in place here: two buffers
+// and the post pass's LDS leave a CU one workgroup (512 x 512 nodes, 258 workgroups: 15.0 us,
+// in place 11.4; 500 x 500 11.8 both).
+constexpr bool post_two_buffers(int n) { return n <= 512; }
 template <int N>
 __global__ __launch_bounds__(kFFTThreads) void fft_rows_r2c_post(
     const double* __restrict__ rho, int nrows_in, int ncols_in, double2* __restrict__ out,
@@ -1110,7 +1113,8 @@ __global__ __launch_bounds__(kFFTThreads) void fft_rows_r2c_post(
     double* __restrict__ zg, double* __restrict__ zd, Tile2D tg, int zrows, int moments) {
   const int rb = (nrows_in + 1) / 2;
   if ((int)blockIdx.x < rb) {
-    rows_r2c_body<N>(rho, nrows_in, ncols_in, ncols_in, out, tw, nmax, st, blockIdx.x);
+    rows_r2c_body<N, post_two_buffers(N)>(rho, nrows_in, ncols_in, ncols_in, out, tw, nmax, st,
+                                          blockIdx.x);
     return;
   }
   // two more workgroups: the line density part and the moments part of the post pass
@@ -1136,7 +1140,8 @@ __device__ __forceinline__ void rows_sum_body(const SlabDep& D, double* __restri
   extern __shared__ double sm[];
   __shared__ double red[THREADS / 64][5];
   constexpr int H = N / 2 + 1;
-  double* acc = sm + line_lds_bytes(N) / sizeof(double);
+  constexpr int ACC = (int)(line_lds_bytes(N) / sizeof(double));  // evaluated at compile time
+  double* acc = sm + ACC;
   LineFft<N, THREADS> F(sm, tw, nmax);
   constexpr int NG = THREADS / kSumGroups;
   const int grp = (int)threadIdx.x / NG, l = (int)threadIdx.x % NG;
@@ -1152,7 +1157,7 @@ __device__ __forceinline__ void rows_sum_body(const SlabDep& D, double* __restri
       rho[(int64_t)r * ny + j] = t;
       moment_add(mom, t, r, j, xMin, dx);
     }
-    F.a[j] = make_double2(t, 0.0);
+    F.set(j, make_double2(t, 0.0));
   }
   const int nw = (ny + 63) / 64;  // waves that hold nodes
   if (mpart && (int)threadIdx.x < 64 * nw) {
@@ -1167,8 +1172,8 @@ __device__ __forceinline__ void rows_sum_body(const SlabDep& D, double* __restri
     for (int w = 0; w < nw; w++) t += red[w][threadIdx.x];
     mpart[(size_t)r * 5 + threadIdx.x] = t;
   }
-  F.run(1.0);
-  for (int k = threadIdx.x; k < H; k += THREADS) out[(int64_t)r * H + k] = F.a[k];
+  F.forward();
+  for (int k = threadIdx.x; k < H; k += THREADS) out[(int64_t)r * H + k] = F.get(k);
 }
 
 template <int N>
@@ -1207,13 +1212,13 @@ __device__ __forceinline__ void cols_body(double2* __restrict__ spec, int nrows_
 #pragma unroll
   for (int u = 0; u < CI; u++) {
     const int i = (int)threadIdx.x + u * kFFTThreads;
-    if (i < N) F.a[i] = i < nrows_in ? cv[u] : make_double2(0.0, 0.0);
+    if (i < N) F.set(i, i < nrows_in ? cv[u] : make_double2(0.0, 0.0));
   }
   F.commit();
   __syncthreads();
-  F.run(1.0);
+  F.forward();
   if constexpr (GREEN) {
-    for (int i = threadIdx.x; i < N; i += kFFTThreads) ghat_t[(int64_t)k * N + i] = F.a[i];
+    for (int i = threadIdx.x; i < N; i += kFFTThreads) ghat_t[(int64_t)k * N + i] = F.get(i);
     return;
   } else {
     // PoissonSolverFFT2D.cc:215-236: Green spectrum rescaled to the rho grid step
@@ -1222,15 +1227,15 @@ __device__ __forceinline__ void cols_body(double2* __restrict__ spec, int nrows_
     for (int u = 0; u < CI; u++) {
       const int i = (int)threadIdx.x + u * kFFTThreads;
       if (i >= N) continue;
-      const double2 g = gv[u], z = F.a[i];
+      const double2 g = gv[u], z = F.get(i);
       const double gr_re = ((i == 0 && k == 0) ? (g.x + s * npad) : g.x) - s;
       const double gr_im = g.y;
-      F.a[i] = make_double2(z.x * gr_re - z.y * gr_im, z.x * gr_im + z.y * gr_re);
+      F.set(i, make_double2(z.x * gr_re - z.y * gr_im, z.x * gr_im + z.y * gr_re));
     }
     __syncthreads();
-    F.run(-1.0);
+    F.inverse();
     for (int i = threadIdx.x; i < nrows_in; i += kFFTThreads)
-      spec[(int64_t)i * H + k] = F.a[i];
+      spec[(int64_t)i * H + k] = F.get(i);
   }
 }
 
@@ -1286,14 +1291,14 @@ __device__ __forceinline__ void rows_c2r_body(const double2* __restrict__ spec, 
       b.y = 0.0;
     }
     // Z = X0 + i X1 with X(N-k) = conj(X(k))
-    F.a[k] = make_double2(a.x - b.y, a.y + b.x);
-    if (k > 0 && k < N / 2) F.a[N - k] = make_double2(a.x + b.y, b.x - a.y);
+    F.set(k, make_double2(a.x - b.y, a.y + b.x));
+    if (k > 0 && k < N / 2) F.set(N - k, make_double2(a.x + b.y, b.x - a.y));
   }
   F.commit();
   __syncthreads();
-  F.run(-1.0);
+  F.inverse();
   for (int j = threadIdx.x; j < ncols_out; j += kFFTThreads) {
-    const double2 z = F.a[j];
+    const double2 z = F.get(j);
     out[(int64_t)r0 * ld_out + j] = denom * z.x;
     if (has1) out[(int64_t)r1 * ld_out + j] = denom * z.y;
   }
@@ -1556,7 +1561,13 @@ struct ob_sc2p5d : ob_sc2p5drb {};
 namespace ob {
 namespace {
 template <int N>
-size_t fft_lds() { return line_lds_bytes(N); }
+constexpr size_t fft_lds() { return line_lds_bytes(N); }
+
+// A workgroup's LDS, and what sc2d_post_body declares of it: the kernels that run the post pass
+// beside transforms have both, whichever a workgroup does.
+constexpr size_t kLdsPerGroup = 160 * 1024;
+constexpr size_t kPostLds =
+    sizeof(double) * (kMaxZBinsLDS + kSetupThreads + kSetupThreads / 64);
 
 // Dynamic LDS above 64 KiB has to be allowed per kernel; done once per instantiation.
 template <typename K>
@@ -1636,15 +1647,17 @@ void launch_fft_pipeline(ob_sc2p5drb* c, SC2DState* st, double* phi,
     dispatch_pow2(c->M1, [&](auto NC) {
       constexpr int N = decltype(NC)::value;
       if constexpr (N >= 8) {
+        constexpr size_t lds = line_lds_bytes(N, post_two_buffers(N));
+        static_assert(lds + kPostLds <= kLdsPerGroup, "row pass: LDS");
         static bool ready = false;
         if (!ready) {
-          allow_lds(fft_rows_r2c_post<N>, fft_lds<N>());
+          allow_lds(fft_rows_r2c_post<N>, lds);
           ready = true;
         }
         ob::ProfScope ps_("fft_rows_r2c_post");
         OB_REQUIRE(!post->P.plain, "2.5D post pass: the split form is for SpaceChargeCalc2p5Drb");
         hipLaunchKernelGGL(fft_rows_r2c_post<N>, dim3((c->nx + 1) / 2 + 2), dim3(kFFTThreads),
-                           fft_lds<N>(), stream(), c->rho, c->nx, c->ny, c->spec, c->tw, c->nmax,
+                           lds, stream(), c->rho, c->nx, c->ny, c->spec, c->tw, c->nmax,
                            post->P, st, c->zg, c->zd, post->tg, post->zrows, post->moments);
       }
     });
@@ -1662,13 +1675,14 @@ void launch_slab_solve(ob_sc2p5drb* c, const SC2DParams& P, const SlabDep& D, do
   dispatch_pow2(c->M1, [&](auto NC) {
     constexpr int N = decltype(NC)::value;
     if constexpr (N >= 8 && N <= 2 * kSlabMaxNy) {
-      const size_t lds = line_lds_bytes(N) + sizeof(double) * kSumGroups * c->ny;
+      constexpr size_t most = fft_lds<N>() + sizeof(double) * kSumGroups * (N / 2 + 1);
+      static_assert(most + kPostLds + sizeof(double) * 5 * (kSumThreads / 64) <= kLdsPerGroup,
+                    "row pass with the copies: LDS");
+      const size_t lds = fft_lds<N>() + sizeof(double) * kSumGroups * c->ny;
       static bool ready = false;
       if (!ready) {
         OB_HIP(hipFuncSetAttribute((const void*)fft_rows_sum_post<N>,
-                                   hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   (int)(line_lds_bytes(N) +
-                                         sizeof(double) * kSumGroups * (N / 2 + 1))));
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)most));
         ready = true;
       }
       ob::ProfScope ps_("fft_rows_sum_post");
@@ -1683,6 +1697,7 @@ void launch_slab_solve(ob_sc2p5drb* c, const SC2DParams& P, const SlabDep& D, do
     if constexpr (N >= 8) {
       static bool ready = false;
       if (!ready) {
+        static_assert(fft_lds<N>() + kPostLds <= kLdsPerGroup, "column pass: LDS");
         allow_lds(fft_cols_post<N>, fft_lds<N>());
         ready = true;
       }

@@ -53,6 +53,31 @@ def test_step_on_every_split(grid, weights):
         assert rel_l2(out[k] - c[k], ob.coords[k] - c[k]) < 1e-10, k
 
 
+# padded lengths 1024 to 4096 (the longest lines transform in place), on an axis of the copies'
+# split, of the tile sort and of both
+@pytest.mark.parametrize("grid", [(1100, 40, 64), (40, 1100, 64), (1025, 3, 1), (3, 2048, 4096),
+                                  (2048, 9, 8), (1030, 1024, 16), (600, 260, 8)])
+@pytest.mark.parametrize("plain", [False, True])
+def test_step_on_long_axes(grid, plain):
+    import spacecharge
+    n = 30_011
+    c = _coords(n, 4)
+    b, ob = _bunches(c)
+    if plain:
+        calc, ocalc = spacecharge.SpaceChargeCalc2p5D(*grid), O.SC2p5D(*grid)
+    else:
+        calc, ocalc = spacecharge.SpaceChargeCalc2p5Drb(*grid), O.SC2p5Drb(*grid)
+    args = (0.5,) if plain else (0.5, 0.1)
+    calc.trackBunch(b, *args)
+    ocalc.trackBunch(ob, *args)
+    out = b.getCoordinates()
+    for g in range(3):
+        a = (calc.getRhoGrid(), calc.getPhiGrid(), calc.getLongGrid())[g].array()
+        assert rel_l2(a, ocalc.grid(g)[0]) < 1e-12, g
+    for k in (1, 3):
+        assert rel_l2(out[k] - c[k], ob.coords[k] - c[k]) < 1e-10, k
+
+
 @pytest.mark.parametrize("n", [2, 3, 1023, 1024, 1025, 2049, 262_145, 600_003])
 def test_bunch_sizes_on_one_calculator(n):
     """Growing and shrinking bunches: the copies of an earlier, larger step are not read."""
