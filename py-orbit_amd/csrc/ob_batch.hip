@@ -333,6 +333,14 @@ void batch_flush_owner(ob_batch* B) {
 
 std::vector<ob_batch*> g_live_batches;
 
+void batch_flush_kicks(ob_sc2p5drb* const* calcs, size_t n) {
+  for (ob_batch* B : g_live_batches)
+    if (B->kick.active && std::any_of(calcs, calcs + n, [&](ob_sc2p5drb* c) {
+          return std::find(B->calcs.begin(), B->calcs.end(), c) != B->calcs.end();
+        }))
+      flush(B, false);
+}
+
 void batch_forget_calc(ob_sc2p5drb* c) {
   for (ob_batch* B : g_live_batches) {
     if (std::find(B->calcs.begin(), B->calcs.end(), c) == B->calcs.end()) continue;
@@ -454,6 +462,8 @@ OB_API int ob_batch_sc2p5drb_track(ob_batch* B, double length, double pipe_radiu
     ob::autotune(B);
   }
   ob::flush(B, true);
+  // (a capture began with every other kick of these calculators applied)
+  if (!B->capturing) ob::sc2d_flush_kicks(B->calcs.data(), B->calcs.size());
   std::vector<ob::DenoiseJob> jobs;
   for (ob_sc2p5drb* c : B->calcs) {
     ob::DenoiseJob j;
@@ -507,6 +517,7 @@ OB_API int ob_batch_capture_begin(ob_batch* B) {
     ob::autotune(B);
   }
   ob::flush(B, false);  // nothing pending inside the graph's boundaries
+  ob::sc2d_flush_kicks(B->calcs.data(), B->calcs.size());
   OB_HIP(hipStreamSynchronize(ob::stream()));
   if (B->exec) {
     OB_HIP(hipGraphExecDestroy(B->exec));
@@ -549,6 +560,7 @@ OB_API int ob_batch_replay(ob_batch* B, int count) {
   OB_REQUIRE(B->version == B->graph_version,
              "batch: bunch sizes, weights, constants or buffers changed since the capture; "
              "capture again");
+  ob::sc2d_flush_kicks(B->calcs.data(), B->calcs.size());
   for (int k = 0; k < count; k++) OB_HIP(hipGraphLaunch(B->exec, ob::stream()));
   const double t = ob::bunch_sync(B->leader).time + count * B->graph_dt;
   for (ob_bunch* b : B->bunches) {

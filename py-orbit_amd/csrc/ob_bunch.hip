@@ -416,16 +416,17 @@ void bunch_set_owner(ob_bunch* b, ob_batch* owner) { b->owner = owner; }
 
 std::vector<ob_bunch*> g_live_bunches;
 
-// A calculator is about to write or free its buffers: apply every waiting space-charge kick that
-// reads them (the kick belongs to a trackBunch call that has already happened).
-void flush_kicks_reading(const void* state) {
-  const double want = ptr_bits(state);
+// Calculators are about to write or free their buffers: apply every waiting space-charge kick
+// that reads them (the kick belongs to a trackBunch call that has already happened).
+void flush_kicks_reading(const void* const* states, size_t n) {
+  auto among = [&](const void* p) { return std::find(states, states + n, p) != states + n; };
   for (ob_bunch* b : g_live_bunches) {
-    bool reads = b->has_tile_kick && b->tile_kick.k.phi == state;
+    bool reads = b->has_tile_kick && among(b->tile_kick.k.phi);
     for (size_t j = 0; j < b->queue.size() && !reads; j++) {
       const Op& op = b->queue[j];
-      reads = (op.kind == OP_SC2P5DRB_KICK || op.kind == OP_SC3D_KICK) &&
-              std::memcmp(&op.p[0], &want, sizeof(double)) == 0;
+      const void* p;
+      std::memcpy(&p, &op.p[0], sizeof(p));
+      reads = (op.kind == OP_SC2P5DRB_KICK || op.kind == OP_SC3D_KICK) && among(p);
     }
     if (!reads) continue;
     try {

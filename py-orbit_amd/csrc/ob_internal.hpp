@@ -379,9 +379,15 @@ namespace ob {
 // A batched bunch's flush applies the whole batch's pending work (ob_batch.hip).
 void bunch_set_owner(ob_bunch* b, ob_batch* owner);
 void batch_flush_owner(ob_batch* B);
-// Live bunches; apply the queued SC kicks whose op p[0] is `state` (before it is freed).
+// Live bunches; apply the waiting SC kicks that read one of the n `states` (a 2.5D calculator's
+// state, a 3D or slice calculator's phi) before it is written or freed.
 extern std::vector<ob_bunch*> g_live_bunches;
-void flush_kicks_reading(const void* state);
+void flush_kicks_reading(const void* const* states, size_t n);
+inline void flush_kicks_reading(const void* state) { flush_kicks_reading(&state, 1); }
+// The same for 2.5D calculators, with the kicks that wait on batches.
+void sc2d_flush_kicks(ob_sc2p5drb* const* calcs, size_t n);
+// Batches with a waiting kick of one of the calculators apply it.
+void batch_flush_kicks(ob_sc2p5drb* const* calcs, size_t n);
 // A 2.5D calculator is going away: batches using it apply their pending kicks and drop it.
 void batch_forget_calc(ob_sc2p5drb* c);
 // Queue one map of the public op list (ob_map_op) exactly as its entry point does.

@@ -1957,6 +1957,13 @@ bool sc2d_tile_same(ob_sc2p5drb* c, const Tile2D& t, int64_t n, bool per_particl
 
 void sc2d_mark_tracked(ob_sc2p5drb* c) { c->tracked = true; }
 
+void sc2d_flush_kicks(ob_sc2p5drb* const* calcs, size_t n) {
+  batch_flush_kicks(calcs, n);
+  std::vector<const void*> states(n);
+  for (size_t k = 0; k < n; k++) states[k] = calcs[k]->st;
+  flush_kicks_reading(states.data(), n);
+}
+
 int sc2d_read_status(ob_sc2p5drb* c) {
   int v = 0;
   OB_HIP(hipMemcpy(&v, &c->st->status, sizeof(int), hipMemcpyDeviceToHost));
@@ -2213,6 +2220,7 @@ void sc2d_track(ob_sc2p5drb* c, ob_bunch* b, double length, double pipe_radius,
   if (n < 2) return;  // :112-113 (2p5D :79-80)
   hipStream_t s = stream();
   const int nblk = bunch_flush(b, c->partials);
+  sc2d_flush_kicks(&c, 1);  // (other bunches' waiting kicks)
   DeviceBunchView v = bunch_device_view(b);
   const SyncInfo sy = bunch_sync(b);
   SC2DParams P;
@@ -2370,6 +2378,7 @@ OB_API int ob_sc2p5drb_find_potential(ob_sc2p5drb* c, const double* rho, double 
   OB_REQUIRE(dx > 0.0 && dy > 0.0, "PoissonSolverFFT2D: empty grid");
   OB_REQUIRE(fabs(c->dx_solver / c->dy_solver - dx / dy) <= 1e-8,  // :176-210
              "PoissonSolverFFT2D: the grid sizes or shape are different");
+  ob::sc2d_flush_kicks(&c, 1);
   hipStream_t s = ob::stream();
   OB_HIP(hipStreamSynchronize(s));
   ob::SC2DState h;

@@ -133,3 +133,61 @@ def test_boundary_sizes(npts, nm):
     assert rel_l2(calc.getPhiGrid().array(), ocalc.grid(1)[0]) < bar
     for k in (1, 3):
         assert rel_l2(out[k] - c[k], ob.coords[k] - c[k]) < 100 * bar
+
+
+SLABS, TILES = (32, 24, 8), (40, 600, 8)
+
+
+@pytest.mark.parametrize("between,grid,plain", [
+    ("bunch", SLABS, False), ("bunch", TILES, False), ("bunch", SLABS, True),
+    ("bunch", TILES, True), ("potential", SLABS, False), ("potential", TILES, False),
+    ("batch", SLABS, False), ("batch_first", SLABS, False), ("replay", SLABS, False)])
+def test_kick_waits_while_its_calculator_is_used(between, grid, plain):
+    """A calculator writes its state, potential and line density again (another bunch's step,
+    findPotential, a batch it belongs to) while a kick of it still waits: the kick is that of
+    its own step, as when the bunch is read in between."""
+    import spacecharge
+    import teapot_base as TPB
+    import _obnative as N
+    from batch import BunchBatch
+    from workloads import PIPE_RADIUS
+    outs = []
+    for eager in (False, True):
+        first, second = (_bunches(_coords(n, 90, ax))[0]
+                         for n, ax in ((9001, 3e-3), (20_011, 6e-3)))
+        calc = (spacecharge.SpaceChargeCalc2p5D(*grid) if plain
+                else spacecharge.SpaceChargeCalc2p5Drb(*grid))
+        step = ((lambda b: calc.trackBunch(b, 0.5)) if plain
+                else (lambda b: calc.trackBunch(b, 0.5, PIPE_RADIUS)))
+        read = (lambda b: b.getCoordinates()) if eager else (lambda b: None)
+        if between == "bunch":
+            step(first)
+            TPB.drift(first, 0.3)
+            read(first)
+            step(second)
+        elif between == "potential":
+            step(first)
+            read(first)
+            rho = np.random.default_rng(1).uniform(0, 1e9, grid[:2])
+            phi = np.empty_like(rho)  # (the solver's own box)
+            N.call("ob_sc2p5drb_find_potential", calc._h, N.dptr(rho), -1.0, 1.0, -1.0, 1.0,
+                   N.dptr(phi))
+        else:
+            bb = BunchBatch([second], [calc])
+            if between == "replay":
+                bb.capture(lambda: bb.calculator().trackBunch(bb.bunch(), 0.5, PIPE_RADIUS))
+            if between == "batch_first":
+                bb.calculator().trackBunch(bb.bunch(), 0.5, PIPE_RADIUS)
+                read(second)
+                step(first)
+            else:
+                step(first)
+                read(first)
+                if between == "replay":
+                    bb.replay(1)
+                else:
+                    bb.calculator().trackBunch(bb.bunch(), 0.5, PIPE_RADIUS)
+        outs.append([first.getCoordinates(), second.getCoordinates()])
+    for lazy, now in zip(*outs):
+        for k in range(6):
+            assert rel_l2(lazy[k], now[k]) < 1e-12, k
