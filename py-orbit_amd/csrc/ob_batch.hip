@@ -51,7 +51,7 @@ struct ob_batch {
   int version = 0;                     // incremented by every rebuild of the records
   // graph
   int graph_version = -1;              // records version the graph was captured with
-  bool capturing = false;
+  bool capturing = false, put_off = false;
   hipGraphExec_t exec = nullptr;
   double graph_dt = 0.0;               // synchronous time advanced by one replay
 };
@@ -333,6 +333,31 @@ void batch_flush_owner(ob_batch* B) {
 
 std::vector<ob_batch*> g_live_batches;
 
+namespace {
+std::vector<std::function<void()>> g_put_off;
+
+// The recording of B ends: the graph (null if the recording failed), then what was put off.
+hipError_t end_capture(ob_batch* B, hipGraph_t* g) {
+  *g = nullptr;
+  const hipError_t e = hipStreamEndCapture(stream(), g);
+  B->capturing = false;
+  std::vector<std::function<void()>> ends;
+  ends.swap(g_put_off);
+  for (auto& f : ends) f();
+  return e;
+}
+}  // namespace
+
+bool put_off_end(std::function<void()> end) {
+  if (std::none_of(g_live_batches.begin(), g_live_batches.end(),
+                   [](const ob_batch* B) { return B->capturing; }))
+    return false;
+  g_put_off.push_back(std::move(end));
+  return true;
+}
+
+bool batch_put_off(const ob_batch* B) { return B && B->put_off; }
+
 void batch_flush_kicks(ob_sc2p5drb* const* calcs, size_t n) {
   for (ob_batch* B : g_live_batches)
     if (B->kick.active && std::any_of(calcs, calcs + n, [&](ob_sc2p5drb* c) {
@@ -400,7 +425,18 @@ OB_API int ob_batch_create(ob_bunch** bunches, int nb, ob_batch** out) {
 
 OB_API int ob_batch_destroy(ob_batch* B) {
   OB_TRY if (!B) return 0;
-  if (!B->capturing) ob::flush(B, false);  // nothing pending is lost
+  if (B->capturing) {  // the recording goes with it
+    hipGraph_t g = nullptr;
+    (void)ob::end_capture(B, &g);
+    if (g) (void)hipGraphDestroy(g);
+    B->queue.clear();
+    B->kick = ob::BatchKick{};
+  }
+  if (ob::put_off_end([=] { (void)ob_batch_destroy(B); })) {
+    B->put_off = true;
+    return 0;
+  }
+  ob::flush(B, false);  // nothing pending is lost
   auto& lb = ob::g_live_batches;
   lb.erase(std::remove(lb.begin(), lb.end(), B), lb.end());
   for (ob_bunch* b : B->bunches) ob::bunch_set_owner(b, nullptr);
@@ -536,13 +572,11 @@ OB_API int ob_batch_capture_end(ob_batch* B) {
   try {
     ob::flush(B, false);
   } catch (...) {
-    (void)hipStreamEndCapture(ob::stream(), &g);
+    (void)ob::end_capture(B, &g);
     if (g) (void)hipGraphDestroy(g);
-    B->capturing = false;
     throw;
   }
-  OB_HIP(hipStreamEndCapture(ob::stream(), &g));
-  B->capturing = false;
+  OB_HIP(ob::end_capture(B, &g));
   OB_HIP(hipGraphInstantiate(&B->exec, g, nullptr, nullptr, 0));
   OB_HIP(hipGraphDestroy(g));
   B->graph_dt = ob::bunch_sync(B->leader).time - B->graph_dt;

@@ -483,6 +483,7 @@ OB_API int ob_boundary2d_create_shaped(int nPoints, int nModes, const char* shap
 
 OB_API int ob_boundary2d_destroy(ob_boundary2d* b) {
   OB_TRY if (!b) return 0;
+  if (ob::put_off_end([=] { (void)ob_boundary2d_destroy(b); })) return 0;
   (void)hipStreamSynchronize(ob::stream());  // queued steps may read its arrays
   for (void* p : {(void*)b->d_bx, (void*)b->d_by, (void*)b->d_lsq, (void*)b->d_geo,
                   (void*)b->d_work3})

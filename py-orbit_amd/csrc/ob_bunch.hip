@@ -608,7 +608,9 @@ OB_API int ob_bunch_create(ob_bunch** out) {
 
 OB_API int ob_bunch_destroy(ob_bunch* b) {
   OB_TRY if (!b) return 0;
-  OB_REQUIRE(b->owner == nullptr, "bunch belongs to a batch: destroy the batch first");
+  OB_REQUIRE(b->owner == nullptr || ob::batch_put_off(b->owner),
+             "bunch belongs to a batch: destroy the batch first");
+  if (ob::put_off_end([=] { (void)ob_bunch_destroy(b); })) return 0;
   auto& lb = ob::g_live_bunches;
   lb.erase(std::remove(lb.begin(), lb.end(), b), lb.end());
   (void)hipStreamSynchronize(ob::stream());

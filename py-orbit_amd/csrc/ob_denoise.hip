@@ -1475,6 +1475,7 @@ OB_API int ob_dn_create(int H, int W, int max_batch, ob_denoiser** out) {
 
 OB_API int ob_dn_destroy(ob_denoiser* d) {
   OB_TRY if (!d) return 0;
+  if (ob::put_off_end([=] { (void)ob_dn_destroy(d); })) return 0;
   (void)hipStreamSynchronize(ob::stream());
   for (void* p : {(void*)d->w, (void*)d->g, (void*)d->m, (void*)d->v, (void*)d->pf, (void*)d->pt,
                   (void*)d->gcat4, (void*)d->gcat5, (void*)d->gtmp0, (void*)d->gtmp1,

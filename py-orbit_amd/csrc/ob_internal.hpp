@@ -6,6 +6,8 @@
 #include <cfloat>
 #include <cstdint>
 #include <cstring>
+#include <functional>
+#include <functional>
 #include <string>
 #include <vector>
 
@@ -376,9 +378,14 @@ void bunch_copy_kinematics(ob_bunch* dst, const ob_bunch* src);
 }  // namespace ob
 struct ob_batch;
 namespace ob {
+// While a batch records a graph nothing may wait for the stream or free memory.  An object that
+// goes meanwhile (Python collects cycles at any time) is put off: end() runs when the recording
+// ends.  False: nothing is being recorded, the caller goes on.
+bool put_off_end(std::function<void()> end);
 // A batched bunch's flush applies the whole batch's pending work (ob_batch.hip).
 void bunch_set_owner(ob_bunch* b, ob_batch* owner);
 void batch_flush_owner(ob_batch* B);
+bool batch_put_off(const ob_batch* B);  // its end has been put off
 // Live bunches; apply the waiting SC kicks that read one of the n `states` (a 2.5D calculator's
 // state, a 3D or slice calculator's phi) before it is written or freed.
 extern std::vector<ob_bunch*> g_live_bunches;

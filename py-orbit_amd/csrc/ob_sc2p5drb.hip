@@ -2307,6 +2307,7 @@ OB_API int ob_sc2p5drb_create(int nx, int ny, int nz, double xy_ratio, ob_sc2p5d
 OB_API int ob_sc2p5drb_destroy(ob_sc2p5drb* c) {
   OB_TRY if (!c) return 0;
   OB_REQUIRE(!c->plain, "not a SpaceChargeCalc2p5Drb handle");
+  if (ob::put_off_end([=] { (void)ob_sc2p5drb_destroy(c); })) return 0;
   ob::sc2d_destroy(c);
   OB_CATCH
 }
@@ -2327,6 +2328,7 @@ OB_API int ob_sc2p5d_create(int nx, int ny, int nz, double xy_ratio, ob_sc2p5d**
 OB_API int ob_sc2p5d_destroy(ob_sc2p5d* c) {
   OB_TRY if (!c) return 0;
   OB_REQUIRE(c->plain, "not a SpaceChargeCalc2p5D handle");
+  if (ob::put_off_end([=] { (void)ob_sc2p5d_destroy(c); })) return 0;
   ob::sc2d_destroy(c);
   OB_CATCH
 }

@@ -914,6 +914,7 @@ OB_API int ob_sc3d_create(int nx, int ny, int nz, ob_sc3d** out) {
 
 OB_API int ob_sc3d_destroy(ob_sc3d* c) {
   OB_TRY if (!c) return 0;
+  if (ob::put_off_end([=] { (void)ob_sc3d_destroy(c); })) return 0;
   // Pending kicks read phi: apply them before the buffers go.
   std::string err;
   try {
@@ -1445,6 +1446,7 @@ OB_API int ob_slice2d_create(int nx, int ny, int nz, double xy_ratio, ob_slice2d
 
 OB_API int ob_slice2d_destroy(ob_slice2d* c) {
   OB_TRY if (!c) return 0;
+  if (ob::put_off_end([=] { (void)ob_slice2d_destroy(c); })) return 0;
   std::string err;
   try {
     ob::flush_kicks_reading(c->phi);

@@ -187,3 +187,35 @@ def test_weights_of_a_bunch_brought_back_to_user_order():
     for a, b in zip(*outs):
         for j in range(6):
             assert rel_l2(b[j], a[j]) < 1e-9, j
+
+
+def test_objects_that_go_during_a_capture():
+    """A bunch is in a reference cycle with its synchronous particle, so the collector may free
+    it, and a calculator, while a cell is being recorded: their end waits for the recording's."""
+    import gc
+    import spacecharge
+    from batch import BunchBatch
+    from workloads import gaussian_coords, make_bunch, PIPE_RADIUS
+    sizes, grids = [3000, 5000], [(32, 32, 16), (16, 16, 8)]
+    ref, _ = _single(2, sizes, grids)
+    bunches, calcs = _setup(sizes, grids)
+    bb = BunchBatch(bunches, calcs)
+    lat = _lattice(bb.calculator(), 1)
+    lat.trackBunch(bb.bunch())
+    other = [make_bunch(gaussian_coords(2000, seed=3)), spacecharge.SpaceChargeCalc2p5Drb(8, 8, 4),
+             spacecharge.SpaceChargeCalc3D(8, 8, 8), spacecharge.Boundary2D(16, 3, "Circle", 0.1)]
+    other.append(BunchBatch([make_bunch(gaussian_coords(900, seed=4))]))
+    other[1].trackBunch(other[0], 0.1, PIPE_RADIUS)
+
+    def cell():
+        other.clear()
+        gc.collect()
+        lat.trackBunch(bb.bunch())
+
+    bb.capture(cell)
+    bb.replay(1)
+    bb.synchronize()
+    for k, b in enumerate(bunches):
+        out = b.getCoordinates()
+        for j in range(6):
+            assert rel_l2(out[j], ref[k][j]) < 1e-9, (k, j)
