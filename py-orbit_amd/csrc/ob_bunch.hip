@@ -486,9 +486,14 @@ int bunch_flush(ob_bunch* b, double* ext_partials) {
   DeviceBunchView v = bunch_device_view(b);
   size_t pos = 0;
   int blocks = 0;
-  do {
-    pos += launch_front(b, v, pos, ext_partials, &blocks);
-  } while (pos < b->queue.size());
+  try {
+    do {
+      pos += launch_front(b, v, pos, ext_partials, &blocks);
+    } while (pos < b->queue.size());
+  } catch (const Error&) {  // what has been launched is not launched again
+    b->queue.erase(b->queue.begin(), b->queue.begin() + (ptrdiff_t)pos);
+    throw;
+  }
   b->queue.clear();
   b->host_valid = false;
   return blocks;

@@ -124,17 +124,18 @@ __device__ __forceinline__ void drift_one(double length, double gamma2i, double 
 }
 
 // wedgebend / wedgebendCF (teapotbase.cc:1037-1080, 1447-1509).  w: ct, rho, poles (4 bits
-// each), then kl of the nm multipoles; ia = inout | nm << 1 | skew bits << 8 | nst << 16.  The
-// multipole kick of each step is multpi (:280-315) with kl * sm, divided by pole! per particle
+// each, low half) and nst, then kl of the nm multipoles; ia = inout | nm << 1 | skew bits << 8.
+// The multipole kick of each step is multpi (:280-315) with kl * sm, divided by pole! per particle
 // as there.
 template <typename W>
 __device__ __forceinline__ void wedgebend(W w, uint32_t ia, double gamma2i, double dp_p,
                                           double KNL, double& x, double& xp, double& y,
                                           double& yp, double& z) {
   const double ct = w[0], rho = w[1];
-  const uint32_t poles = (uint32_t)__double_as_longlong(w[2]);
+  const uint64_t pn = (uint64_t)__double_as_longlong(w[2]);
+  const uint32_t poles = (uint32_t)pn;
   const int inout = ia & 1, nm = (ia >> 1) & 15, skews = (ia >> 8) & 255;
-  const int nst = (int)(ia >> 16);
+  const int nst = (int)(pn >> 32);
   double s;
   if (inout == 0) {
     s = -x / ct;
@@ -912,12 +913,11 @@ size_t program_encode(const Op* ops, size_t count, OpProgram& prog) {
         break;
       case OP_WEDGEBEND: {
         const int nm = (o.i0 >> 1) & 15;
-        OB_REQUIRE(o.i1 < 65536, "wedgebend: more than 131071 steps");
         put(o.p[0]); put(o.p[1]);
-        put(word_of((uint32_t)o.i2, 0u));
+        put(word_of((uint32_t)o.i2, (uint32_t)o.i1));
         for (int l = 0; l < nm; l++) put(o.p[4 + l]);
         dpc(o.p[2]); g2i(o.p[3]);
-        ia = (uint32_t)(o.i0 & 0xFFFF) | ((uint32_t)o.i1 << 16);
+        ia = (uint32_t)o.i0;
         break;
       }
       case OP_SOLN: put(o.p[0]); put(o.p[1]); g2i(o.p[2]); dpc(o.p[3]); break;

@@ -61,6 +61,12 @@ def test_program_lengths(op, count):
     _check([op] * count, n=65)
 
 
+@pytest.mark.parametrize("steps", [131_069, 131_072, 262_147])
+def test_wedgebend_of_many_steps(steps):
+    _check([("drift", 0.01)] * 240 + [("wedgebendCF", 0.1, 1, 10.0, 1, [1], [0.1], [0], steps),
+                                      ("wedgebend", 0.1, 0, 10.0, steps), ("drift", 0.1)], n=33)
+
+
 @pytest.mark.parametrize("seed", range(4))
 def test_random_programs(seed):
     r = np.random.default_rng(seed)
