@@ -160,8 +160,9 @@ __global__ __launch_bounds__(kCoefThreads) void bnd_coef_slices(
   bnd_coefs(lsq, nf, np, bphi, work + (size_t)nz * np + (size_t)iz * nf);
 }
 
-__global__ __launch_bounds__(256) void bnd_apply_slices(double* __restrict__ phi, int nx, int ny,
-                                                        int nz, const SC2DState* st,
+// dst = src - the harmonic field; src and dst may be one array.
+__global__ __launch_bounds__(256) void bnd_apply_slices(const double* src, double* dst, int nx,
+                                                        int ny, int nz, const SC2DState* st,
                                                         const double* __restrict__ coefs,
                                                         int nm, double rnorm) {
   if (st->skip) return;
@@ -192,7 +193,7 @@ __global__ __launch_bounds__(256) void bnd_apply_slices(double* __restrict__ phi
       csk = c1;
     }
   }
-  phi[t] -= v;
+  dst[t] = src[t] - v;
 }
 
 // The mode functions at one point (BaseBoundary2D.cc:316-345), host side.
@@ -317,13 +318,46 @@ void set_point(ob_boundary2d* b, int i, double x, double y) {
 }
 }  // namespace
 
+namespace {
+// Each of nz slices of src minus its harmonic field into dst (which may be src).
+void subtract_slices(ob_boundary2d* b, const double* src, double* dst, int nx, int ny, int nz,
+                     const SC2DState* st, hipStream_t s) {
+  const int nf = 2 * b->nm + 1;
+  const int64_t need = (int64_t)nz * (b->np + nf);
+  if (need > b->work3_cap) {
+    OB_HIP(hipStreamSynchronize(s));
+    if (b->d_work3) OB_HIP(hipFree(b->d_work3));
+    b->d_work3 = nullptr;
+    b->work3_cap = 0;
+    OB_HIP(hipMalloc((void**)&b->d_work3, sizeof(double) * need));
+    b->work3_cap = need;
+  }
+  {
+    ProfScope ps("bnd_coef_slices", s);
+    hipLaunchKernelGGL(bnd_coef_slices, dim3(nz), dim3(kCoefThreads), 0, s, src, nx, ny, nz, st,
+                       b->d_bx, b->d_by, b->np, b->d_lsq, nf, b->d_work3);
+  }
+  {
+    ProfScope ps("bnd_apply_slices", s);
+    const int64_t tot = (int64_t)nx * ny * nz;
+    hipLaunchKernelGGL(bnd_apply_slices, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s,
+                       src, dst, nx, ny, nz, st, b->d_work3 + (size_t)nz * b->np, b->nm,
+                       b->rnorm);
+  }
+  OB_HIP(hipGetLastError());
+}
+}  // namespace
+
 void boundary_add_potential(ob_boundary2d* b, const double* src, double* dst, int nx, int ny,
                             const SC2DState* st, hipStream_t s) {
   OB_REQUIRE(b->initialized,
              "Boundary2D addBoundaryPotential: the boundary was not initialized");
   const int nf = 2 * b->nm + 1;
   const size_t lds = sizeof(double) * (b->np + nf);
-  OB_REQUIRE(lds <= 160 * 1024, "Boundary2D addBoundaryPotential: too many boundary points");
+  if (lds > 160 * 1024) {  // more points than a workgroup's LDS holds: through global memory
+    subtract_slices(b, src, dst, nx, ny, 1, st, s);
+    return;
+  }
   if (lds > 64 * 1024)
     OB_HIP(hipFuncSetAttribute((const void*)bnd_subtract,
                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
@@ -340,26 +374,7 @@ void boundary_add_potential_slices(ob_boundary2d* b, double* phi, int nx, int ny
                                    const SC2DState* st, hipStream_t s) {
   OB_REQUIRE(b->initialized,
              "Boundary2D addBoundaryPotential: the boundary was not initialized");
-  const int nf = 2 * b->nm + 1;
-  const int64_t need = (int64_t)nz * (b->np + nf);
-  if (need > b->work3_cap) {
-    OB_HIP(hipStreamSynchronize(s));
-    if (b->d_work3) OB_HIP(hipFree(b->d_work3));
-    OB_HIP(hipMalloc((void**)&b->d_work3, sizeof(double) * need));
-    b->work3_cap = need;
-  }
-  {
-    ProfScope ps("bnd_coef_slices", s);
-    hipLaunchKernelGGL(bnd_coef_slices, dim3(nz), dim3(kCoefThreads), 0, s, phi, nx, ny, nz, st,
-                       b->d_bx, b->d_by, b->np, b->d_lsq, nf, b->d_work3);
-  }
-  {
-    ProfScope ps("bnd_apply_slices", s);
-    const int64_t tot = (int64_t)nx * ny * nz;
-    hipLaunchKernelGGL(bnd_apply_slices, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s,
-                       phi, nx, ny, nz, st, b->d_work3 + (size_t)nz * b->np, b->nm, b->rnorm);
-  }
-  OB_HIP(hipGetLastError());
+  subtract_slices(b, phi, phi, nx, ny, nz, st, s);
 }
 
 int boundary_describe(ob_boundary2d* b, double* bnd6) {

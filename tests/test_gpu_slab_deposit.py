@@ -114,10 +114,12 @@ def test_green_rebuild_with_the_deposit(grid):
             assert rel_l2(out[q] - c[q], ob.coords[q] - c[q]) < 1e-10
 
 
-@pytest.mark.parametrize("npts,nm", [(8, 1), (64, 0), (64, 16), (68, 31), (200, 33), (1000, 5)])
+@pytest.mark.parametrize("npts,nm", [(8, 1), (64, 0), (64, 16), (68, 31), (200, 33), (1000, 5),
+                                      (20_475, 2), (20_476, 2), (30_000, 5)])
 def test_boundary_sizes(npts, nm):
     """The boundary's correction for fewer points than lanes, one to seventeen rounds of rows
-    per wave, and no modes, on a grid whose nodes end within a workgroup."""
+    per wave, no modes, and the most points that a workgroup's LDS holds and more, on a grid
+    whose nodes end within a workgroup."""
     import spacecharge
     bnd = spacecharge.Boundary2D(npts, nm, "Ellipse", 0.05, 0.04)
     obnd = O.Boundary2D(npts, nm, "Ellipse", 0.05, 0.04)
