@@ -109,7 +109,7 @@ void build_records(ob_batch* B, bool force) {
   OB_REQUIRE(!B->capturing, "batch: bunch sizes, weights or constants changed during a graph capture");
   B->h_bb.assign(nb, BatchBunch{});
   B->h_items.clear();
-  int rows = 0, cols = 0, max_M = 16, slots = 0;
+  int rows = 0, cols = 0, max_M = 16, max_nz = 1, slots = 0;
   size_t hist_lds = 0, dep_lds = 0, slab_lds = 0, srow_lds = 0;
   int slabs = 0, srows = 0, scols = 0;
   std::vector<SlabDep> split;
@@ -138,6 +138,7 @@ void build_records(ob_batch* B, bool force) {
       rows += (r.nx + 1) / 2;
       cols += r.H;
       max_M = std::max(max_M, std::max(r.M0, r.M1));
+      max_nz = std::max(max_nz, r.nz);
       if (!split.empty()) {
         r.sd = split[b];
         r.slab_begin = slabs;
@@ -181,8 +182,8 @@ void build_records(ob_batch* B, bool force) {
     OB_HIP(hipMemcpyAsync(B->d_items, B->h_items.data(), sizeof(BatchItem) * ni,
                           hipMemcpyHostToDevice, s));
   OB_HIP(hipStreamSynchronize(s));  // host vectors may change before the copies run
-  B->shape = BatchShape{nb,    ni,    rows,  cols,     max_M,   slots, hist_lds, dep_lds,
-                        slabs, srows, scols, slab_lds, srow_lds};
+  B->shape = BatchShape{nb,       ni,      rows,  cols,  max_M, max_nz,   slots,
+                        hist_lds, dep_lds, slabs, srows, scols, slab_lds, srow_lds};
   B->seen_n.resize(nb);
   B->seen_ptr.resize(nb);
   for (int b = 0; b < nb; b++) {

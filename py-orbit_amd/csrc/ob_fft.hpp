@@ -325,15 +325,11 @@ __device__ __forceinline__ double2* line_fft(double2* a, double2* b, const doubl
 // imaginary parts apart, in less than half the LDS.  The line lies where two buffers leave a
 // CU one workgroup and the solve has more of them than the chip has CUs: a step on 1000 x 1000
 // nodes (2048 points) took 140 us with two buffers and takes 116 in place, on 600 x 520 124 and
-// 103; on 500 x 500 (1024 points) both take 80.7.  Two buffers of 4096 points beside the post
-// pass would be more LDS than a workgroup has.
+// 103; on 500 x 500 (1024 points) both take 80.7.
 constexpr int kLineTwoBuffers = 1024;
 __host__ __device__ constexpr bool line_two_buffers(int n) { return n <= kLineTwoBuffers; }
-__host__ __device__ constexpr size_t line_lds_bytes(int n, bool two) {
-  return two ? sizeof(double2) * (2 * n + n / 2) : sizeof(double) * 2 * fft_line(n);
-}
 __host__ __device__ constexpr size_t line_lds_bytes(int n) {
-  return line_lds_bytes(n, line_two_buffers(n));
+  return line_two_buffers(n) ? sizeof(double2) * (2 * n + n / 2) : sizeof(double) * 2 * fft_line(n);
 }
 template <int N, int NT, bool TWO = line_two_buffers(N)>
 struct LineFft {

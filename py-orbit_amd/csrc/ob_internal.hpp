@@ -267,7 +267,7 @@ void launch_push_batch(const BatchBunch* bb, const BatchItem* items, int nitems,
                        int threads, hipStream_t s);
 // SpaceChargeCalc2p5Drb steps of all bunches after launch_push_batch with extrema.
 struct BatchShape {
-  int nb, nitems, row_blocks, col_blocks, max_M, dep_slots;
+  int nb, nitems, row_blocks, col_blocks, max_M, max_nz, dep_slots;
   size_t hist_lds, dep_lds;  // dynamic LDS of the hist/scatter and tile-deposit passes
   int slab_blocks, srow_blocks, scol_blocks;  // grid-copy deposit (slab_blocks 0: tile sort)
   size_t slab_lds, srow_lds;

@@ -871,6 +871,14 @@ __device__ __forceinline__ double ipow(double x, int j) {  // exact for the smal
   return r;
 }
 
+// Its LDS is the kernel's dynamic one (post_lds_bytes), so that where other workgroups of the
+// launch transform lines, these have the CU's LDS to themselves: declared beside the lines
+// (41 KiB for 4096 bins) it halved the workgroups of a column pass (32 bunches on 256 x 256
+// nodes: 129 us, so 77).
+__host__ __device__ constexpr size_t post_lds_bytes(int nz, int threads) {
+  return sizeof(double) * (kSetupThreads / 64 + nz + threads);
+}
+
 // zg: when zpart is given, the sum of its zrows rows of per-block line densities.
 // Moments: the sum of the deposit items' partial moments mpart[nitems][5] (or mpart[mrows][5]
 // without nitems: the solve beside this pass reads the scale coefficient, which the deposit
@@ -883,10 +891,10 @@ __device__ __forceinline__ void sc2d_post_body(const SC2DParams& P, SC2DState* s
                                                const double* __restrict__ mpart,
                                                const uint32_t* nitems, int part = 7,
                                                int mrows = 0) {
-  __shared__ double sh[kSetupThreads / 64];
-  // the z line density, read below many times per bin, is kept in LDS
-  __shared__ double zl[kMaxZBinsLDS];
   const int nz = P.nz;
+  extern __shared__ double post_lds[];
+  double* sh = post_lds;
+  double* zl = sh + kSetupThreads / 64;  // the z line density, read many times per bin
   // part 1: z line density (SpaceChargeCalc2p5D: and the total); 4: its derivative, of zg when
   // part 1 ran earlier; 2: rho moments and kick factors (parts 2 and 4, and 2 and 1 with 4, may
   // run side by side: neither reads what the other writes)
@@ -894,7 +902,7 @@ __device__ __forceinline__ void sc2d_post_body(const SC2DParams& P, SC2DState* s
   } else if ((part & 1) && zpart) {
     // g = blockDim / nz threads per bin (when nz < blockDim) sum the rows in turn, then
     // their partial sums meet in LDS
-    __shared__ double zs[kSetupThreads];
+    double* zs = zl + nz;
     const int g = nz < (int)blockDim.x ? (int)blockDim.x / nz : 1;
     for (int i0 = 0; i0 < nz; i0 += (int)blockDim.x / g) {
       const int i = i0 + (int)threadIdx.x / g, r = (int)threadIdx.x % g;
@@ -1063,7 +1071,7 @@ __global__ __launch_bounds__(kSetupThreads) void sc2d_post(SC2DParams P, SC2DSta
 // (a) two real rows per complex FFT along y, r2c split.  rows >= nrows_in are zero;
 // columns >= ncols_in are zero (padding).  out: spectrum [*][H] complex (H = N/2+1).
 // blk: row pair (rows 2 blk, 2 blk + 1).
-template <int N, bool TWO = line_two_buffers(N)>
+template <int N>
 __device__ __forceinline__ void rows_r2c_body(const double* __restrict__ in, int nrows_in,
                                               int ncols_in, int ld_in,
                                               double2* __restrict__ out,
@@ -1071,7 +1079,7 @@ __device__ __forceinline__ void rows_r2c_body(const double* __restrict__ in, int
                                               const SC2DState* st, int blk) {
   if (st && st->skip) return;
   extern __shared__ double sm[];
-  LineFft<N, kFFTThreads, TWO> F(sm, tw, nmax);
+  LineFft<N, kFFTThreads> F(sm, tw, nmax);
   const int r0 = 2 * blk, r1 = r0 + 1;
   for (int j = threadIdx.x; j < N; j += kFFTThreads)
     F.set(j, make_double2((j < ncols_in) ? in[(int64_t)r0 * ld_in + j] : 0.0,
@@ -1102,10 +1110,7 @@ __global__ __launch_bounds__(kFFTThreads) void fft_rows_r2c(const double* __rest
 // independent halves side by side (z line density and derivative; rho moments and kick
 // factors).  All only read rho; the post pass writes the state's kick factors, z line
 // density and derivative, which the column pass after this launch (scale_coeff) and the
-// next map kernel read.  One launch fewer per step.  1024 points go in place here: two buffers
-// and the post pass's LDS leave a CU one workgroup (512 x 512 nodes, 258 workgroups: 15.0 us,
-// in place 11.4; 500 x 500 11.8 both).
-constexpr bool post_two_buffers(int n) { return n <= 512; }
+// next map kernel read.  One launch fewer per step.
 template <int N>
 __global__ __launch_bounds__(kFFTThreads) void fft_rows_r2c_post(
     const double* __restrict__ rho, int nrows_in, int ncols_in, double2* __restrict__ out,
@@ -1113,8 +1118,7 @@ __global__ __launch_bounds__(kFFTThreads) void fft_rows_r2c_post(
     double* __restrict__ zg, double* __restrict__ zd, Tile2D tg, int zrows, int moments) {
   const int rb = (nrows_in + 1) / 2;
   if ((int)blockIdx.x < rb) {
-    rows_r2c_body<N, post_two_buffers(N)>(rho, nrows_in, ncols_in, ncols_in, out, tw, nmax, st,
-                                          blockIdx.x);
+    rows_r2c_body<N>(rho, nrows_in, ncols_in, ncols_in, out, tw, nmax, st, blockIdx.x);
     return;
   }
   // two more workgroups: the line density part and the moments part of the post pass
@@ -1563,11 +1567,6 @@ namespace {
 template <int N>
 constexpr size_t fft_lds() { return line_lds_bytes(N); }
 
-// A workgroup's LDS, and what sc2d_post_body declares of it: the kernels that run the post pass
-// beside transforms have both, whichever a workgroup does.
-constexpr size_t kLdsPerGroup = 160 * 1024;
-constexpr size_t kPostLds =
-    sizeof(double) * (kMaxZBinsLDS + kSetupThreads + kSetupThreads / 64);
 
 // Dynamic LDS above 64 KiB has to be allowed per kernel; done once per instantiation.
 template <typename K>
@@ -1647,17 +1646,16 @@ void launch_fft_pipeline(ob_sc2p5drb* c, SC2DState* st, double* phi,
     dispatch_pow2(c->M1, [&](auto NC) {
       constexpr int N = decltype(NC)::value;
       if constexpr (N >= 8) {
-        constexpr size_t lds = line_lds_bytes(N, post_two_buffers(N));
-        static_assert(lds + kPostLds <= kLdsPerGroup, "row pass: LDS");
         static bool ready = false;
         if (!ready) {
-          allow_lds(fft_rows_r2c_post<N>, lds);
+          allow_lds(fft_rows_r2c_post<N>, fft_lds<N>());
           ready = true;
         }
         ob::ProfScope ps_("fft_rows_r2c_post");
         OB_REQUIRE(!post->P.plain, "2.5D post pass: the split form is for SpaceChargeCalc2p5Drb");
         hipLaunchKernelGGL(fft_rows_r2c_post<N>, dim3((c->nx + 1) / 2 + 2), dim3(kFFTThreads),
-                           lds, stream(), c->rho, c->nx, c->ny, c->spec, c->tw, c->nmax,
+                           std::max(fft_lds<N>(), post_lds_bytes(c->nz, kFFTThreads)), stream(),
+                           c->rho, c->nx, c->ny, c->spec, c->tw, c->nmax,
                            post->P, st, c->zg, c->zd, post->tg, post->zrows, post->moments);
       }
     });
@@ -1675,10 +1673,11 @@ void launch_slab_solve(ob_sc2p5drb* c, const SC2DParams& P, const SlabDep& D, do
   dispatch_pow2(c->M1, [&](auto NC) {
     constexpr int N = decltype(NC)::value;
     if constexpr (N >= 8 && N <= 2 * kSlabMaxNy) {
-      constexpr size_t most = fft_lds<N>() + sizeof(double) * kSumGroups * (N / 2 + 1);
-      static_assert(most + kPostLds + sizeof(double) * 5 * (kSumThreads / 64) <= kLdsPerGroup,
-                    "row pass with the copies: LDS");
-      const size_t lds = fft_lds<N>() + sizeof(double) * kSumGroups * c->ny;
+      constexpr size_t most =
+          std::max(fft_lds<N>() + sizeof(double) * kSumGroups * (N / 2 + 1),
+                   post_lds_bytes(kMaxZBinsLDS, kSumThreads));
+      const size_t lds = std::max(fft_lds<N>() + sizeof(double) * kSumGroups * c->ny,
+                                  post_lds_bytes(c->nz, kSumThreads));
       static bool ready = false;
       if (!ready) {
         OB_HIP(hipFuncSetAttribute((const void*)fft_rows_sum_post<N>,
@@ -1697,13 +1696,12 @@ void launch_slab_solve(ob_sc2p5drb* c, const SC2DParams& P, const SlabDep& D, do
     if constexpr (N >= 8) {
       static bool ready = false;
       if (!ready) {
-        static_assert(fft_lds<N>() + kPostLds <= kLdsPerGroup, "column pass: LDS");
         allow_lds(fft_cols_post<N>, fft_lds<N>());
         ready = true;
       }
       ob::ProfScope ps_("fft_cols_post");
       hipLaunchKernelGGL(fft_cols_post<N>, dim3(c->H + (P.plain ? 0 : 2)), dim3(kFFTThreads),
-                         fft_lds<N>(), stream(), c->spec, c->nx, c->H, c->ghat_t, c->tw, c->nmax,
+                         std::max(fft_lds<N>(), post_lds_bytes(c->nz, kFFTThreads)), stream(), c->spec, c->nx, c->H, c->ghat_t, c->tw, c->nmax,
                          c->st, (double)c->M0 * (double)c->M1, P.plain ? c->gate : nullptr,
                          c->gspec, P, D.mrows, c->nx, c->zg, c->zd);
     }
@@ -1982,7 +1980,8 @@ void launch_sc2d_batch(const BatchBunch* bb, const BatchItem* items, const Batch
   OB_REQUIRE(sh.hist_lds <= 64 * 1024 && sh.dep_lds <= 64 * 1024,
              "batch deposit: LDS block too large");
   OB_REQUIRE(sh.max_M <= 1024, "batch: grids up to 512 points per axis");
-  const size_t fl = line_lds_bytes(sh.max_M);  // (grows with N; at most 1024 points here)
+  // (line_lds_bytes grows with N up to the 1024 points of a batch)
+  const size_t fl = line_lds_bytes(sh.max_M);
   if (sh.slab_blocks) {
     OB_REQUIRE(jobs.empty(), "batch: a denoiser with the grid-copy deposit");
     {
@@ -1997,8 +1996,9 @@ void launch_sc2d_batch(const BatchBunch* bb, const BatchItem* items, const Batch
     }
     {
       ProfScope ps("fft_cols_post_batch");
-      hipLaunchKernelGGL(cols_post_batch, dim3(sh.scol_blocks), dim3(kFFTThreads), fl, s, bb,
-                         sh.nb, length, pipe_radius);
+      hipLaunchKernelGGL(cols_post_batch, dim3(sh.scol_blocks), dim3(kFFTThreads),
+                         std::max(fl, post_lds_bytes(sh.max_nz, kFFTThreads)), s, bb, sh.nb,
+                         length, pipe_radius);
     }
     {
       ProfScope ps("fft_rows_c2r_batch");
@@ -2031,8 +2031,8 @@ void launch_sc2d_batch(const BatchBunch* bb, const BatchItem* items, const Batch
   if (!jobs.empty()) dn_denoise_rhos(jobs);
   {
     ProfScope ps("sc2d_post_batch");
-    hipLaunchKernelGGL(sc2d_post_batch, dim3(sh.nb), dim3(kSetupThreads), 0, s, bb, length,
-                       pipe_radius);
+    hipLaunchKernelGGL(sc2d_post_batch, dim3(sh.nb), dim3(kSetupThreads),
+                       post_lds_bytes(sh.max_nz, kSetupThreads), s, bb, length, pipe_radius);
   }
   {
     ProfScope ps("fft_rows_r2c_batch");
@@ -2201,7 +2201,8 @@ void sc2d_tile_step(ob_sc2p5drb* c, ob_bunch* b, const DeviceBunchView& v, const
   if (c->plain) {  // its solve reads the post pass's results: it runs first
     {
       ProfScope ps_("sc2d_post");
-      hipLaunchKernelGGL(sc2d_post, dim3(1), dim3(kSetupThreads), 0, s, P, c->st, c->rho,
+      hipLaunchKernelGGL(sc2d_post, dim3(1), dim3(kSetupThreads),
+                         post_lds_bytes(c->nz, kSetupThreads), s, P, c->st, c->rho,
                          c->zg, c->zd, tg, hb, moments);
     }
     launch_fft_pipeline(c, c->st, phi);
