@@ -145,7 +145,7 @@ void build_records(ob_batch* B, bool force) {
         r.srows_begin = srows;
         r.scols_begin = scols;
         slabs += r.sd.slabs * r.sd.parts;
-        srows += r.nx;
+        srows += sc2d_row_blocks(r);
         scols += r.H + 2;
         slab_lds = std::max(slab_lds, sc2d_slab_lds(r));
         srow_lds = std::max(srow_lds, sc2d_row_lds(r));

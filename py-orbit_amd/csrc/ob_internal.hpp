@@ -320,6 +320,7 @@ bool sc2d_batch_slabs(const std::vector<ob_sc2p5drb*>& calcs, const std::vector<
 bool sc2d_slab_same(ob_sc2p5drb* c, const SlabDep& D);
 size_t sc2d_slab_lds(const BatchBunch& r);
 size_t sc2d_row_lds(const BatchBunch& r);
+int sc2d_row_blocks(const BatchBunch& r);  // workgroups of its row pass
 void sc2d_mark_tracked(ob_sc2p5drb* c);
 int sc2d_read_status(ob_sc2p5drb* c);
 int push_grid_blocks(int64_t n);

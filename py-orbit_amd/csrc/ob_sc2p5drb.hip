@@ -1468,10 +1468,42 @@ __global__ __launch_bounds__(kSlabThreads) void sc2d_gdeposit_batch(const BatchB
 }
 
 constexpr int kBatchSumThreads = 512;  // a row has fewer copies than a single bunch's
+// The parts' line densities: kBatchZBins bins per workgroup, the threads of a bin take every
+// kBatchZGroups-th part, their sums meet in LDS in group order.  (One workgroup of the column
+// pass walked all parts and bins: 141 us for 128 parts of 4096 bins.)
+constexpr int kBatchZBins = 64, kBatchZGroups = kBatchSumThreads / kBatchZBins;
+__device__ __forceinline__ void zpart_sum(const SlabDep& D, int nz, double* __restrict__ zg,
+                                          int blk) {
+  extern __shared__ double sm[];
+  const int l = (int)threadIdx.x % kBatchZBins, grp = (int)threadIdx.x / kBatchZBins;
+  const int i = blk * kBatchZBins + l;
+  const gptr<const double> zp = to_global((const double*)D.zpart);
+  double acc = 0.0;
+  if (i < nz)
+    for (int p = grp; p < D.parts; p += 8 * kBatchZGroups) {
+      double v[8];  // (past the last part: one repeated and not added)
+#pragma unroll
+      for (int u = 0; u < 8; u++)
+        v[u] = zp[(int64_t)(p + u * kBatchZGroups < D.parts ? p + u * kBatchZGroups : p) * nz + i];
+#pragma unroll
+      for (int u = 0; u < 8; u++)
+        if (p + u * kBatchZGroups < D.parts) acc += v[u];
+    }
+  sm[threadIdx.x] = acc;
+  __syncthreads();
+  if (grp != 0 || i >= nz) return;
+  for (int q = 1; q < kBatchZGroups; q++) acc += sm[q * kBatchZBins + l];
+  zg[i] = acc;
+}
+
 __global__ __launch_bounds__(kBatchSumThreads) void rows_sum_batch(const BatchBunch* bb, int nb) {
   const int b = batch_find(bb, nb, blockIdx.x, &BatchBunch::srows_begin);
   const BatchBunch& B = bb[b];
   const int r = (int)blockIdx.x - B.srows_begin;
+  if (r >= B.nx) {
+    zpart_sum(B.sd, B.nz, B.zg, r - B.nx);
+    return;
+  }
   switch (B.M1) {
 #define OB_CASE(n)                                                                          \
   case n:                                                                                   \
@@ -1492,8 +1524,8 @@ __global__ __launch_bounds__(kFFTThreads) void cols_post_batch(const BatchBunch*
   const int k = (int)blockIdx.x - B.scols_begin;
   if (k >= B.H) {
     const SC2DParams P = batch_params(B, length, pipe_radius);
-    sc2d_post_body(P, B.st, nullptr, B.zg, B.zd, B.sd.zpart, B.sd.parts, B.sd.mrows, nullptr,
-                   k == B.H ? 2 : 5, B.nx);
+    sc2d_post_body(P, B.st, nullptr, B.zg, B.zd, nullptr, 0, B.sd.mrows, nullptr,
+                   k == B.H ? 2 : 4, B.nx);
     return;
   }
   const double npad = (double)B.M0 * (double)B.M1;
@@ -1943,7 +1975,11 @@ size_t sc2d_slab_lds(const BatchBunch& r) {
   return sizeof(double) * ((size_t)r.sd.R * r.ny + r.nz);
 }
 size_t sc2d_row_lds(const BatchBunch& r) {
-  return line_lds_bytes(r.M1) + sizeof(double) * kSumGroups * r.ny;
+  return std::max(line_lds_bytes(r.M1) + sizeof(double) * kSumGroups * r.ny,
+                  sizeof(double) * kBatchSumThreads);
+}
+int sc2d_row_blocks(const BatchBunch& r) {
+  return r.nx + (r.nz + kBatchZBins - 1) / kBatchZBins;
 }
 
 bool sc2d_tile_same(ob_sc2p5drb* c, const Tile2D& t, int64_t n, bool per_particle_m) {
