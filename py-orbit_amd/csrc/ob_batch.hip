@@ -6,8 +6,8 @@
 //   push     one workgroup per work item (a chunk of one bunch's particles): deferred SC
 //            kick, the map program, per-item extrema;
 //   setup    one workgroup per bunch (extrema of its items, grid sizing, clearing);
-//   deposit  where every grid fits and nothing changes rho, LDS copies of the grids (three
-//            passes with the solve, see sc2d_gdeposit_batch); otherwise setup and a tile sort
+//   deposit  where every grid fits, nothing changes rho and it is the faster one, LDS copies of
+//            the grids (three passes with the solve, see sc2d_gdeposit_batch); otherwise setup and a tile sort
 //            per bunch: hist and scatter one workgroup per work item, then one
 //            workgroup per tile work item accumulating rho in LDS;
 //   post     one workgroup per bunch; FFT row / column / row passes over all bunches'
@@ -234,7 +234,7 @@ float time_ms(hipEvent_t a, hipEvent_t b) {
   return ms;
 }
 
-// Tuning results of this process by device and batch shape (bunch count, then every
+// Tuning results of this process by device and batch shape (bunch count, deposit, then every
 // bunch's particle count, grid and macro-size attribute): a batch of the same shape takes
 // them instead of timing the candidates again.
 std::map<std::vector<int64_t>, std::pair<int, int>>& tuning_cache() {
@@ -244,7 +244,8 @@ std::map<std::vector<int64_t>, std::pair<int, int>>& tuning_cache() {
 std::vector<int64_t> tuning_key(const ob_batch* B) {
   int dev = 0;
   OB_HIP(hipGetDevice(&dev));
-  std::vector<int64_t> k{dev, (int64_t)B->h_bb.size(), B->calcs.empty() ? 0 : 1};
+  std::vector<int64_t> k{dev, (int64_t)B->h_bb.size(),
+                         B->calcs.empty() ? 0 : B->shape.slab_blocks ? 1 : 2};
   for (const BatchBunch& r : B->h_bb) {
     k.push_back(r.v.n);
     k.push_back(r.nx);

@@ -313,7 +313,7 @@ Tile2D sc2d_tile_reserve(ob_sc2p5drb* c, int64_t n, bool per_particle_m, int ite
 // Whether `t` still describes the calculator's tile buffers and fits such a bunch.
 bool sc2d_tile_same(ob_sc2p5drb* c, const Tile2D& t, int64_t n, bool per_particle_m);
 // Grid-copy deposit of a batch: the split of every bunch (n particles each), or false if a
-// grid does not fit it or a calculator has a denoiser.  sc2d_slab_same: D's buffers are still
+// grid does not fit it, a calculator has a denoiser or the tile sort is the faster one.  sc2d_slab_same: D's buffers are still
 // the calculator's.
 bool sc2d_batch_slabs(const std::vector<ob_sc2p5drb*>& calcs, const std::vector<int64_t>& n,
                       std::vector<SlabDep>& out);

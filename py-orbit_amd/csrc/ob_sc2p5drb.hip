@@ -1926,17 +1926,30 @@ void launch_gdeposit(ob_sc2p5drb* c, const SC2DParams& P, const DeviceBunchView&
 // twelve steps: 0.75 rounds 2947 us, 1 2937, 1.5 2891, 2 2981, 3 3410 (the tile sort of the
 // same batch: 3245).  The middle two of four slabs hold nearly all of a beam, so a bunch counts
 // as two slabs at most.
+// The copies pay where the batch has few nodes (the launches' latency counts) or enough
+// particles for them; else the tile sort, whose work goes with the particles, is the faster
+// one.  A step in us, copies and tile sort: 32 bunches of 50k on 256 x 256 nodes 361 and 294,
+// of 400k 1047 and 957, of 800k 1842 and 1760, but 8 of 50k 121 and 123, 8 of 1M 583 and 585;
+// 64 of 20k on 128 x 128 250 and 234, of 50k 343 and 351, of 80k 433 and 455; 256 of 5k on
+// 64 x 64 425 and 375, of 20k 574 and 577; 32 of 150k on 200 x 150 450 and 447, of 300k 706 and
+// 742.  So many nodes or rows take the copies from 3, 5 or 14 particles a node on, for grids of
+// one, two or four slabs.
+constexpr int64_t kSlabBatchNodes = 512 * 1024, kSlabBatchRows = 4608;
 bool sc2d_batch_slabs(const std::vector<ob_sc2p5drb*>& calcs, const std::vector<int64_t>& n,
                       std::vector<SlabDep>& out) {
   size_t lds = 0;
-  int64_t total = 0;
+  int64_t total = 0, nodes = 0, grid_rows = 0, worth = 0;
   for (size_t b = 0; b < calcs.size(); b++) {
     const ob_sc2p5drb* c = calcs[b];
     if (c->slab.slabs == 0 || c->denoiser) return false;
+    nodes += (int64_t)c->nx * c->ny;
+    grid_rows += c->nx;
+    worth += (int64_t)c->nx * c->ny * (c->slab.slabs == 1 ? 3 : c->slab.slabs == 2 ? 5 : 14);
     const int rows = (c->nx - 2 + c->slab.slabs - 1) / c->slab.slabs;
     lds = std::max(lds, sizeof(double) * ((size_t)(rows + 2) * c->ny + c->nz));
     total += n[b];
   }
+  if ((nodes > kSlabBatchNodes || grid_rows > kSlabBatchRows) && total < worth) return false;
   const int64_t room = (int64_t)device_cu_count() * (lds <= 76 * 1024 ? 2 : 1) * 3 / 2;
   auto busy = [&](size_t b) { return std::min(calcs[b]->slab.slabs, 2); };
   auto parts = [&](size_t b, int64_t per) {

@@ -1,6 +1,6 @@
 """Batches whose grids take the grid-copy deposit: one to four slabs, from five particles to
-several parts a bunch, more bunches than the chip has CUs, a grid that sends the whole batch to
-the tile sort, buffers that a calculator moves between two steps, macrosizes, and graph
+several parts a bunch, more bunches than the chip has CUs, a grid and a number of nodes that
+send the whole batch to the tile sort, buffers that a calculator moves between two steps, macrosizes, and graph
 replays.  Against each bunch on its own, with the bars of test_gpu_batch.py."""
 import numpy as np
 import pytest
@@ -18,6 +18,7 @@ CASES = {
     "one": ([262_147], [(128, 128, 64)]),
     "bins": ([5000, 400_003, 30_000], [(16, 16, 65), (64, 64, 4096), (40, 30, 127)]),
     "tiles": ([5000, 9000], [(32, 32, 16), (400, 400, 8)]),
+    "nodes": ([2000 + 300 * k for k in range(11)], [(256, 256, 8)] * 8 + [(20, 30, 4)] * 3),
 }
 
 
