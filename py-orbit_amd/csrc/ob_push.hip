@@ -672,9 +672,10 @@ __device__ __forceinline__ void push_batch_body(const BatchBunch* __restrict__ b
 }
 
 
-// Levels 0 and 1 fit three waves per SIMD (168 VGPRs) without spilling, at most 12 bytes
-// at level 1; the bound measured 7% faster than the compiler's own 169-register, two-wave
-// allocation.  Level 2 would spill 220 bytes at that bound and keeps two waves.
+// Levels 0 and 1 are bounded to three waves per SIMD (168 VGPRs): they take 121 to 141 without
+// spills.  (With the interpreter of fixed op records they took 169, and the bound was 7%
+// faster.)  Level 2 spilled 220 bytes at the bound then and was left out of it; by itself it
+// now takes 157, with extrema 169, one register more than three waves allow.
 template <bool EXTREMA, int LEVEL>
 __global__ __launch_bounds__(kPushThreads) __attribute__((amdgpu_waves_per_eu(3))) void
 push_batch_kernel(const BatchBunch* __restrict__ bb, const BatchItem* __restrict__ items,

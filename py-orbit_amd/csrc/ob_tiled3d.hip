@@ -53,9 +53,10 @@ __device__ __forceinline__ uint32_t tile_key(const TileGeom& g, double x, double
   return (uint32_t)(((iX / g.T) * g.ty + (iY / g.T)) * g.tz + iZ / g.Tz);
 }
 
-// Workgroups past hist_blocks clear rho, which the deposit needs: the histogram waits for
-// particle loads and LDS, so the stores cost next to nothing beside it (a launch of their own
-// took 3.3 us at 64 x 64 x 64 nodes and 12.5 us at 128 x 128 x 256, and the gap before it).
+// Workgroups past hist_blocks clear rho, which the deposit needs, beside the histogram.  That
+// saves the launch and its gap, not the stores: 4M particles on 256 x 256 x 128 nodes take 34.5
+// us so, 25.0 without the clearing, whose own launch took 10.8; on 64 x 64 x 64 that one took
+// 3.3 us.
 __global__ __launch_bounds__(1024) void tile_hist(const double* __restrict__ cur, int64_t cap,
                                                       int64_t n, TileGeom g,
                                                       uint32_t* __restrict__ key,
