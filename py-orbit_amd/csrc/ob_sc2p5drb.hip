@@ -689,10 +689,10 @@ __host__ __device__ constexpr int green_pairs(int n) { return n >= 1024 ? 1 : 4;
 // whole; the row pass adds the copies.  There is no rho to clear beforehand, no tile sort
 // and no global atomic: at 100k on 128 x 128 it takes 11.9 us in the place of a bin pass
 // (7.4 us) and a private-grid deposit with atomics (11.8 us), at 1M on 200 x 150 26 us in the
-// place of bin (21 us), scatter (20 us) and tile deposit (25 us).  What bounds it is the LDS
-// atomic rate (nine per particle, 0.6 clocks a lane) and, for few particles, the extrema and
-// grid (2.5 us), clearing and storing the copy (2 us).  The workgroups of a part are `parts`
-// apart, so with a multiple of 8 parts its slabs read x, y, z through the same L2.
+// place of bin (21 us), scatter (20 us) and tile deposit (25 us).  It waits for loads and
+// barriers 55% of its wave time at 100k and 43% at 1M (on LDS issue 5% and 7%): the extrema and
+// grid (2.5 us), clearing and storing the copy (2 us; 31 MB of copies at 1M) and the rounds of
+// loads between them.  The workgroups of a part are `parts` apart, so with a multiple of 8 parts its slabs read x, y, z through the same L2.
 // GN > 0: SpaceChargeCalc2p5D, M1 = GN; the workgroups after the deposit's transform the
 // rows of the Green function on the new solver box when the grid asks for a rebuild.
 // blk: workgroup of the bunch's deposit; its extrema are partials rows pb .. pe - 1.
