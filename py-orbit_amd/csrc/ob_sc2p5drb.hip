@@ -98,8 +98,9 @@ struct Grid2Step {
 // Every thread of the block gets the grid of partials [pb, pe) (blockDim.x <= 1024, a
 // multiple of 64).  st is read (entry P.par) only for SpaceChargeCalc2p5D.  The first four
 // waves, one per SIMD, read the partials (all sixteen would queue 1152 shuffles on the LDS);
-// their extrema meet in LDS and wave 0 alone reduces them and sizes the grid.  One thread
-// walking sixteen rows of six values, as before, took 5.5 us of a 1024-thread workgroup.
+// their extrema meet in LDS and thread 0 reduces four of them and sizes the grid (a whole wave
+// doing that made the bin pass of 2000 particles 33.1 us, 31.1 so).  One thread walking sixteen
+// rows of six values, as before, took 5.5 us of a 1024-thread workgroup.
 constexpr int kGridWaves = 4;
 __device__ __forceinline__ void sc2d_grid_body(const SC2DParams& P,
                                                const double* __restrict__ partials, int pb,
@@ -135,7 +136,7 @@ __device__ __forceinline__ void sc2d_grid_body(const SC2DParams& P,
       for (int k = 0; k < 6; k++) red[k][threadIdx.x >> 6] = r[k];
   }
   __syncthreads();
-  if (threadIdx.x < 64) {
+  if (threadIdx.x == 0) {
 #pragma unroll
     for (int k = 0; k < 6; k++) {
       r[k] = red[k][0];
@@ -206,7 +207,7 @@ __device__ __forceinline__ void sc2d_grid_body(const SC2DParams& P,
     g.zMin = zMin;
     g.zMax = zMax;
     g.dz = (zMax - zMin) / P.nz;        // Grid1D.cc:88-93
-    if (threadIdx.x == 0) gs = g;
+    gs = g;
   }
   __syncthreads();
   out = gs;
