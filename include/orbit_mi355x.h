@@ -327,8 +327,10 @@ int ob_batch_set_tuning(ob_batch* batch, int chunk, int deposit_item);
 int ob_batch_get_tuning(ob_batch* batch, int* chunk, int* deposit_item, int* tuned);
 /* hipGraph: the batch calls between begin and end are recorded (not run) and replayed by
  * ob_batch_replay(count).  Pending work is applied before and at the end of the capture,
- * so a replay starts and ends with nothing pending.  Bunch sizes must not change between
- * the capture and its replays. */
+ * so a replay starts and ends with nothing pending.  A replay is refused ("capture again")
+ * when a bunch's size, weights, macrosize or kick constants, or a calculator's buffers or
+ * averaging length, have changed since the capture.  Objects destroyed while a capture runs
+ * are freed when it ends. */
 int ob_batch_capture_begin(ob_batch* batch);
 int ob_batch_capture_end(ob_batch* batch);
 int ob_batch_replay(ob_batch* batch, int count);

@@ -431,6 +431,7 @@ OB_API int ob_batch_destroy(ob_batch* B) {
     hipGraph_t g = nullptr;
     (void)ob::end_capture(B, &g);
     if (g) (void)hipGraphDestroy(g);
+    ob::collect(B);  // (maps that were to be recorded)
     B->queue.clear();
     B->kick = ob::BatchKick{};
   }

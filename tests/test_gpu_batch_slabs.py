@@ -221,3 +221,28 @@ def test_objects_that_go_during_a_capture():
         out = b.getCoordinates()
         for j in range(6):
             assert rel_l2(out[j], ref[k][j]) < 1e-9, (k, j)
+
+
+def test_a_batch_that_goes_while_it_records():
+    """Its recording goes with it, and with that the maps and steps recorded: the bunches are
+    left as they were, and track alone."""
+    import _obnative as N
+    from batch import BunchBatch
+    from workloads import PIPE_RADIUS
+    sizes, grids = [3000, 5000], [(32, 32, 16), (16, 16, 8)]
+    bunches, calcs = _setup(sizes, grids)
+    ref, rcalcs = _setup(sizes, grids)
+    bb = BunchBatch(bunches, calcs)
+    for b in ref:
+        b.getCoordinates()
+    N.call("ob_batch_capture_begin", bb._h)
+    bb.calculator().trackBunch(bb.bunch(), 0.5, PIPE_RADIUS)
+    bb.trackSequence([("drift", 0.7)])
+    bb.__del__()
+    for b, c, r, rc in zip(bunches, calcs, ref, rcalcs):
+        assert np.array_equal(b.getCoordinates(), r.getCoordinates())
+        c.trackBunch(b, 0.5, PIPE_RADIUS)
+        rc.trackBunch(r, 0.5, PIPE_RADIUS)
+        out, want = b.getCoordinates(), r.getCoordinates()
+        for j in range(6):
+            assert rel_l2(out[j], want[j]) < 1e-12, j
