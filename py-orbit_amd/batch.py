@@ -98,7 +98,8 @@ class BunchBatch:
     def _push_attrs(self):
         """Particle attributes set one by one (partAttrValue) reach the device."""
         for b in self.bunches:
-            b._push_attrs()
+            if b._msize_dirty:
+                b._push_attrs()
 
 
 class _BatchBunch:

@@ -95,11 +95,8 @@ void build_records(ob_batch* B, bool force) {
               : sc2d_tile_same(B->calcs[b], B->h_bb[b].tg, views[b].n, views[b].msize != nullptr)))
       same = false;
     if (same && !record_holds(B->h_bb[b], views[b], bunch_sync(B->bunches[b]))) same = false;
-    if (same && !B->calcs.empty()) {
-      BatchBunch now{};
-      sc2d_batch_record(B->calcs[b], now);
-      if (now.n_long_avg != B->h_bb[b].n_long_avg) same = false;
-    }
+    if (same && !B->calcs.empty() && sc2d_long_avg(B->calcs[b]) != B->h_bb[b].n_long_avg)
+      same = false;
     DenoiseJob dj;  // a denoiser set or cleared since: the moments come from elsewhere
     if (same && !B->calcs.empty() &&
         (sc2d_denoise_job(B->calcs[b], &dj) ? 1 : 0) != B->h_bb[b].moments_from_rho)

@@ -322,6 +322,7 @@ size_t sc2d_slab_lds(const BatchBunch& r);
 size_t sc2d_row_lds(const BatchBunch& r);
 int sc2d_row_blocks(const BatchBunch& r);  // workgroups of its row pass
 void sc2d_mark_tracked(ob_sc2p5drb* c);
+int sc2d_long_avg(const ob_sc2p5drb* c);
 int sc2d_read_status(ob_sc2p5drb* c);
 int push_grid_blocks(int64_t n);
 // The calculator's denoiser job (false: none set).

@@ -1469,9 +1469,12 @@ __global__ __launch_bounds__(kSlabThreads) void sc2d_gdeposit_batch(const BatchB
 }
 
 constexpr int kBatchSumThreads = 512;  // a row has fewer copies than a single bunch's
-// The parts' line densities: kBatchZBins bins per workgroup, the threads of a bin take every
-// kBatchZGroups-th part, their sums meet in LDS in group order.  (One workgroup of the column
-// pass walked all parts and bins: 141 us for 128 parts of 4096 bins.)
+// The parts' line densities of more bins than a column workgroup has threads: kBatchZBins bins
+// per workgroup, the threads of a bin take every kBatchZGroups-th part, their sums meet in LDS
+// in group order.  (One workgroup of the column pass walked all parts and bins: 141 us for 128
+// parts of 4096 bins.  Up to 256 bins it does so beside the columns without lasting longer,
+// and the row pass is 1 to 2 us shorter without these workgroups.)
+constexpr int kBatchZCols = kFFTThreads;
 constexpr int kBatchZBins = 64, kBatchZGroups = kBatchSumThreads / kBatchZBins;
 __device__ __forceinline__ void zpart_sum(const SlabDep& D, int nz, double* __restrict__ zg,
                                           int blk) {
@@ -1525,8 +1528,8 @@ __global__ __launch_bounds__(kFFTThreads) void cols_post_batch(const BatchBunch*
   const int k = (int)blockIdx.x - B.scols_begin;
   if (k >= B.H) {
     const SC2DParams P = batch_params(B, length, pipe_radius);
-    sc2d_post_body(P, B.st, nullptr, B.zg, B.zd, nullptr, 0, B.sd.mrows, nullptr,
-                   k == B.H ? 2 : 4, B.nx);
+    sc2d_post_body(P, B.st, nullptr, B.zg, B.zd, B.sd.zpart, B.sd.parts, B.sd.mrows, nullptr,
+                   k == B.H ? 2 : B.nz > kBatchZCols ? 4 : 5, B.nx);
     return;
   }
   const double npad = (double)B.M0 * (double)B.M1;
@@ -1993,7 +1996,7 @@ size_t sc2d_row_lds(const BatchBunch& r) {
                   sizeof(double) * kBatchSumThreads);
 }
 int sc2d_row_blocks(const BatchBunch& r) {
-  return r.nx + (r.nz + kBatchZBins - 1) / kBatchZBins;
+  return r.nx + (r.nz > kBatchZCols ? (r.nz + kBatchZBins - 1) / kBatchZBins : 0);
 }
 
 bool sc2d_tile_same(ob_sc2p5drb* c, const Tile2D& t, int64_t n, bool per_particle_m) {
@@ -2004,6 +2007,7 @@ bool sc2d_tile_same(ob_sc2p5drb* c, const Tile2D& t, int64_t n, bool per_particl
 }
 
 void sc2d_mark_tracked(ob_sc2p5drb* c) { c->tracked = true; }
+int sc2d_long_avg(const ob_sc2p5drb* c) { return c->n_long_avg; }
 
 void sc2d_flush_kicks(ob_sc2p5drb* const* calcs, size_t n) {
   batch_flush_kicks(calcs, n);

@@ -16,7 +16,8 @@ CASES = {
     "few": ([5, 9, 1025, 2049], [(3, 3, 1), (5, 7, 2), (64, 64, 32), (33, 20, 5)]),
     "many": ([400 + 7 * k for k in range(280)], [(8 + k % 9, 8 + k % 5, 4) for k in range(280)]),
     "one": ([262_147], [(128, 128, 64)]),
-    "bins": ([5000, 400_003, 30_000], [(16, 16, 65), (64, 64, 4096), (40, 30, 127)]),
+    "bins": ([5000, 400_003, 30_000, 2000], [(16, 16, 256), (64, 64, 4096), (40, 30, 257),
+                                             (8, 8, 65)]),
     "tiles": ([5000, 9000], [(32, 32, 16), (400, 400, 8)]),
     "nodes": ([2000 + 300 * k for k in range(11)], [(256, 256, 8)] * 8 + [(20, 30, 4)] * 3),
 }
